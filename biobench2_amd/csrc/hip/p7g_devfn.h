@@ -83,9 +83,10 @@ __device__ __forceinline__ float wave_sum_f(float v)
   v += dppz<ROW_SHR2>(v);
   v += dppz<ROW_SHR4>(v);
   v += dppz<ROW_SHR8>(v);
-  v += dppz<ROW_BCAST15, 0xa>(v);
-  v += dppz<ROW_BCAST31, 0xc>(v);
-  return readlanef(v, 63);
+  // the row totals through scalar registers, added as row_bcast:15 and
+  // row_bcast:31 would add them (those moves take 20 cycles each)
+  const float a = readlanef(v, 31) + readlanef(v, 15), b = readlanef(v, 63) + readlanef(v, 47);
+  return b + a;
 }
 // The same moves leave every lane with the inclusive prefix sum over lanes 0..lane.
 __device__ __forceinline__ float wave_scan_f(float v)

@@ -1,0 +1,199 @@
+// What the list kernels (Viterbi, Forward, Backward: one target per wave or
+// workgroup, taken from a list through its work queue) share.
+#pragma once
+#include "p7g_devfn.h"
+
+// Where a list kernel finds its profile tables (template argument TM):
+//   TM_LDS   the whole table in LDS, transitions pinned in registers
+//   TM_PIN   the table in global memory (L2-resident), transitions pinned
+//   TM_TLDS  transitions in LDS, read per row; emission rows from global memory
+//   TM_GLOB  the table in global memory, transitions read per row
+// Large models take the last two: B positions of every transition pinned in
+// registers would not fit the register file, and the whole table not in LDS.
+// The per-row reads go through an offset the compiler cannot see through, so
+// that they are not hoisted out of the row loop into registers again.
+enum { TM_LDS = 0, TM_PIN = 1, TM_TLDS = 2, TM_GLOB = 3 };
+
+__device__ __forceinline__ int opaque_zero()
+{
+  int v = 0;
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// The residues of a row loop, 64 rows at a time, as table offsets (residue *
+// stride): while the loop's step s (0, 1, ...) runs, ahead(s & 63) is the offset
+// of the step after it, so that its emission row can be loaded a row early; lane
+// l of `cur` holds that of step s0 + l + 1. One vector load per 64 rows and one
+// v_readlane per row; taking the bytes out of a 16-byte chunk in scalar registers
+// cost six branches a row, about 200 cycles of a wave that runs alone. Step s
+// reads residue s (ascending), or residue L-1-s (descending); steps past the end
+// read the byte behind the target, which is always readable, or residue 0.
+template <bool DESC>
+struct RowRes {
+  const uint8_t *sq;
+  int L, z, s0, stride, cur, far;
+  __device__ __forceinline__ int byte(int s) const { return (int) sq[DESC ? max(L - 1 - s, 0) : min(s, L)]; }
+  __device__ __forceinline__ int init(const uint8_t *q, int len, int lane, int str)
+  {
+    sq = q; L = len; z = lane; s0 = 0; stride = str;
+    const int x0 = uni(byte(0));
+    cur = byte(1 + z) * stride; far = byte(65 + z);
+    return x0 * stride;                          // the first step's offset
+  }
+  __device__ __forceinline__ int ahead(int u) const { return __builtin_amdgcn_readlane(cur, u); }
+  __device__ __forceinline__ void advance() { s0 += 64; cur = far * stride; far = byte(s0 + 65 + z); }
+};
+// x > lim for a wave-uniform x held in a scalar register, as the float compare
+// (false for NaN) on its bit pattern; lim is positive. A scalar compare and
+// branch, where the vector compare took the branch through VCC.
+__device__ __forceinline__ bool gt_bits(int xbits, int limbits)
+{ return __builtin_expect((unsigned) (xbits - limbits - 1) <= 0x7f800000u - (unsigned) limbits - 1u, 0); }
+#define BITS_1E4  0x461c4000      // 1.0e4f
+#define BITS_1E16 0x5a0e1bca      // 1.0e16f
+#define BITS_ONE  0x3f800000      // 1.0f
+
+// A workgroup barrier that orders LDS alone: global loads in flight (the next
+// row's odds) stay in flight, where __syncthreads would wait for them.
+__device__ __forceinline__ void lds_barrier()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Workgroup sizes of the list kernels: 8 waves, or 4 (one per SIMD, so that a
+// wave may hold 512 registers with the accumulation registers) where the
+// per-lane state of large models does not fit in 256.
+#define VIT_THREADS(ND) ((ND) >= 40 ? 256 : 512)
+#define FWD_THREADS(B)  ((B) >= 64 ? 256 : 512)
+#define BCK_THREADS(B)  ((B) >= 28 ? 256 : 512)
+
+// a*b + c*d in one rounding order, whatever the compiler would contract in the
+// place it stands: the product of SW ? the first : the second pair is rounded,
+// the other one fused onto it.
+template <bool SW>
+__device__ __forceinline__ float fma2(float a, float b, float c, float d)
+{
+#pragma clang fp contract(off)
+  return SW ? __builtin_fmaf(c, d, a * b) : __builtin_fmaf(a, b, c * d);
+}
+
+// v where the lane's bit of a constant mask is set, else w: one v_cndmask. The
+// carry of a lane's 16-lane row is selected with these; left to itself the
+// compiler branched over the lanes' rows inside the row loop.
+__device__ __forceinline__ float lane_sel(float w, float v, unsigned long long mask)
+{
+  float r;
+  asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(w), "v"(v), "s"(mask));
+  return r;
+}
+#define LANES_ROW(r) (0xffffull << (16 * (r)))
+
+// The D->D chain of a parser row as an affine scan: lane maps f(x) = P x + C
+// composed over 16-lane rows with DPP, rows joined by readlane carries. The
+// products P depend only on the profile's D->D odds: they are computed once
+// per kernel (AffConst, with the same multiplications in the same order as a
+// per-row computation would make), so a row costs the C recurrence alone.
+struct AffConst {
+  float w1, w2, w4, w8;      // window products the four row steps multiply by
+  float prow;                // product over the row part the lane's window covers after the steps
+  float pa, pb;              // wave-uniform row products used by the row carries
+};
+
+template <int B>
+__device__ __forceinline__ void aff_fwd_setup(AffConst &k, const float (&a)[B])
+{
+  float P = 1.0f;
+#pragma unroll
+  for (int j = 0; j < B; j++) P *= a[j];
+  k.w1 = P; P = P * dppf<ROW_SHR1>(1.0f, P);
+  k.w2 = P; P = P * dppf<ROW_SHR2>(1.0f, P);
+  k.w4 = P; P = P * dppf<ROW_SHR4>(1.0f, P);
+  k.w8 = P; P = P * dppf<ROW_SHR8>(1.0f, P);
+  k.prow = P; k.pa = readlanef(P, 31); k.pb = readlanef(P, 47);
+}
+
+template <int B>
+__device__ __forceinline__ void aff_bck_setup(AffConst &k, const float (&a)[B])
+{
+  float P = 1.0f;
+#pragma unroll
+  for (int j = B-1; j >= 0; j--) P *= a[j];
+  k.w1 = P; P = P * dppf<ROW_SHL1>(1.0f, P);
+  k.w2 = P; P = P * dppf<ROW_SHL2>(1.0f, P);
+  k.w4 = P; P = P * dppf<ROW_SHL4>(1.0f, P);
+  k.w8 = P; P = P * dppf<ROW_SHL8>(1.0f, P);
+  k.prow = P; k.pa = readlanef(P, 32); k.pb = readlanef(P, 16);
+}
+
+template <int B>
+__device__ __forceinline__ void affine_fwd_scan(float (&D)[B], const float (&a)[B], const AffConst &k, int z)
+{
+  // D(j) = D0(j) + a(j) * D(j-1), carried across lanes in increasing k
+  float C = 0.0f;
+#pragma unroll
+  for (int j = 0; j < B; j++) C = D[j] + a[j] * C;
+  C = C + k.w1 * dppz<ROW_SHR1>(C);
+  C = C + k.w2 * dppz<ROW_SHR2>(C);
+  C = C + k.w4 * dppz<ROW_SHR4>(C);
+  C = C + k.w8 * dppz<ROW_SHR8>(C);
+  {
+    const float c1 = readlanef(C, 15);
+    const float c2 = k.pa * c1 + readlanef(C, 31);
+    const float c3 = k.pb * c2 + readlanef(C, 47);
+    const float rc = lane_sel(lane_sel(lane_sel(0.0f, c1, LANES_ROW(1)), c2, LANES_ROW(2)), c3, LANES_ROW(3));
+    C = C + k.prow * rc;
+  }
+  const float cin = dppz<WAVE_SHR1>(C);
+  float cur = cin;
+#pragma unroll
+  for (int j = 0; j < B; j++) { cur = D[j] + a[j] * cur; D[j] = cur; }
+}
+
+// a(j) gives the D->D odds of the lane's position j (read twice per call, so
+// that large models need not hold them in registers through the scan).
+template <int B, typename A>
+__device__ __forceinline__ void affine_bck_scan(float (&D)[B], A a, const AffConst &k, int z)
+{
+  // D(j) = c(j) + a(j) * D(j+1), carried across lanes in decreasing k
+  float C = 0.0f;
+#pragma unroll
+  for (int j = B-1; j >= 0; j--) C = D[j] + a(j) * C;
+  C = C + k.w1 * dppz<ROW_SHL1>(C);
+  C = C + k.w2 * dppz<ROW_SHL2>(C);
+  C = C + k.w4 * dppz<ROW_SHL4>(C);
+  C = C + k.w8 * dppz<ROW_SHL8>(C);
+  {
+    const float c2 = readlanef(C, 48);
+    const float c1 = k.pa * c2 + readlanef(C, 32);
+    const float c0 = k.pb * c1 + readlanef(C, 16);
+    const float rc = lane_sel(lane_sel(lane_sel(0.0f, c2, LANES_ROW(2)), c1, LANES_ROW(1)), c0, LANES_ROW(0));
+    C = C + k.prow * rc;
+  }
+  const float cin = dppz<WAVE_SHL1>(C);
+  float cur = cin;
+#pragma unroll
+  for (int j = B-1; j >= 0; j--) { cur = D[j] + a(j) * cur; D[j] = cur; }
+}
+
+// Forward/Backward: the whole table in LDS up to B = 12 (150 KB); B = 14 reads
+// the table from global memory with transitions pinned in registers;
+// B = 16..48 keep the transitions in LDS (at most 160 KB) and read them per
+// row; B = 64, 80 read everything from global memory per row.
+#define FB_LDS_LIMIT (150 * 1024)
+static inline int fb_mode(const DevProfile &p)
+{
+  if (p.fb_floats * 4 <= FB_LDS_LIMIT && p.fb_floats * 4 <= (size_t) lds_block_limit()) return TM_LDS;
+  if (p.fb_B <= 14) return TM_PIN;
+  if ((size_t) P7G_FB_NT * 64 * p.fb_B * 4 <= (size_t) lds_block_limit()) return TM_TLDS;
+  return TM_GLOB;
+}
+static inline size_t fb_lds(const DevProfile &p, int tm)
+{
+  return (tm == TM_LDS) ? p.fb_floats * 4 : (tm == TM_TLDS) ? (size_t) P7G_FB_NT * 64 * p.fb_B * 4 : 0;
+}
+#define FB_CASES(X) \
+  X(1, TM_LDS) X(2, TM_LDS) X(3, TM_LDS) X(4, TM_LDS) X(5, TM_LDS) X(6, TM_LDS) X(7, TM_LDS) X(8, TM_LDS) \
+  X(10, TM_LDS) X(12, TM_LDS) X(14, TM_PIN) X(16, TM_TLDS) X(20, TM_TLDS) X(24, TM_TLDS) X(28, TM_TLDS) \
+  X(32, TM_TLDS) X(40, TM_TLDS) X(48, TM_TLDS) X(64, TM_GLOB) X(80, TM_GLOB)
