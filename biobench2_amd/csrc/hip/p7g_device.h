@@ -211,24 +211,26 @@ __host__ __device__ inline int64_t md_q(int M) { return (M - 1) / 4 + 1 < 2 ? 2 
 // checkpoints per row of the E state's running sum over the 8Q M and D
 // cells (one at the end of every 64 of them, and the last)
 __host__ __device__ inline int md_ncp(int64_t Q) { return (int) ((8 * Q + 63) / 64); }
-// LDS, in floats: the transitions staged for the Forward (10 rows of M + 2),
-// the Forward's rows, and the traces' buffers (from the start of LDS): a
-// domain's counts (4Q), its null2 odds (32), the trace's domains, the
-// residues' sums
+// LDS, in floats: the transitions staged for the Forward (10 rows of M + 2)
+// and the Forward's rows
 __host__ __device__ inline int64_t md_stage_floats(int M) { return (10 * ((int64_t) M + 2) + 3) & ~(int64_t) 3; }
 __host__ __device__ inline bool md_stage_t(int M) { return (md_stage_floats(M) + 32 * md_q(M)) * 4 <= P7G_LDS_MAX; }
-__host__ __device__ inline int64_t md_acc_at(int64_t Q) { return 4 * Q + 32 + MD_TSEG * 4; }
-// then, when it fits, the emission odds of 20 residues in striped order
-// ([x][q][r]) for the sampled domains' null2
+// the replay's: 64 domains' null2 odds (32 codes each) and records, then per
+// wave a domain's counts (4Q), then, when they fit beside one wave's counts,
+// the emission odds of 20 residues in striped order ([x][q][r])
+#define MD_CHUNK 64
+#define MD_REPLAY_WAVES 8
 __host__ __device__ inline int64_t md_em_floats(int M) { return 20 * 4 * md_q(M); }
-// a launch's room for the residue sums (floats) and the residues (bytes):
-// its longest region's length + 1, rounded up, at most MD_ACC_LDS
-__host__ __device__ inline int md_acc_cap(int max_lr)
-{ const int c = (max_lr + 1 + 63) & ~63; return c < MD_ACC_LDS ? c : MD_ACC_LDS; }
-__host__ __device__ inline bool md_em_lds(int M, int acc_cap)
-{ return (md_acc_at(md_q(M)) + acc_cap + acc_cap / 4 + md_em_floats(M)) * 4 <= P7G_LDS_MAX; }
-__host__ __device__ inline int64_t md_trace_floats(int M, int acc_cap)
-{ return md_acc_at(md_q(M)) + acc_cap + acc_cap / 4 + (md_em_lds(M, acc_cap) ? md_em_floats(M) : 0); }
+__host__ __device__ inline int64_t md_rec_floats() { return MD_CHUNK * 32 + MD_CHUNK * 4 + 8; }
+__host__ __device__ inline bool md_em_lds(int M) { return (md_rec_floats() + 4 * md_q(M) + md_em_floats(M)) * 4 <= P7G_LDS_MAX / 2; }
+__host__ __device__ inline int md_replay_waves(int M)
+{
+  const int64_t room = P7G_LDS_MAX / 2 / 4 - md_rec_floats() - (md_em_lds(M) ? md_em_floats(M) : 0);
+  const int64_t w = room / (4 * md_q(M));
+  return w < 1 ? 1 : w > MD_REPLAY_WAVES ? MD_REPLAY_WAVES : (int) w;
+}
+__host__ __device__ inline int64_t md_replay_floats(int M)
+{ return md_rec_floats() + md_replay_waves(M) * 4 * md_q(M) + (md_em_lds(M) ? md_em_floats(M) : 0); }
 struct MdJob {
   int64_t res_off;
   int64_t area;
@@ -239,23 +241,46 @@ struct MdJob {
 // or 5 (a capacity above was exceeded); nc envelopes ci..cj, 1-based in the
 // region, in start order; nseg the ensemble's size. The region's residues'
 // null2 scores are left at pool + area + md_n2sc_at(M, Lr), residues 1..Lr.
+// rng, trace, wdom, rdom: how far the traces have come (k_md_walk, k_md_replay):
+// the generator's state, traces walked, domains walked and replayed
 struct MdOut {
-  int32_t status, nc, nseg, pad;
+  int32_t status, nc, nseg, done;
+  uint32_t rng;
+  int32_t trace, rtrace, rdom;
   int32_t ci[MD_MAXC], cj[MD_MAXC];
 };
 __host__ __device__ inline int64_t md_n2sc_at(int M, int Lr)
 { return (int64_t) (Lr + 1) * 12 * md_q(M) + 6 * (int64_t) (Lr + 1); }
 // then the endpoint counts, the sampled domains (5 ints each), the
-// clustering's element clusters and cluster counts (segcap ints each), and
-// (doubles) the traces' thresholds: 5 per cell, 3 per row, md_ncp running-sum
-// checkpoints per row
+// clustering's element clusters and cluster counts (segcap ints each; before it
+// where each domain's steps are in the log, and its last row), doubles: the
+// traces' thresholds of each row (3) and md_ncp running-sum checkpoints per row;
+// words: the thresholds of each cell (MD_THR_WORDS); and the walk's log
+#define MD_THR_WORDS 6
 __host__ __device__ inline int64_t md_seg_at(int M, int Lr)
 { return md_n2sc_at(M, Lr) + (Lr + 1) + ((Lr > M ? Lr : M) + 2); }
 __host__ __device__ inline int64_t md_clu_at(int M, int Lr, int segcap)
 { return md_seg_at(M, Lr) + 5 * (int64_t) segcap; }
-__host__ __device__ inline int64_t md_thr_at(int M, int Lr, int segcap)
+__host__ __device__ inline int64_t md_xthr_at(int M, int Lr, int segcap)
 { return (md_clu_at(M, Lr, segcap) + 2 * (int64_t) segcap + 1) & ~(int64_t) 1; }
-size_t  md_lds_bytes(int M, int segcap, int acc_cap);
+__host__ __device__ inline int64_t md_ecum_at(int M, int Lr, int segcap)
+{ return md_xthr_at(M, Lr, segcap) + 2 * 3 * ((int64_t) Lr + 1); }
+__host__ __device__ inline int64_t md_thr_at(int M, int Lr, int segcap)
+{ return md_ecum_at(M, Lr, segcap) + 2 * (int64_t) md_ncp(md_q(M)) * ((int64_t) Lr + 1); }
+__host__ __device__ inline int64_t md_log_at(int M, int Lr, int segcap)
+{ return md_thr_at(M, Lr, segcap) + MD_THR_WORDS * ((int64_t) Lr + 1) * ((int64_t) M + 1); }
+// The log, 16 bits an entry: what one launch of the walk may write, and the
+// most one trace can take. With thresholds of six words instead of five doubles
+// and 8 M Lr entries an area is no larger than it was without a log; traces
+// that find no room are walked by the next of md_passes launches.
+__host__ __device__ inline int64_t md_log_entries(int M, int Lr) { return (int64_t) (M > 4 ? 8 * (int64_t) M : 32) * (Lr + 1) + 64; }
+__host__ __device__ inline int64_t md_log_trace(int M, int Lr) { return (int64_t) (Lr + 1) * (7 + M / 64); }
+__host__ __device__ inline int md_passes(int M, int Lr, int nsamples)
+{
+  const int64_t per = md_log_entries(M, Lr) / md_log_trace(M, Lr);
+  return (int) ((nsamples + (per < 1 ? 1 : per) - 1) / (per < 1 ? 1 : per));
+}
+size_t  md_lds_bytes(int M, int segcap);
 int64_t md_area_floats(int M, int Lr, int segcap);
 // thr_done (optional): recorded on st once the traces' thresholds are filled
 hipError_t launch_md_regions(const DevProfile &p, const uint8_t *res, const MdJob *jobs, MdOut *out, int njobs,

@@ -1,6 +1,6 @@
 // Multidomain regions: region_trace_ensemble (HMMER/src/p7_domaindef.c:600-690)
 // as p7_domaindef_ByPosteriorHeuristics runs it for a region that looks like
-// more than one domain (:431-476). One 64-lane workgroup per region:
+// more than one domain (:431-476), one workgroup per region:
 //
 //  1. p7_Forward over the region's residues with the profile in multihit
 //     mode, length-configured to the whole target, keeping every row
@@ -125,25 +125,17 @@ __device__ __forceinline__ bool md_linked(const MdSeg &a, const MdSeg &b)
 struct MdSig { int c, i, j, k, m; float prob; };
 
 __global__ __launch_bounds__(64) void
-k_md_region(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__restrict__ jobs, MdOut *__restrict__ out,
-            float *__restrict__ pool, int nsamples, uint32_t seed, int phase, int acc_cap)
+k_md_fwd(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__restrict__ jobs, float *__restrict__ pool)
 {
   extern __shared__ float lds[];
   const int z = threadIdx.x;
   const MdJob J = jobs[blockIdx.x];
-  MdOut *O = out + blockIdx.x;
   const int M = p.M, Q = max(2, (M - 1) / 4 + 1), Lr = J.Lr, L = J.Ltarget;
   const int TR = p.nrows;                                  // first transition row of the table
   const float xEmove = p.xfE_move, xEloop = p.xfE_loop, floop = p.xf_loop[L], fmove = p.xf_move[L];
   const uint8_t *dsq = res + J.res_off;                    // residue i (1-based) at dsq[i-1]
   float *mat = pool + J.area;                              // rows 0..Lr, [q][s][r], s = 0 M, 1 D, 2 I
   float *xmx = mat + (size_t) (Lr + 1) * 12 * Q;           // rows 0..Lr: E N J B C SCALE
-  float *acc = xmx + (size_t) 6 * (Lr + 1);                // residues 0..Lr
-  int   *hist = (int *) (acc + (Lr + 1));                  // max(Lr, M) + 2 endpoint counts
-  MdSeg *segs = (MdSeg *) (pool + J.area + md_seg_at(M, Lr));   // the ensemble, J.segcap entries
-  int status = 0;
-#define CELL(i_, q_, s_, r_) mat[(((size_t) (i_) * Q + (q_)) * 3 + (s_)) * 4 + (r_)]
-
   // The profile's transitions, staged in LDS when they fit (md_stage_t): rows
   // BM MM IM DM (into k), MDS DDS (into D_k), MI II, MD DD (out of k), each
   // [k = 0..M+1] with 0 outside 1..M
@@ -151,7 +143,7 @@ k_md_region(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__
   const int TW = M + 2;
   float *tl = lds;
   float *ph = lds + (stage ? md_stage_floats(M) : 0);       // the phases' own LDS
-  if (stage && phase == 0)
+  if (stage)
     for (int c = z; c < 10 * TW; c += 64) tl[c] = md_tv(p, TR + md_trow(c / TW), c % TW);
   auto tv = [&](int row, int k) -> float {                 // row: 0..9 as staged
     if (stage) return tl[row * TW + k];
@@ -160,324 +152,303 @@ k_md_region(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__
   enum { T_BM = 0, T_MM, T_IM, T_DM, T_MDS, T_DDS, T_MI, T_II, T_MD, T_DD };
 
   // ---------------- 1. the region's Forward matrix ----------------
-  if (phase == 0) {
-    float *prev = ph, *cur = ph + 12 * Q, *tdd = ph + 24 * Q, *erow = ph + 28 * Q;   // erow: 4Q emissions
-    __syncthreads();
-    for (int c = z; c < 12 * Q; c += 64) { prev[c] = 0.0f; mat[c] = 0.0f; }
-    for (int c = z; c < 4 * Q; c += 64) tdd[c] = tv(T_DD, min((c & 3) * Q + (c >> 2) + 1, M + 1));
-    float xN = 1.0f, xJ = 0.0f, xB = fmove, xC = 0.0f, xE = 0.0f;
-    if (z == 0) { xmx[0] = 0.0f; xmx[1] = xN; xmx[2] = xJ; xmx[3] = xB; xmx[4] = xC; xmx[5] = 1.0f; }
-    __syncthreads();
-    // a row's odds in striped order, eight per lane: loaded one row ahead
-    // while the row before is computed (models up to M = 512; larger ones load
-    // theirs at the row)
-    const bool pre = 4 * Q <= 64 * 8;
-    float enext[8];
-    auto load_row = [&](int i1) {
-      const int x = dsq[i1 - 1];
+  float *prev = ph, *cur = ph + 12 * Q, *tdd = ph + 24 * Q, *erow = ph + 28 * Q;   // erow: 4Q emissions
+  __syncthreads();
+  for (int c = z; c < 12 * Q; c += 64) { prev[c] = 0.0f; mat[c] = 0.0f; }
+  for (int c = z; c < 4 * Q; c += 64) tdd[c] = tv(T_DD, min((c & 3) * Q + (c >> 2) + 1, M + 1));
+  float xN = 1.0f, xJ = 0.0f, xB = fmove, xC = 0.0f, xE = 0.0f;
+  if (z == 0) { xmx[0] = 0.0f; xmx[1] = xN; xmx[2] = xJ; xmx[3] = xB; xmx[4] = xC; xmx[5] = 1.0f; }
+  __syncthreads();
+  // a row's odds in striped order, eight per lane: loaded one row ahead
+  // while the row before is computed (models up to M = 512; larger ones load
+  // theirs at the row)
+  const bool pre = 4 * Q <= 64 * 8;
+  float enext[8];
+  auto load_row = [&](int i1) {
+    const int x = dsq[i1 - 1];
 #pragma unroll
-      for (int u = 0; u < 8; u++) { const int c = u * 64 + z; enext[u] = md_tv(p, x, (c & 3) * Q + (c >> 2) + 1); }
-    };
-    // with the row's odds in registers (pre), lane z's cells are c = 64 u + z
-    // for u < 8, and their transitions are the row loop's constants: in
-    // registers too
-    float ecur[8], tBMr[8], tMMr[8], tIMr[8], tDMr[8], tMIr[8], tIIr[8], tMDr[8];
+    for (int u = 0; u < 8; u++) { const int c = u * 64 + z; enext[u] = md_tv(p, x, (c & 3) * Q + (c >> 2) + 1); }
+  };
+  // with the row's odds in registers (pre), lane z's cells are c = 64 u + z
+  // for u < 8, and their transitions are the row loop's constants: in
+  // registers too
+  float ecur[8], tBMr[8], tMMr[8], tIMr[8], tDMr[8], tMIr[8], tIIr[8], tMDr[8];
+  if (pre) {
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int c = u * 64 + z, q = c >> 2, r = c & 3, k = r * Q + q + 1, kk = min(k, M + 1);
+      const bool in = c < 4 * Q;
+      tBMr[u] = in ? tv(T_BM, kk) : 0.0f; tMMr[u] = in ? tv(T_MM, kk) : 0.0f;
+      tIMr[u] = in ? tv(T_IM, kk) : 0.0f; tDMr[u] = in ? tv(T_DM, kk) : 0.0f;
+      tMIr[u] = in ? tv(T_MI, kk) : 0.0f; tIIr[u] = in ? tv(T_II, kk) : 0.0f;
+      tMDr[u] = in ? tv(T_MD, min(k - 1, M + 1)) : 0.0f;
+    }
+    load_row(1);
+  }
+  for (int i = 1; i <= Lr; i++) {
+    if (pre) {
+#pragma unroll
+      for (int u = 0; u < 8; u++) ecur[u] = enext[u];
+      if (i < Lr) load_row(i + 1);
+    } else {
+      const int x = dsq[i - 1];
+      for (int c0 = 0; c0 < 4 * Q; c0 += 64 * 8) {         // this residue's odds, striped order
+        float e[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) { const int c = c0 + u * 64 + z; e[u] = md_tv(p, x, (c & 3) * Q + (c >> 2) + 1); }
+#pragma unroll
+        for (int u = 0; u < 8; u++) { const int c = c0 + u * 64 + z; if (c < 4 * Q) erow[c] = e[u]; }
+      }
+    }
+    md_sync();
     if (pre) {
 #pragma unroll
       for (int u = 0; u < 8; u++) {
-        const int c = u * 64 + z, q = c >> 2, r = c & 3, k = r * Q + q + 1, kk = min(k, M + 1);
-        const bool in = c < 4 * Q;
-        tBMr[u] = in ? tv(T_BM, kk) : 0.0f; tMMr[u] = in ? tv(T_MM, kk) : 0.0f;
-        tIMr[u] = in ? tv(T_IM, kk) : 0.0f; tDMr[u] = in ? tv(T_DM, kk) : 0.0f;
-        tMIr[u] = in ? tv(T_MI, kk) : 0.0f; tIIr[u] = in ? tv(T_II, kk) : 0.0f;
-        tMDr[u] = in ? tv(T_MD, min(k - 1, M + 1)) : 0.0f;
-      }
-      load_row(1);
-    }
-    for (int i = 1; i <= Lr; i++) {
-      if (pre) {
-#pragma unroll
-        for (int u = 0; u < 8; u++) ecur[u] = enext[u];
-        if (i < Lr) load_row(i + 1);
-      } else {
-        const int x = dsq[i - 1];
-        for (int c0 = 0; c0 < 4 * Q; c0 += 64 * 8) {         // this residue's odds, striped order
-          float e[8];
-#pragma unroll
-          for (int u = 0; u < 8; u++) { const int c = c0 + u * 64 + z; e[u] = md_tv(p, x, (c & 3) * Q + (c >> 2) + 1); }
-#pragma unroll
-          for (int u = 0; u < 8; u++) { const int c = c0 + u * 64 + z; if (c < 4 * Q) erow[c] = e[u]; }
+        const int c = u * 64 + z, q = c >> 2, r = c & 3;
+        if (c < 4 * Q) {
+          float mp = 0.0f, dp = 0.0f, ip = 0.0f;       // row i-1 at k-1 (esl_sse_rightshift_ps at q = 0)
+          if (q > 0)      { mp = prev[((q-1)*3+0)*4 + r]; dp = prev[((q-1)*3+1)*4 + r]; ip = prev[((q-1)*3+2)*4 + r]; }
+          else if (r > 0) { mp = prev[((Q-1)*3+0)*4 + r-1]; dp = prev[((Q-1)*3+1)*4 + r-1]; ip = prev[((Q-1)*3+2)*4 + r-1]; }
+          float sv = __fmul_rn(xB, tBMr[u]);
+          sv = __fadd_rn(sv, __fmul_rn(mp, tMMr[u]));
+          sv = __fadd_rn(sv, __fmul_rn(ip, tIMr[u]));
+          sv = __fadd_rn(sv, __fmul_rn(dp, tDMr[u]));
+          sv = __fmul_rn(sv, ecur[u]);
+          cur[(q*3+0)*4 + r] = sv;
+          cur[(q*3+2)*4 + r] = __fadd_rn(__fmul_rn(prev[(q*3+0)*4 + r], tMIr[u]),
+                                         __fmul_rn(prev[(q*3+2)*4 + r], tIIr[u]));
         }
-      }
-      md_sync();
-      if (pre) {
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int c = u * 64 + z, q = c >> 2, r = c & 3;
-          if (c < 4 * Q) {
-            float mp = 0.0f, dp = 0.0f, ip = 0.0f;       // row i-1 at k-1 (esl_sse_rightshift_ps at q = 0)
-            if (q > 0)      { mp = prev[((q-1)*3+0)*4 + r]; dp = prev[((q-1)*3+1)*4 + r]; ip = prev[((q-1)*3+2)*4 + r]; }
-            else if (r > 0) { mp = prev[((Q-1)*3+0)*4 + r-1]; dp = prev[((Q-1)*3+1)*4 + r-1]; ip = prev[((Q-1)*3+2)*4 + r-1]; }
-            float sv = __fmul_rn(xB, tBMr[u]);
-            sv = __fadd_rn(sv, __fmul_rn(mp, tMMr[u]));
-            sv = __fadd_rn(sv, __fmul_rn(ip, tIMr[u]));
-            sv = __fadd_rn(sv, __fmul_rn(dp, tDMr[u]));
-            sv = __fmul_rn(sv, ecur[u]);
-            cur[(q*3+0)*4 + r] = sv;
-            cur[(q*3+2)*4 + r] = __fadd_rn(__fmul_rn(prev[(q*3+0)*4 + r], tMIr[u]),
-                                           __fmul_rn(prev[(q*3+2)*4 + r], tIIr[u]));
-          }
-        }
-        md_sync();
-        // D before the D->D passes: cell q holds M(q-1)·tMD (the q loop's dcv); q = 0 holds 0
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int c = u * 64 + z, q = c >> 2, r = c & 3;
-          if (c < 4 * Q) cur[(q*3+1)*4 + r] = q ? __fmul_rn(cur[((q-1)*3+0)*4 + r], tMDr[u]) : 0.0f;
-        }
-      } else {
-      for (int c = z; c < 4 * Q; c += 64) {
-        const int q = c >> 2, r = c & 3, k = r * Q + q + 1, kk = min(k, M + 1);
-        float mp = 0.0f, dp = 0.0f, ip = 0.0f;           // row i-1 at k-1 (esl_sse_rightshift_ps at q = 0)
-        if (q > 0)      { mp = prev[((q-1)*3+0)*4 + r]; dp = prev[((q-1)*3+1)*4 + r]; ip = prev[((q-1)*3+2)*4 + r]; }
-        else if (r > 0) { mp = prev[((Q-1)*3+0)*4 + r-1]; dp = prev[((Q-1)*3+1)*4 + r-1]; ip = prev[((Q-1)*3+2)*4 + r-1]; }
-        float sv = __fmul_rn(xB, tv(T_BM, kk));
-        sv = __fadd_rn(sv, __fmul_rn(mp, tv(T_MM, kk)));
-        sv = __fadd_rn(sv, __fmul_rn(ip, tv(T_IM, kk)));
-        sv = __fadd_rn(sv, __fmul_rn(dp, tv(T_DM, kk)));
-        sv = __fmul_rn(sv, erow[c]);
-        cur[(q*3+0)*4 + r] = sv;
-        cur[(q*3+2)*4 + r] = __fadd_rn(__fmul_rn(prev[(q*3+0)*4 + r], tv(T_MI, kk)),
-                                       __fmul_rn(prev[(q*3+2)*4 + r], tv(T_II, kk)));
       }
       md_sync();
       // D before the D->D passes: cell q holds M(q-1)·tMD (the q loop's dcv); q = 0 holds 0
-      for (int c = z; c < 4 * Q; c += 64) {
-        const int q = c >> 2, r = c & 3, k = r * Q + q + 1;
-        cur[(q*3+1)*4 + r] = q ? __fmul_rn(cur[((q-1)*3+0)*4 + r], tv(T_MD, min(k - 1, M + 1))) : 0.0f;
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const int c = u * 64 + z, q = c >> 2, r = c & 3;
+        if (c < 4 * Q) cur[(q*3+1)*4 + r] = q ? __fmul_rn(cur[((q-1)*3+0)*4 + r], tMDr[u]) : 0.0f;
       }
+    } else {
+    for (int c = z; c < 4 * Q; c += 64) {
+      const int q = c >> 2, r = c & 3, k = r * Q + q + 1, kk = min(k, M + 1);
+      float mp = 0.0f, dp = 0.0f, ip = 0.0f;           // row i-1 at k-1 (esl_sse_rightshift_ps at q = 0)
+      if (q > 0)      { mp = prev[((q-1)*3+0)*4 + r]; dp = prev[((q-1)*3+1)*4 + r]; ip = prev[((q-1)*3+2)*4 + r]; }
+      else if (r > 0) { mp = prev[((Q-1)*3+0)*4 + r-1]; dp = prev[((Q-1)*3+1)*4 + r-1]; ip = prev[((Q-1)*3+2)*4 + r-1]; }
+      float sv = __fmul_rn(xB, tv(T_BM, kk));
+      sv = __fadd_rn(sv, __fmul_rn(mp, tv(T_MM, kk)));
+      sv = __fadd_rn(sv, __fmul_rn(ip, tv(T_IM, kk)));
+      sv = __fadd_rn(sv, __fmul_rn(dp, tv(T_DM, kk)));
+      sv = __fmul_rn(sv, erow[c]);
+      cur[(q*3+0)*4 + r] = sv;
+      cur[(q*3+2)*4 + r] = __fadd_rn(__fmul_rn(prev[(q*3+0)*4 + r], tv(T_MI, kk)),
+                                     __fmul_rn(prev[(q*3+2)*4 + r], tv(T_II, kk)));
+    }
+    md_sync();
+    // D before the D->D passes: cell q holds M(q-1)·tMD (the q loop's dcv); q = 0 holds 0
+    for (int c = z; c < 4 * Q; c += 64) {
+      const int q = c >> 2, r = c & 3, k = r * Q + q + 1;
+      cur[(q*3+1)*4 + r] = q ? __fmul_rn(cur[((q-1)*3+0)*4 + r], tv(T_MD, min(k - 1, M + 1))) : 0.0f;
+    }
+    }
+    md_sync();
+    float xe = 0.0f;
+    if (z < 4) {                                         // lane z is SSE lane r
+      // The row's sums along q and its D->D passes, each a chain in q order
+      // (esl_sse_hsum_ps's lanes, fwdback.c's D passes): M(q) at cm[12 q],
+      // D(q) at cd[12 q], tDD(q) at tq[4 q]. Eight cells at a time, the next
+      // eight's loads issued before this eight's chain. The M sum and the
+      // first pass are independent chains and run together; every later
+      // pass also sums its new D values onto the M sum, so that the last
+      // pass leaves the row's total (its D values are the final ones).
+      const int r = z;
+      float *cm = cur + r, *cd = cur + 4 + r;
+      const float *tq = tdd + r;
+      float dcv = __fmul_rn(cur[((Q-1)*3+0)*4 + r], tv(T_MD, min(r * Q + Q, M + 1)));
+      float sh = __shfl(dcv, (z + 3) & 3, 4);
+      dcv = r ? sh : 0.0f;
+      // Reads past the row's last q stay inside the phase's LDS (the next
+      // buffers) and feed no result.
+      float xm = 0.0f;
+      {
+        // two chunk buffers in turn: the next chunk loads into one while
+        // the other's chain runs
+        float am[8], ad[8], at[8], bm[8], bd[8], bt[8];
+        auto ld = [&](int q0, float (&m)[8], float (&d)[8], float (&t)[8]) {
+#pragma unroll
+          for (int u = 0; u < 8; u++) { m[u] = cm[12*(q0+u)]; d[u] = cd[12*(q0+u)]; t[u] = tq[4*(q0+u)]; }
+        };
+        auto run = [&](int q0, const float (&m)[8], const float (&d)[8], const float (&t)[8]) {
+          auto step = [&](int u) {
+            xm = __fadd_rn(xm, m[u]);
+            const float dd = __fadd_rn(dcv, d[u]);
+            dcv = __fmul_rn(dd, t[u]);
+            cd[12*(q0+u)] = dd;
+          };
+          if (q0 + 8 <= Q) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) step(u);
+          } else {
+#pragma unroll
+            for (int u = 0; u < 8; u++) if (q0 + u < Q) step(u);
+          }
+        };
+        ld(0, am, ad, at);
+        for (int q0 = 0; q0 < Q; q0 += 16) {
+          if (q0 + 8 < Q) ld(q0 + 8, bm, bd, bt);
+          run(q0, am, ad, at);
+          if (q0 + 8 >= Q) break;
+          if (q0 + 16 < Q) ld(q0 + 16, am, ad, at);
+          run(q0 + 8, bm, bd, bt);
+        }
       }
-      md_sync();
-      float xe = 0.0f;
-      if (z < 4) {                                         // lane z is SSE lane r
-        // The row's sums along q and its D->D passes, each a chain in q order
-        // (esl_sse_hsum_ps's lanes, fwdback.c's D passes): M(q) at cm[12 q],
-        // D(q) at cd[12 q], tDD(q) at tq[4 q]. Eight cells at a time, the next
-        // eight's loads issued before this eight's chain. The M sum and the
-        // first pass are independent chains and run together; every later
-        // pass also sums its new D values onto the M sum, so that the last
-        // pass leaves the row's total (its D values are the final ones).
-        const int r = z;
-        float *cm = cur + r, *cd = cur + 4 + r;
-        const float *tq = tdd + r;
-        float dcv = __fmul_rn(cur[((Q-1)*3+0)*4 + r], tv(T_MD, min(r * Q + Q, M + 1)));
-        float sh = __shfl(dcv, (z + 3) & 3, 4);
+      for (int pass = 1; pass < 4; pass++) {
+        sh = __shfl(dcv, (z + 3) & 3, 4);
         dcv = r ? sh : 0.0f;
-        // Reads past the row's last q stay inside the phase's LDS (the next
-        // buffers) and feed no result.
-        float xm = 0.0f;
-        {
-          // two chunk buffers in turn: the next chunk loads into one while
-          // the other's chain runs
-          float am[8], ad[8], at[8], bm[8], bd[8], bt[8];
-          auto ld = [&](int q0, float (&m)[8], float (&d)[8], float (&t)[8]) {
+        int changed = 0;
+        float xd = xm;
+        float ad[8], at[8], bd[8], bt[8];
+        auto ld = [&](int q0, float (&d)[8], float (&t)[8]) {
 #pragma unroll
-            for (int u = 0; u < 8; u++) { m[u] = cm[12*(q0+u)]; d[u] = cd[12*(q0+u)]; t[u] = tq[4*(q0+u)]; }
+          for (int u = 0; u < 8; u++) { d[u] = cd[12*(q0+u)]; t[u] = tq[4*(q0+u)]; }
+        };
+        auto run = [&](int q0, const float (&d)[8], const float (&t)[8]) {
+          auto step = [&](int u) {
+            const float dd = __fadd_rn(dcv, d[u]);
+            changed |= (dd > d[u]);
+            dcv = __fmul_rn(dcv, t[u]);
+            xd = __fadd_rn(dd, xd);
+            cd[12*(q0+u)] = dd;
           };
-          auto run = [&](int q0, const float (&m)[8], const float (&d)[8], const float (&t)[8]) {
-            auto step = [&](int u) {
-              xm = __fadd_rn(xm, m[u]);
-              const float dd = __fadd_rn(dcv, d[u]);
-              dcv = __fmul_rn(dd, t[u]);
-              cd[12*(q0+u)] = dd;
-            };
-            if (q0 + 8 <= Q) {
+          if (q0 + 8 <= Q) {
 #pragma unroll
-              for (int u = 0; u < 8; u++) step(u);
-            } else {
+            for (int u = 0; u < 8; u++) step(u);
+          } else {
 #pragma unroll
-              for (int u = 0; u < 8; u++) if (q0 + u < Q) step(u);
-            }
-          };
-          ld(0, am, ad, at);
-          for (int q0 = 0; q0 < Q; q0 += 16) {
-            if (q0 + 8 < Q) ld(q0 + 8, bm, bd, bt);
-            run(q0, am, ad, at);
-            if (q0 + 8 >= Q) break;
-            if (q0 + 16 < Q) ld(q0 + 16, am, ad, at);
-            run(q0 + 8, bm, bd, bt);
+            for (int u = 0; u < 8; u++) if (q0 + u < Q) step(u);
           }
+        };
+        ld(0, ad, at);
+        for (int q0 = 0; q0 < Q; q0 += 16) {
+          if (q0 + 8 < Q) ld(q0 + 8, bd, bt);
+          run(q0, ad, at);
+          if (q0 + 8 >= Q) break;
+          if (q0 + 16 < Q) ld(q0 + 16, ad, at);
+          run(q0 + 8, bd, bt);
         }
-        for (int pass = 1; pass < 4; pass++) {
-          sh = __shfl(dcv, (z + 3) & 3, 4);
-          dcv = r ? sh : 0.0f;
-          int changed = 0;
-          float xd = xm;
-          float ad[8], at[8], bd[8], bt[8];
-          auto ld = [&](int q0, float (&d)[8], float (&t)[8]) {
-#pragma unroll
-            for (int u = 0; u < 8; u++) { d[u] = cd[12*(q0+u)]; t[u] = tq[4*(q0+u)]; }
-          };
-          auto run = [&](int q0, const float (&d)[8], const float (&t)[8]) {
-            auto step = [&](int u) {
-              const float dd = __fadd_rn(dcv, d[u]);
-              changed |= (dd > d[u]);
-              dcv = __fmul_rn(dcv, t[u]);
-              xd = __fadd_rn(dd, xd);
-              cd[12*(q0+u)] = dd;
-            };
-            if (q0 + 8 <= Q) {
-#pragma unroll
-              for (int u = 0; u < 8; u++) step(u);
-            } else {
-#pragma unroll
-              for (int u = 0; u < 8; u++) if (q0 + u < Q) step(u);
-            }
-          };
-          ld(0, ad, at);
-          for (int q0 = 0; q0 < Q; q0 += 16) {
-            if (q0 + 8 < Q) ld(q0 + 8, bd, bt);
-            run(q0, ad, at);
-            if (q0 + 8 >= Q) break;
-            if (q0 + 16 < Q) ld(q0 + 16, ad, at);
-            run(q0 + 8, bd, bt);
-          }
-          xe = xd;
-          const bool any = (__ballot(changed) & 0xfull) != 0ull;
-          if (M >= 100 && ! any) break;
-        }
+        xe = xd;
+        const bool any = (__ballot(changed) & 0xfull) != 0ull;
+        if (M >= 100 && ! any) break;
       }
-      // esl_sse_hsum_ps: (e0 + e1) + (e2 + e3)
-      xE = __fadd_rn(__fadd_rn(readlanef(xe, 0), readlanef(xe, 1)), __fadd_rn(readlanef(xe, 2), readlanef(xe, 3)));
-      xN = __fmul_rn(xN, floop);
-      xC = __fadd_rn(__fmul_rn(xC, floop), __fmul_rn(xE, xEmove));
-      xJ = __fadd_rn(__fmul_rn(xJ, floop), __fmul_rn(xE, xEloop));
-      xB = __fadd_rn(__fmul_rn(xJ, fmove), __fmul_rn(xN, fmove));
-      float scale = 1.0f;
-      md_sync();
-      if (xE > 1.0e4f) {
-        xN = __fdiv_rn(xN, xE); xC = __fdiv_rn(xC, xE); xJ = __fdiv_rn(xJ, xE); xB = __fdiv_rn(xB, xE);
-        const float inv = (float) (1.0 / (double) xE);
-        for (int c = z; c < 12 * Q; c += 64) cur[c] = __fmul_rn(cur[c], inv);
-        scale = xE;
-        xE = 1.0f;
-        md_sync();
-      }
-      float *row = mat + (size_t) i * 12 * Q;
-      for (int c = z; c < 12 * Q; c += 64) row[c] = cur[c];
-      if (z == 0) {
-        float *xr = xmx + (size_t) i * 6;
-        xr[0] = xE; xr[1] = xN; xr[2] = xJ; xr[3] = xB; xr[4] = xC; xr[5] = scale;
-      }
-      float *t = prev; prev = cur; cur = t;
+    }
+    // esl_sse_hsum_ps: (e0 + e1) + (e2 + e3)
+    xE = __fadd_rn(__fadd_rn(readlanef(xe, 0), readlanef(xe, 1)), __fadd_rn(readlanef(xe, 2), readlanef(xe, 3)));
+    xN = __fmul_rn(xN, floop);
+    xC = __fadd_rn(__fmul_rn(xC, floop), __fmul_rn(xE, xEmove));
+    xJ = __fadd_rn(__fmul_rn(xJ, floop), __fmul_rn(xE, xEloop));
+    xB = __fadd_rn(__fmul_rn(xJ, fmove), __fmul_rn(xN, fmove));
+    float scale = 1.0f;
+    md_sync();
+    if (xE > 1.0e4f) {
+      xN = __fdiv_rn(xN, xE); xC = __fdiv_rn(xC, xE); xJ = __fdiv_rn(xJ, xE); xB = __fdiv_rn(xB, xE);
+      const float inv = (float) (1.0 / (double) xE);
+      for (int c = z; c < 12 * Q; c += 64) cur[c] = __fmul_rn(cur[c], inv);
+      scale = xE;
+      xE = 1.0f;
       md_sync();
     }
-    __syncthreads();                                       // the matrix in global memory, for every lane
-    return;
+    float *row = mat + (size_t) i * 12 * Q;
+    for (int c = z; c < 12 * Q; c += 64) row[c] = cur[c];
+    if (z == 0) {
+      float *xr = xmx + (size_t) i * 6;
+      xr[0] = xE; xr[1] = xN; xr[2] = xJ; xr[3] = xB; xr[4] = xC; xr[5] = scale;
+    }
+    float *t = prev; prev = cur; cur = t;
+    md_sync();
   }
+}
 
-  // ---------------- 2. the sampled traces ----------------
-  // (their thresholds were filled by k_md_thr, md_thr_fill)
-  double *thr = (double *) (pool + J.area + md_thr_at(M, Lr, J.segcap));
-  double *xthr = thr + (size_t) 5 * (Lr + 1) * (M + 1);
-  double *ecum = xthr + (size_t) 3 * (Lr + 1);
-  // LDS: a domain's counts, its null2 odds, the trace's domains, and the
-  // residues' odds sums when the region is short
-  float *cnt = lds;                                        // [q][r] counts of one sampled domain
-  float *n2v = lds + 4 * Q;                                // its null2 odds, 32 codes
-  int   *tseg = (int *) (n2v + 32);                        // this trace's domains, last first
-  const bool acc_lds = (Lr + 1) <= acc_cap;
-  float *accp = acc_lds ? lds + md_acc_at(Q) : acc;        // residue sums
-  uint8_t *rl = (uint8_t *) (lds + md_acc_at(Q) + acc_cap);   // and the residues, with them in LDS
-  const uint8_t *rsq = acc_lds ? rl : dsq;
-  auto cnt_at = [&](int k) {                               // the count cell of model position k
-    const int r = (k - 1 >= Q) + (k - 1 >= 2 * Q) + (k - 1 >= 3 * Q);
-    return (k - 1 - r * Q) * 4 + r; };
-  const bool em_lds = md_em_lds(M, acc_cap) && p.K <= 20;
-  float *em = lds + md_acc_at(Q) + acc_cap + acc_cap / 4;  // [x][q][r] odds, when em_lds
-  if (em_lds)
-    for (int c = z; c < p.K * 4 * Q; c += 64) {
-      const int x = c / (4 * Q), rem = c - x * 4 * Q;
-      em[c] = md_tv(p, x, min((rem & 3) * Q + (rem >> 2) + 1, M + 1));
-    }
-  for (int c = z; c < 4 * Q; c += 64) cnt[c] = 0.0f;
-  for (int pos = z; pos <= Lr; pos += 64) accp[pos] = 0.0f;
-  if (acc_lds) for (int pos = z; pos < Lr; pos += 64) rl[pos] = dsq[pos];
-  __syncthreads();
-  uint32_t rng = md_mix3(seed, 87654321u, 12345678u);
-  if (rng == 0) rng = 42;
+// The comparison of a draw x with a threshold th in (0, 1], as the walk makes
+// it on integers: x / 2^32 < th is x < T, T = ceil(2^32 th), or always when T is
+// 2^32 (bit a of the cell's flags). T = 0 for thresholds that no draw is under,
+// NaN among them.
+__device__ __forceinline__ uint32_t md_thr_word(double th, int a, uint32_t &flags)
+{
+  const double v = ceil(th * 4294967296.0);
+  if (! (v >= 1.0)) return 0u;
+  if (v > 4294967295.0) { flags |= 1u << a; return 0u; }
+  return (uint32_t) v;
+}
+enum { MD_NAN_M = 5, MD_NAN_D = 6, MD_NAN_I = 7 };         // flag bits: the cell's weights gave NaN
+
+// The traces' walks: one wave per region. A walk is a chain of dependent
+// steps, each a random draw against the thresholds of the state it is in, and
+// its loads' latency bounds the stage: nothing else is done here. In a state
+// that can repeat (M along its diagonal, D along its row, I, C and J down their
+// column) lane l takes the step that follows l repeats, with the (l+1)-th draw
+// from here (the generator's jump) and that cell's thresholds; the first lane
+// whose step leaves the state (or fails) is the step the walk takes after those
+// repeats. What a sampled domain's steps mean (its counts, null2 odds, ends) is
+// left to k_md_replay, for which each run goes to the log: bits 0-6 the
+// repeats, 7-9 the state it leads to (0: the run goes on), 10 whether that I
+// or D state steps back to M at once; a domain starts with its last node and
+// state. 60 regions of up to 600 residues, walk + replay: M = 86 3.3 + 1.7 ms,
+// M = 400 6.2 + 1.2 ms; with the steps' bookkeeping and the null2 sums of each
+// domain in the walk's chain, one wave a region, it was 9.1 and 13.7 ms.
+__global__ __launch_bounds__(64) void
+k_md_walk(const DevProfile p, const MdJob *__restrict__ jobs, MdOut *__restrict__ out, float *__restrict__ pool,
+          int nsamples, uint32_t seed, int first)
+{
+  const int z = threadIdx.x;
+  const MdJob J = jobs[blockIdx.x];
+  MdOut *O = out + blockIdx.x;
+  const int M = p.M, Q = max(2, (M - 1) / 4 + 1), Lr = J.Lr;
+  float *area = pool + J.area;
+  const float *mat = area, *xmx = mat + (size_t) (Lr + 1) * 12 * Q;
+  const double *xthr = (const double *) (area + md_xthr_at(M, Lr, J.segcap));
+  const double *ecum = (const double *) (area + md_ecum_at(M, Lr, J.segcap));
+  const uint2 *thr = (const uint2 *) (area + md_thr_at(M, Lr, J.segcap));
+  uint16_t *lg = (uint16_t *) (area + md_log_at(M, Lr, J.segcap));
+  MdSeg *segs = (MdSeg *) (area + md_seg_at(M, Lr));
+  int *dlog = (int *) (area + md_clu_at(M, Lr, J.segcap)), *drow = dlog + J.segcap;
+  uint32_t rng;
+  int t = 0, nseg = 0, status = 0;
+  if (first) {
+    rng = md_mix3(seed, 87654321u, 12345678u);
+    if (rng == 0) rng = 42;
+  } else {
+    status = O->status; t = O->trace; nseg = O->nseg; rng = O->rng;
+    if (status || t >= nsamples) return;
+  }
+  rng = (uint32_t) uni((int) rng); t = uni(t); nseg = uni(nseg);
   // lane l's jump: l + 1 draws of x -> 69069 x + 1 are x -> jA x + jC
   uint32_t jA = 1u, jC = 0u;
   for (int l = 0; l <= z; l++) { jA *= 69069u; jC = jC * 69069u + 1u; }
-  int nseg = 0;
   const int64_t max_steps = 64 * ((int64_t) Lr + M + 16);
-  for (int t = 0; t < nsamples && ! status; t++) {
-    int s0 = MS_C, i = Lr, k = 0, hi = Lr, nd = 0;
-    int sqfrom = 0, sqto = 0, hmmfrom = 0, hmmto = 0, Ld = 0, kmin = 0x7fffffff, kmax = 0;
+  const int64_t log_end = md_log_entries(M, Lr) - md_log_trace(M, Lr);
+  int lbuf = 0;                                            // lane u: the log's entry n with n mod 64 = u
+  int n = 0;
+  auto put = [&](int v) {
+    lbuf = (z == (n & 63)) ? v : lbuf;
+    if ((n & 63) == 63) lg[n - 63 + z] = (uint16_t) lbuf;
+    n++;
+  };
+  for (; t < nsamples && ! status && n <= log_end; t++) {
+    int i = Lr, k = 0, nd = 0;
     int64_t steps = 0;
-    while (s0 != MS_S) {
-      int s1 = -1;
-      bool back = false;                                   // s1 (I or D) steps back to M at once
-      if (s0 == MS_M || s0 == MS_D || s0 == MS_I || s0 == MS_C || s0 == MS_J) {
-        // A state that can repeat: M along its diagonal, D along its row, I,
-        // C and J down their column. Lane l takes the step that follows l
-        // repeats, with the (l+1)-th draw from here and that cell's
-        // thresholds; the first lane whose step leaves the state (or fails)
-        // is the step the walk takes after those repeats.
+    bool over = false;
+    int col = 0;                                           // 0 the C state, 1 J
+    for (;;) {
+      // down C's or J's column to an E
+      for (;;) {
         const uint32_t xl = jA * rng + jC;
         const double roll = (double) xl / 4294967296.0;
-        const int li = (s0 == MS_D) ? i : i - z, lk = (s0 == MS_M) ? k - z : (s0 == MS_D) ? k - z : k;
-        int sl = -1;
-        // An M run's step to I or D is most often followed by one step back
-        // to M. Lane l also takes that step ahead, as if it stopped here:
-        // the I or D cell is lane l+1's, whose thresholds that lane loads
-        // anyway, and the draw the next one. spec: that step leads to M
-        // (and its M cell is inside the matrix).
-        bool spec = false;
-        if (s0 == MS_C || s0 == MS_J) {
-          if (li >= 1) {
-            const double th = xthr[(size_t) li * 3 + (s0 == MS_J)];
-            sl = (roll < th) ? s0 : (th == th) ? MS_E : -1;
-          }
-        } else if (s0 == MS_M) {
-          const bool in = (li >= 1 && lk >= 1);
-          double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0, t4 = 0.0;
-          if (in) {
-            const double *th = thr + ((size_t) li * (M + 1) + lk) * 5;
-            t0 = th[0]; t1 = th[1]; t2 = th[2]; t3 = th[3]; t4 = th[4];
-            sl = (roll < t0) ? MS_B : (roll < t1) ? MS_M : (roll < t2) ? MS_I : (t0 == t0) ? MS_D : -1;
-          }
-          const double n3 = __shfl_down(t3, 1, 64), n4 = __shfl_down(t4, 1, 64);   // cell (li - 1, lk - 1)
-          const bool nin = __shfl_down((int) in, 1, 64) != 0 && z < 63;
-          if (nin && (sl == MS_I || sl == MS_D)) {
-            const double tt = (sl == MS_I) ? n4 : n3;
-            const double roll2 = (double) (69069u * xl + 1u) / 4294967296.0;
-            // back to M at (li - 2, lk - 1) from I, (li - 1, lk - 2) from D
-            spec = (roll2 < tt) && ((sl == MS_I) ? li - 2 >= 1 : lk - 2 >= 1);
-          }
-        } else if (li >= 1 && lk >= 1) {
-          const double *th = thr + ((size_t) li * (M + 1) + lk) * 5;
-          const double tt = th[(s0 == MS_D) ? 3 : 4];
-          sl = (roll < tt) ? MS_M : (tt == tt) ? s0 : -1;
+        const int li = i - z;
+        int sl = -1;                                       // 0 stays, 1 E
+        if (li >= 1) {
+          const double th = xthr[(size_t) li * 3 + col];
+          sl = (roll < th) ? 0 : (th == th) ? 1 : -1;
         }
-        const unsigned long long stop = __ballot(sl != s0);
+        const unsigned long long stop = __ballot(sl != 0);
         const int f = stop ? (int) __ffsll((long long) stop) - 1 : 64;
-        if (f > 0) {                                       // the repeats: M and I states emit
-          if (s0 == MS_M) {
-            if (z < f) atomicAdd(&cnt[cnt_at(k - 1 - z)], 1.0f);
-            kmin = min(kmin, k - f); kmax = max(kmax, k - 1);
-            Ld += f;
-            if (sqto == 0) { sqto = i - 1; hmmto = k - 1; }
-            sqfrom = i - f; hmmfrom = k - f;
-            i -= f; k -= f;
-          } else if (s0 == MS_I) {
-            if (z == 0) atomicAdd(&cnt[cnt_at(k)], (float) f);
-            kmin = min(kmin, k); kmax = max(kmax, k);
-            Ld += f;
-            i -= f;
-          } else if (s0 == MS_D) k -= f;
-          else i -= f;
-        }
+        i -= f;
         steps += f;
         if (f == 64) {
           rng = (uint32_t) __builtin_amdgcn_readlane((int) xl, 63);
@@ -485,196 +456,347 @@ k_md_region(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__
           continue;
         }
         rng = (uint32_t) __builtin_amdgcn_readlane((int) xl, f);
-        s1 = __builtin_amdgcn_readlane(sl, f);
-        back = (s0 == MS_M) && __builtin_amdgcn_readlane((int) spec, f) != 0;
-        if (++steps > max_steps) { status = 1; break; }
-      } else {
-        if (++steps > max_steps) { status = 1; break; }
-        switch (s0) {
-        case MS_N: s1 = MS_S; i = 0; break;                // N repeats down to row 0 without draws
-        case MS_B: {
-          rng = rng * 69069u + 1u;
-          const double roll = (double) rng / 4294967296.0, th = xthr[(size_t) i * 3 + 2];
-          s1 = (roll < th) ? MS_N : (th == th) ? MS_J : -1;
-          break;
+        if (++steps > max_steps || __builtin_amdgcn_readlane(sl, f) < 0) status = 1;
+        break;
+      }
+      if (status) break;
+      // E: one roll; the first running sum above it
+      if (++steps > max_steps || i < 1) { status = 1; break; }
+      int s = -1;
+      {
+        rng = rng * 69069u + 1u;
+        const double roll = (double) rng / 4294967296.0;
+        // the row's running sums are kept at every 64th element (ecum,
+        // md_ncp per row): the first checkpoint above the roll names the
+        // chunk, whose sums are formed again from the checkpoint before it
+        const int NCP = md_ncp(Q);
+        const double *cp = ecum + (size_t) i * NCP;
+        int c = -1;
+        for (int c0 = 0; c0 < NCP && c < 0; c0 += 64) {
+          const int cc = c0 + z;
+          const double v = cp[min(cc, NCP - 1)];
+          const unsigned long long m = __ballot(cc < NCP && roll < v);
+          if (m) c = c0 + (int) __ffsll((long long) m) - 1;
         }
-        case MS_E: {                                       // one roll; the first running sum above it
-          if (i < 1) break;
-          rng = rng * 69069u + 1u;
-          const double roll = (double) rng / 4294967296.0;
-          // the row's running sums are kept at every 64th element (ecum,
-          // md_ncp per row): the first checkpoint above the roll names the
-          // chunk, whose sums are formed again from the checkpoint before it
-          const int NCP = md_ncp(Q);
-          const double *cp = ecum + (size_t) i * NCP;
-          int c = -1;
-          for (int c0 = 0; c0 < NCP && c < 0; c0 += 64) {
-            const int cc = c0 + z;
-            const double v = cp[min(cc, NCP - 1)];
-            const unsigned long long m = __ballot(cc < NCP && roll < v);
-            if (m) c = c0 + (int) __ffsll((long long) m) - 1;
+        int found = -1;
+        const float nf = (float) (1.0 / (double) xmx[(size_t) i * 6 + 0]);
+        if (c >= 0) {
+          const int j = 64 * c + z, q = j >> 3;
+          const float u = (j < 8 * Q) ? __fmul_rn(mat[((size_t) i * Q + q) * 12 + (j & 7)], nf) : 0.0f;
+          double sum = c ? cp[c - 1] : 0.0;
+          for (int l = 0; l < 64; l++) {
+            sum = sum + (double) readlanef(u, l);
+            if (roll < sum) { found = 64 * c + l; break; }
           }
-          int found = -1;
-          const float nf = (float) (1.0 / (double) xmx[(size_t) i * 6 + 0]);
-          if (c >= 0) {
-            const int j = 64 * c + z, q = j >> 3;
-            const float u = (j < 8 * Q) ? __fmul_rn(mat[((size_t) i * Q + q) * 12 + (j & 7)], nf) : 0.0f;
-            double sum = c ? cp[c - 1] : 0.0;
-            for (int l = 0; l < 64; l++) {
-              sum = sum + (double) readlanef(u, l);
-              if (roll < sum) { found = 64 * c + l; break; }
-            }
-          }
-          if (found >= 0) {
-            k = (found & 3) * Q + (found >> 3) + 1;
-            s1 = ((found >> 2) & 1) ? MS_D : MS_M;
-          } else {
-            // the reference scans the row again, the sum going on from its total
-            double sum = cp[NCP - 1];
-            for (int pass = 1; pass < 4 && s1 < 0; pass++)
-              for (int q0 = 0; q0 < Q && s1 < 0; q0 += 8) {
-                const int q = q0 + (z >> 3), sm = (z >> 2) & 1, r = z & 3;
-                const float u = (q < Q) ? __fmul_rn(CELL(i, q, sm, r), nf) : 0.0f;
-                for (int l = 0; l < 64; l++) {
-                  sum = sum + (double) readlanef(u, l);
-                  if (roll < sum) { k = (l & 3) * Q + q0 + (l >> 3) + 1; s1 = ((l >> 2) & 1) ? MS_D : MS_M; break; }
-                }
+        }
+        if (found >= 0) {
+          k = (found & 3) * Q + (found >> 3) + 1;
+          s = ((found >> 2) & 1) ? MS_D : MS_M;
+        } else {
+          // the reference scans the row again, the sum going on from its total
+          double sum = cp[NCP - 1];
+          for (int pass = 1; pass < 4 && s < 0; pass++)
+            for (int q0 = 0; q0 < Q && s < 0; q0 += 8) {
+              const int q = q0 + (z >> 3), sm = (z >> 2) & 1, r = z & 3;
+              const float u = (q < Q) ? __fmul_rn(mat[(((size_t) i * Q + q) * 3 + sm) * 4 + r], nf) : 0.0f;
+              for (int l = 0; l < 64; l++) {
+                sum = sum + (double) readlanef(u, l);
+                if (roll < sum) { k = (l & 3) * Q + q0 + (l >> 3) + 1; s = ((l >> 2) & 1) ? MS_D : MS_M; break; }
               }
-          }
-          break;
-        }
+            }
         }
       }
-      if (s1 < 0) { status = 1; break; }
-      if (s0 == MS_M) { k--; i--; }
-      else if (s0 == MS_D) k--;
-      else if (s0 == MS_I) i--;
-      // the trace element s1 at (i, k), in backward order
-      if (s1 == MS_M || s1 == MS_I) {
-        if (k < 1 || k > M || i < 1) { status = 1; break; }
-        if (z == 0) atomicAdd(&cnt[cnt_at(k)], 1.0f);      // the node's M cell
+      if (s < 0 || k < 1 || k > M) { status = 1; break; }
+      if (nseg + nd < J.segcap) {
+        if (z == 0) { dlog[nseg + nd] = n; drow[nseg + nd] = i; segs[nseg + nd].idx = t; }
+      } else over = true;
+      put(k | (s == MS_D ? 0x8000 : 0));
+      // the domain's runs, to its B
+      while (s != MS_B) {
+        const uint32_t xl = jA * rng + jC;
+        const int li = (s == MS_D) ? i : i - z, lk = (s == MS_I) ? k : k - z;
+        int sl = -1;
+        // An M run's step to I or D is most often followed by one step back
+        // to M. Lane l also takes that step ahead, as if it stopped here:
+        // the I or D cell is lane l+1's, whose thresholds that lane loads
+        // anyway, and the draw the next one. spec: that step leads to M
+        // (and its M cell is inside the matrix).
+        bool spec = false;
+        if (s == MS_M) {
+          const bool in = (li >= 1 && lk >= 1);
+          uint2 ta = make_uint2(0u, 0u), tb = ta, tc = ta;
+          if (in) {
+            const uint2 *c = thr + ((size_t) li * (M + 1) + lk) * 3;
+            ta = c[0]; tb = c[1]; tc = c[2];
+          }
+          const uint32_t F = tc.y;
+          if (in)
+            sl = (xl < ta.x || (F & 1u)) ? MS_B : (xl < ta.y || (F & 2u)) ? MS_M : (xl < tb.x || (F & 4u)) ? MS_I
+                 : (F >> MD_NAN_M & 1u) ? -1 : MS_D;
+          // cell (li - 1, lk - 1): lane 63 has no next lane
+          const uint32_t n3 = (uint32_t) wave_shl1((int) tb.y, 0), n4 = (uint32_t) wave_shl1((int) tc.x, 0);
+          const uint32_t nF = (uint32_t) wave_shl1((int) F, 0);
+          const bool nin = wave_shl1((int) in, 0) != 0;
+          const uint32_t x2 = 69069u * xl + 1u;
+          // back to M at (li - 2, lk - 1) from I, (li - 1, lk - 2) from D
+          if (sl == MS_I) spec = nin && (x2 < n4 || (nF & 16u)) && li - 2 >= 1;
+          if (sl == MS_D) spec = nin && (x2 < n3 || (nF & 8u)) && lk - 2 >= 1;
+        } else if (li >= 1 && lk >= 1) {
+          const uint2 *c = thr + ((size_t) li * (M + 1) + lk) * 3;
+          const uint2 tb = c[1], tc = c[2];
+          const uint32_t tt = (s == MS_D) ? tb.y : tc.x;
+          const uint32_t F = tc.y, all = (s == MS_D) ? 8u : 16u, nan = 1u << ((s == MS_D) ? MD_NAN_D : MD_NAN_I);
+          sl = (xl < tt || (F & all)) ? MS_M : (F & nan) ? -1 : s;
+        }
+        const unsigned long long stop = __ballot(sl != s);
+        const int f = stop ? (int) __ffsll((long long) stop) - 1 : 64;
+        if (s != MS_D) i -= f;
+        if (s != MS_I) k -= f;
+        steps += f;
+        if (f == 64) {
+          rng = (uint32_t) __builtin_amdgcn_readlane((int) xl, 63);
+          if (steps > max_steps) { status = 1; break; }
+          put(64);
+          continue;
+        }
+        rng = (uint32_t) __builtin_amdgcn_readlane((int) xl, f);
+        const int s1 = __builtin_amdgcn_readlane(sl, f);
+        const bool back = (s == MS_M) && __builtin_amdgcn_readlane((int) spec, f) != 0;
+        if (++steps > max_steps || s1 < 0) { status = 1; break; }
+        if (s != MS_D) i--;
+        if (s != MS_I) k--;
+        if (s1 != MS_B && (k < 1 || k > M || i < 1)) { status = 1; break; }
+        put(f | (s1 << 7) | ((int) back << 10));
+        s = s1;
+        // the I or D state's step back to M, taken ahead in the M run's ballot:
+        // its draw, then the M element at (i - 1, k) from I, (i, k - 1) from D
+        if (back) {
+          rng = rng * 69069u + 1u;
+          if (s1 == MS_I) i--; else k--;
+          if (++steps > max_steps || k < 1 || k > M || i < 1) { status = 1; break; }
+          s = MS_M;
+        }
+      }
+      if (status) break;
+      if (nd >= MD_TSEG) { status = 5; break; }
+      nd++;
+      // B: N (which repeats down to row 0 without draws) or J
+      if (++steps > max_steps) { status = 1; break; }
+      rng = rng * 69069u + 1u;
+      const double roll = (double) rng / 4294967296.0, th = xthr[(size_t) i * 3 + 2];
+      if (roll < th) { if (++steps > max_steps) status = 1; break; }
+      if (! (th == th)) { status = 1; break; }
+      col = 1;
+    }
+    if (! status && over) status = 5;
+    if (! status) nseg += nd;
+  }
+  if ((n & 63) && z < (n & 63)) lg[(n & ~63) + z] = (uint16_t) lbuf;
+  if (z == 0) {
+    O->status = status; O->trace = t; O->nseg = nseg; O->rng = rng;
+    if (first) { O->nc = 0; O->rtrace = 0; O->rdom = 0; O->done = 0; }
+  }
+}
+
+// What the walked traces mean: one workgroup per region. Each sampled domain
+// (p7_trace_Index, p7_trace.c:1173-1206) is replayed from the log by one wave:
+// its ends in the sequence and the model, and the null2 odds of its own trace
+// segment (p7_Null2_ByTrace, impl_sse/null2.c:134-205: every emitting M or I
+// state counts at the M cell of its node). MD_CHUNK domains at a time; then
+// every residue adds, per trace in trace order, the odds of the domain that
+// holds it or 1 outside domains. After the last trace: n2sc = logf(sum /
+// nsamples), and the clustering.
+__global__ __launch_bounds__(64 * MD_REPLAY_WAVES) void
+k_md_replay(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__restrict__ jobs, MdOut *__restrict__ out,
+            float *__restrict__ pool, int nsamples)
+{
+  extern __shared__ float lds[];
+  const int tid = threadIdx.x, z = tid & 63, wv = tid >> 6, NT = blockDim.x, NW = NT >> 6;
+  const MdJob J = jobs[blockIdx.x];
+  MdOut *O = out + blockIdx.x;
+  const int M = p.M, Q = max(2, (M - 1) / 4 + 1), Lr = J.Lr;
+  const uint8_t *dsq = res + J.res_off;                    // residue i (1-based) at dsq[i-1]
+  float *area = pool + J.area;
+  float *xmx = area + (size_t) (Lr + 1) * 12 * Q;
+  float *acc = xmx + (size_t) 6 * (Lr + 1);                // residues 0..Lr
+  int   *hist = (int *) (acc + (Lr + 1));                  // max(Lr, M) + 2 endpoint counts
+  MdSeg *segs = (MdSeg *) (area + md_seg_at(M, Lr));       // the ensemble, J.segcap entries
+  const uint16_t *lg = (const uint16_t *) (area + md_log_at(M, Lr, J.segcap));
+  const int *dlog = (const int *) (area + md_clu_at(M, Lr, J.segcap)), *drow = dlog + J.segcap;
+  int status = O->status;
+  const int ntr = O->trace, nseg = O->nseg, dom0 = O->rdom;
+  if (O->done) return;
+  if (status) { if (tid == 0) { O->nc = 0; O->done = 1; } return; }
+  const bool last = (ntr >= nsamples);
+  float *n2v = lds;                                        // [MD_CHUNK][32]
+  int4  *drec = (int4 *) (lds + MD_CHUNK * 32);            // trace, sqfrom, sqto, last of its trace
+  float *cnt = lds + md_rec_floats() + wv * 4 * Q;         // [q][r] counts of this wave's domain
+  const bool em_lds = md_em_lds(M) && p.K <= 20;
+  float *em = lds + md_rec_floats() + NW * 4 * Q;          // [x][q][r] odds, when em_lds
+  if (em_lds)
+    for (int c = tid; c < p.K * 4 * Q; c += NT) {
+      const int x = c / (4 * Q), rem = c - x * 4 * Q;
+      em[c] = md_tv(p, x, min((rem & 3) * Q + (rem >> 2) + 1, M + 1));
+    }
+  auto cnt_at = [&](int k) {                               // the count cell of model position k
+    const int r = (k - 1 >= Q) + (k - 1 >= 2 * Q) + (k - 1 >= 3 * Q);
+    return (k - 1 - r * Q) * 4 + r; };
+  if (O->rtrace == 0) for (int pos = tid; pos <= Lr; pos += NT) acc[pos] = 0.0f;
+  for (int c = z; c < 4 * Q; c += 64) cnt[c] = 0.0f;
+  int hi0 = Lr, tr0 = -1;                                  // the domain before the chunk: its sqfrom and trace
+  __syncthreads();
+  for (int c0 = dom0; c0 < nseg; c0 += MD_CHUNK) {
+    const int nc = min(MD_CHUNK, nseg - c0);
+    for (int d = wv; d < nc; d += NW) {
+      const int e = c0 + d, t = uni(segs[e].idx);
+      int at = uni(dlog[e]), i = uni(drow[e]);
+      int w = (int) lg[at + z];                            // 64 entries ahead (the log has room past its end)
+      int o = 0;
+      auto next = [&]() {
+        if (o == 64) { at += 64; w = (int) lg[at + z]; o = 0; }
+        return __builtin_amdgcn_readlane(w, o++);
+      };
+      const int v0 = next();
+      int k = v0 & 0x7fff, s = (v0 & 0x8000) ? MS_D : MS_M;
+      int sqfrom = 0, sqto = 0, hmmfrom = 0, hmmto = 0, Ld = 0, kmin = 0x7fffffff, kmax = 0;
+      auto emit = [&](bool m) {                            // an M (m) or I element at (i, k)
+        if (z == 0) cnt[cnt_at(k)] += 1.0f;
         kmin = min(kmin, k); kmax = max(kmax, k);
         Ld++;
-        if (s1 == MS_M) {
-          if (sqto == 0) { sqto = i; hmmto = k; }
-          sqfrom = i; hmmfrom = k;
-        }
-      } else if (s1 == MS_D) {
-        if (k < 1 || k > M || i < 1) { status = 1; break; }
-      } else if (s1 == MS_E) {
-        sqfrom = sqto = hmmfrom = hmmto = 0; Ld = 0; kmin = 0x7fffffff; kmax = 0;
-      } else if (s1 == MS_B) {
-        // p7_Null2_ByTrace over the domain: four striped sums over q per
-        // canonical residue, their hsum; degenerate codes the mean
+        if (m) { if (sqto == 0) { sqto = i; hmmto = k; } sqfrom = i; hmmfrom = k; }
         md_sync();
-        const float nrm = (float) (1.0 / (double) (float) Ld);
-        // lane z sums x = (base + z) / 4 and, for base + 64 + z, x + 16 (the
-        // same lane r, so the same counts): two chains per lane, one pass
-        for (int base = 0; base < p.K * 4; base += 128) {
-          const int xr = base + z, x = xr >> 2, r = xr & 3, x2 = x + 16;
-          const bool h1 = x < p.K, h2 = x2 < p.K;
-          float sv = 0.0f, sv2 = 0.0f;
-          if (h1) {
-            // positions kmin..kmax in lane r: the other cells' counts are 0, and
-            // adding their products (+0) leaves the striped sum unchanged
-            const int q0 = max(0, kmin - 1 - r * Q), q1 = min(Q - 1, kmax - 1 - r * Q);
-            for (int qa = q0; qa <= q1; qa += 8) {
-              float e[8], e2[8], cq[8];
+      };
+      if (s == MS_M) emit(true);
+      while (s != MS_B) {
+        const int v = next(), f = v & 0x7f, s1 = (v >> 7) & 7;
+        if (f > 0) {                                       // the repeats: M and I states emit
+          if (s == MS_M) {
+            if (z < f) cnt[cnt_at(k - 1 - z)] += 1.0f;
+            kmin = min(kmin, k - f); kmax = max(kmax, k - 1);
+            Ld += f;
+            if (sqto == 0) { sqto = i - 1; hmmto = k - 1; }
+            sqfrom = i - f; hmmfrom = k - f;
+            i -= f; k -= f;
+          } else if (s == MS_I) {
+            if (z == 0) cnt[cnt_at(k)] += (float) f;
+            kmin = min(kmin, k); kmax = max(kmax, k);
+            Ld += f;
+            i -= f;
+          } else k -= f;
+          md_sync();
+        }
+        if (s1 == 0) continue;                             // the run goes on
+        if (s != MS_D) i--;
+        if (s != MS_I) k--;
+        if (s1 == MS_M) emit(true);
+        else if (s1 == MS_I) emit(false);
+        s = s1;
+        if (v & 0x400) {
+          if (s1 == MS_I) i--; else k--;
+          emit(true);
+          s = MS_M;
+        }
+      }
+      // four striped sums over q per canonical residue, their hsum; degenerate
+      // codes the mean. Lane z sums x = z / 4 and, x + 16 (the same lane r, so
+      // the same counts): two chains per lane, one pass
+      float *nv = n2v + d * 32;
+      const float nrm = (float) (1.0 / (double) (float) Ld);
+      for (int base = 0; base < p.K * 4; base += 128) {
+        const int xr = base + z, x = xr >> 2, r = xr & 3, x2 = x + 16;
+        const bool h1 = x < p.K, h2 = x2 < p.K;
+        float sv = 0.0f, sv2 = 0.0f;
+        if (h1) {
+          // positions kmin..kmax in lane r: the other cells' counts are 0, and
+          // adding their products (+0) leaves the striped sum unchanged
+          const int q0 = max(0, kmin - 1 - r * Q), q1 = min(Q - 1, kmax - 1 - r * Q);
+          for (int qa = q0; qa <= q1; qa += 8) {
+            float e1[8], e2[8], cq[8];
 #pragma unroll
-              for (int u = 0; u < 8; u++) cq[u] = cnt[min(qa + u, Q - 1) * 4 + r];
-              if (em_lds) {
-#pragma unroll
-                for (int u = 0; u < 8; u++) {
-                  e[u] = em[(x * Q + min(qa + u, Q - 1)) * 4 + r];
-                  e2[u] = h2 ? em[(x2 * Q + min(qa + u, Q - 1)) * 4 + r] : 0.0f;
-                }
-              } else {
-#pragma unroll
-                for (int u = 0; u < 8; u++) {
-                  e[u] = md_tv(p, x, min(r * Q + qa + u + 1, M + 1));
-                  e2[u] = h2 ? md_tv(p, x2, min(r * Q + qa + u + 1, M + 1)) : 0.0f;
-                }
-              }
-              // a zero count adds +0.0, which leaves the non-negative sums as
-              // they are: no branch per cell
+            for (int u = 0; u < 8; u++) cq[u] = cnt[min(qa + u, Q - 1) * 4 + r];
+            if (em_lds) {
 #pragma unroll
               for (int u = 0; u < 8; u++) {
-                const float w = __fmul_rn(qa + u <= q1 ? cq[u] : 0.0f, nrm);
-                sv = __fadd_rn(sv, __fmul_rn(w, e[u]));
-                sv2 = __fadd_rn(sv2, __fmul_rn(w, e2[u]));
+                e1[u] = em[(x * Q + min(qa + u, Q - 1)) * 4 + r];
+                e2[u] = h2 ? em[(x2 * Q + min(qa + u, Q - 1)) * 4 + r] : 0.0f;
+              }
+            } else {
+#pragma unroll
+              for (int u = 0; u < 8; u++) {
+                e1[u] = md_tv(p, x, min(r * Q + qa + u + 1, M + 1));
+                e2[u] = h2 ? md_tv(p, x2, min(r * Q + qa + u + 1, M + 1)) : 0.0f;
               }
             }
+            // a zero count adds +0.0, which leaves the non-negative sums as
+            // they are: no branch per cell
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+              const float wt = __fmul_rn(qa + u <= q1 ? cq[u] : 0.0f, nrm);
+              sv = __fadd_rn(sv, __fmul_rn(wt, e1[u]));
+              sv2 = __fadd_rn(sv2, __fmul_rn(wt, e2[u]));
+            }
           }
-          // lanes 4x..4x+3 hold x's lane sums
-          const float s01 = __fadd_rn(sv, __shfl_down(sv, 1, 4)), s23 = __shfl_down(s01, 2, 4);
-          if (h1 && r == 0) n2v[x] = __fadd_rn(__fadd_rn(s01, s23), 0.0f);
-          const float t01 = __fadd_rn(sv2, __shfl_down(sv2, 1, 4)), t23 = __shfl_down(t01, 2, 4);
-          if (h2 && r == 0) n2v[x2] = __fadd_rn(__fadd_rn(t01, t23), 0.0f);
         }
-        md_sync();
-        {                                                  // degenerate codes: one lane each
-          const int xx = p.K + 1 + z;
-          if (xx <= p.Kp - 3) {
-            const uint32_t dm = p.degen[xx];
-            float rr = 0.0f;
-            for (int y = 0; y < p.K; y++) if ((dm >> y) & 1u) rr = __fadd_rn(rr, n2v[y]);
-            n2v[xx] = __fdiv_rn(rr, (float) (dm >> 24));
-          }
-          if (z == 0) { n2v[p.K] = 1.0f; n2v[p.Kp - 2] = 1.0f; n2v[p.Kp - 1] = 1.0f; }
-        }
-        md_sync();
-        // residues (sqto, hi] are outside domains (1), (sqfrom, sqto] take the odds
-        for (int pos = z + 1 + ((sqfrom >> 6) << 6); pos <= hi; pos += 64) {
-          // the lane of a residue is fixed (pos mod 64), so its updates stay in order
-          if (pos > sqto)        accp[pos] = __fadd_rn(accp[pos], 1.0f);
-          else if (pos > sqfrom) accp[pos] = __fadd_rn(accp[pos], n2v[rsq[pos - 1]]);
-        }
-        hi = sqfrom;
-        if (nd >= MD_TSEG) { status = 5; break; }
-        if (z == 0) { tseg[nd*4 + 0] = sqfrom; tseg[nd*4 + 1] = sqto; tseg[nd*4 + 2] = hmmfrom; tseg[nd*4 + 3] = hmmto; }
-        nd++;
-        for (int c = z; c < 4 * Q; c += 64) cnt[c] = 0.0f;
-        kmin = 0x7fffffff; kmax = 0;
-        md_sync();
+        // lanes 4x..4x+3 hold x's lane sums
+        const float s01 = __fadd_rn(sv, __shfl_down(sv, 1, 4)), s23 = __shfl_down(s01, 2, 4);
+        if (h1 && r == 0) nv[x] = __fadd_rn(__fadd_rn(s01, s23), 0.0f);
+        const float t01 = __fadd_rn(sv2, __shfl_down(sv2, 1, 4)), t23 = __shfl_down(t01, 2, 4);
+        if (h2 && r == 0) nv[x2] = __fadd_rn(__fadd_rn(t01, t23), 0.0f);
       }
-      // the I or D state's step back to M, taken ahead in the M run's ballot:
-      // its draw, then the M element at (i - 1, k) from I, (i, k - 1) from D
-      if (back) {
-        rng = rng * 69069u + 1u;
-        if (++steps > max_steps) { status = 1; break; }
-        if (s1 == MS_I) i--; else k--;
-        if (k < 1 || k > M || i < 1) { status = 1; break; }
-        if (z == 0) atomicAdd(&cnt[cnt_at(k)], 1.0f);
-        kmin = min(kmin, k); kmax = max(kmax, k);
-        Ld++;
-        if (sqto == 0) { sqto = i; hmmto = k; }
-        sqfrom = i; hmmfrom = k;
-        s1 = MS_M;
+      md_sync();
+      {                                                    // degenerate codes: one lane each
+        const int xx = p.K + 1 + z;
+        if (xx <= p.Kp - 3) {
+          const uint32_t dm = p.degen[xx];
+          float rr = 0.0f;
+          for (int y = 0; y < p.K; y++) if ((dm >> y) & 1u) rr = __fadd_rn(rr, nv[y]);
+          nv[xx] = __fdiv_rn(rr, (float) (dm >> 24));
+        }
+        if (z == 0) { nv[p.K] = 1.0f; nv[p.Kp - 2] = 1.0f; nv[p.Kp - 1] = 1.0f; }
       }
-      // (N, C and J emit on the transition to themselves: the repeats above)
-      s0 = s1;
+      for (int c = z; c < 4 * Q; c += 64) cnt[c] = 0.0f;
+      md_sync();
+      // the trace's domains join the ensemble in sequence order: the walk met
+      // them last first
+      int b0 = e, b1 = e;
+      while (b0 > 0 && segs[b0 - 1].idx == t) b0--;
+      while (b1 + 1 < nseg && segs[b1 + 1].idx == t) b1++;
+      if (z == 0) {
+        MdSeg &sg = segs[b0 + b1 - e];
+        sg.i = sqfrom; sg.j = sqto; sg.k = hmmfrom; sg.m = hmmto;
+        drec[d] = make_int4(t, sqfrom, sqto, e == b1);
+      }
     }
-    if (status) break;
-    for (int pos = z + 1; pos <= hi; pos += 64) accp[pos] = __fadd_rn(accp[pos], 1.0f);
-    // the trace's domains join the ensemble in sequence order
-    if (nseg + nd > J.segcap) { status = 5; break; }
-    md_sync();
-    for (int d = z; d < nd; d += 64) {
-      const int e = nd - 1 - d;
-      segs[nseg + d] = MdSeg{ t, tseg[e*4 + 0], tseg[e*4 + 1], tseg[e*4 + 2], tseg[e*4 + 3] };
+    __syncthreads();
+    // residues (sqto, hi] are outside domains (1), (sqfrom, sqto] take the odds;
+    // hi is the sqfrom of the trace's domain before, or Lr
+    for (int pos = tid + 1; pos <= Lr; pos += NT) {
+      float a = acc[pos];
+      const int x = dsq[pos - 1];
+      int hi = hi0, tp = tr0;
+      for (int d = 0; d < nc; d++) {
+        const int4 r = drec[d];
+        if (r.x != tp) hi = Lr;
+        if (pos > r.y && pos <= hi) a = __fadd_rn(a, pos > r.z ? 1.0f : n2v[d * 32 + x]);
+        if (r.w && pos <= r.y) a = __fadd_rn(a, 1.0f);
+        hi = r.y; tp = r.x;
+      }
+      acc[pos] = a;
     }
-    nseg += nd;
-    md_sync();
+    hi0 = drec[nc - 1].y; tr0 = drec[nc - 1].x;
+    __syncthreads();
   }
-  if (status) { if (z == 0) { O->status = status; O->nc = 0; O->nseg = nseg; } return; }
-  for (int pos = z + 1; pos <= Lr; pos += 64) acc[pos] = logf(__fdiv_rn(accp[pos], (float) nsamples));
+  if (! last) { if (tid == 0) { O->rtrace = ntr; O->rdom = nseg; } return; }
+  for (int pos = tid + 1; pos <= Lr; pos += NT) acc[pos] = logf(__fdiv_rn(acc[pos], (float) nsamples));
+  if (tid == 0) { O->rtrace = ntr; O->rdom = nseg; O->done = 1; }
   __syncthreads();
+  if (wv != 0) return;                                     // the rest is one wave's work
 
   // ---------------- 3. clustering ----------------
   // the two stacks of the linkage in LDS; each element's cluster and each
   // cluster's trace count in the region's area
   int *av = (int *) lds, *bv = av + J.segcap;
-  int *asg = (int *) (pool + J.area + md_clu_at(M, Lr, J.segcap)), *ninc = asg + J.segcap;
+  int *asg = (int *) (area + md_clu_at(M, Lr, J.segcap)), *ninc = asg + J.segcap;
   unsigned long long *lk = (unsigned long long *) (bv + J.segcap);   // link bits of one pass
   MdSig *sig = (MdSig *) (lk + (J.segcap + 63) / 64);
   const int n = nseg;
@@ -798,17 +920,18 @@ k_md_region(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__
     O->nc = min(nc, MD_MAXC);
     O->nseg = nseg;
   }
-#undef CELL
 }
 
 // LDS of one region's workgroup: the Forward's two rows and D->D odds, the
-// traces' counts, odds and per-trace domains, or the clustering's stacks
-size_t md_lds_bytes(int M, int segcap, int acc_cap)
+// replay's odds and counts, or the clustering's stacks
+static size_t md_fwd_lds(int M)
+{ return (size_t) ((md_stage_t(M) ? md_stage_floats(M) : 0) + 32 * md_q(M) + 128) * 4; }
+static size_t md_replay_lds(int M, int segcap)
 {
-  const int64_t fwd = (md_stage_t(M) ? md_stage_floats(M) : 0) + 32 * md_q(M) + 128;
   const size_t clu = (size_t) 2 * segcap * 4 + (size_t) (segcap + 63) / 64 * 8 + (size_t) MD_MAXSIG * sizeof(MdSig);
-  return std::max((size_t) std::max(fwd, md_trace_floats(M, acc_cap)) * 4, clu);
+  return std::max((size_t) md_replay_floats(M) * 4, clu);
 }
+size_t md_lds_bytes(int M, int segcap) { return std::max(md_fwd_lds(M), md_replay_lds(M, segcap)); }
 
 // The traces' cell thresholds of every region (md_thresholds over each cell
 // of its finished Forward matrix): a grid of gridDim.x workgroups of
@@ -816,12 +939,13 @@ size_t md_lds_bytes(int M, int segcap, int acc_cap)
 // depends only on the finished matrix, so its thresholds are computed first,
 // with the same operations p7_StochasticTrace performs at the step
 // (md_thresholds); a step is then one draw and one to three comparisons.
-// thr[(i, k)]: M's three (B | M | I | D), D's one (M | D), I's one (M | I),
-// as doubles. A pass's five-double records go out through LDS, so that the
-// stores of a wave are contiguous. The rows' thresholds are k_md_rows'.
+// thr[(i, k)]: M's three (B | M | I | D), D's one (M | D), I's one (M | I), as
+// the integers a draw is compared with (md_thr_word), and their flags. A pass's
+// six-word records go out through LDS, so that the stores of a wave are
+// contiguous. The rows' thresholds are k_md_rows'.
 #define MD_THR_NT 256
 #define MD_THR_CELLS 2                                     // cells per thread per pass
-#define MD_THR_LDS_OUT ((size_t) 8 * (MD_THR_CELLS * MD_THR_NT * 5 > MD_THR_NT * 8 ? MD_THR_CELLS * MD_THR_NT * 5 : MD_THR_NT * 8))
+#define MD_THR_LDS_OUT ((size_t) 4 * MD_THR_CELLS * MD_THR_NT * MD_THR_WORDS)
 static __host__ __device__ inline size_t md_thr_tl_bytes(int M)      // the staged transitions, when they fit
 {
   const size_t b = ((size_t) 10 * (M + 2) * 4 + 7) & ~(size_t) 7;
@@ -841,7 +965,7 @@ k_md_thr(const DevProfile p, const MdJob *__restrict__ jobs, float *__restrict__
   const int TW = M + 2;
   const size_t tlb = md_thr_tl_bytes(M);
   float *tl = (float *) ldsd;
-  double *ob = ldsd + tlb / 8;                             // the outgoing values
+  uint32_t *ob = (uint32_t *) (ldsd + tlb / 8);            // the outgoing words
   if (tlb) {
     for (int c = t; c < 10 * TW; c += NT) tl[c] = md_tv(p, TR + md_trow(c / TW), c % TW);
     __syncthreads();
@@ -849,7 +973,7 @@ k_md_thr(const DevProfile p, const MdJob *__restrict__ jobs, float *__restrict__
   auto tv = [&](int row, int k) -> float { return tlb ? tl[row * TW + k] : md_tv(p, TR + md_trow(row), k); };
   enum { T_BM = 0, T_MM, T_IM, T_DM, T_MDS, T_DDS, T_MI, T_II, T_MD, T_DD };
 #define CELL(i_, q_, s_, r_) mat[(((size_t) (i_) * Q + (q_)) * 3 + (s_)) * 4 + (r_)]
-  double *thr = (double *) (pool + J.area + md_thr_at(M, Lr, J.segcap));
+  uint32_t *thr = (uint32_t *) (pool + J.area + md_thr_at(M, Lr, J.segcap));
   auto cellk = [&](int i, int k, int s) {                  // the cell of model position k (1..4Q) in row i
     const int r = (k - 1 >= Q) + (k - 1 >= 2 * Q) + (k - 1 >= 3 * Q), q = k - 1 - r * Q;
     return CELL(i, q, s, r); };
@@ -888,7 +1012,8 @@ k_md_thr(const DevProfile p, const MdJob *__restrict__ jobs, float *__restrict__
     for (int u = 0; u < CU; u++) {
       int i, k;
       rowcol(min(u * NT + t, olast), i, k);
-      double *o = ob + (size_t) (u * NT + t) * 5;
+      uint32_t *ow = ob + (size_t) (u * NT + t) * MD_THR_WORDS;
+      double o[5];
       float v[4];
       v[0] = __fmul_rn(in[u][0], tv(T_BM, k));
       v[1] = __fmul_rn(in[u][1], tv(T_MM, k));
@@ -901,16 +1026,20 @@ k_md_thr(const DevProfile p, const MdJob *__restrict__ jobs, float *__restrict__
       v[0] = __fmul_rn(in[u][6], tv(T_MI, k));
       v[1] = __fmul_rn(in[u][7], tv(T_II, k));
       md_thresholds(v, 2, o + 4);
+      uint32_t fl = 0u;
+#pragma unroll
+      for (int a = 0; a < 5; a++) ow[a] = md_thr_word(o[a], a, fl);
+      ow[5] = fl | (isnan(o[0]) ? 1u << MD_NAN_M : 0u) | (isnan(o[3]) ? 1u << MD_NAN_D : 0u) | (isnan(o[4]) ? 1u << MD_NAN_I : 0u);
     }
     __syncthreads();
     // the pass's cells are consecutive in row-major order, each row's cells at
-    // (i (M + 1) + k) 5: the stores run along them
-    for (int d = t; d < CU * NT * 5; d += NT) {
-      const int o = d / 5;
+    // (i (M + 1) + k) MD_THR_WORDS: the stores run along them
+    for (int d = t; d < CU * NT * MD_THR_WORDS; d += NT) {
+      const int o = d / MD_THR_WORDS;
       if (o <= olast) {
         int i, k;
         rowcol(o, i, k);
-        thr[((size_t) i * (M + 1) + k) * 5 + (d - o * 5)] = ob[d];
+        thr[((size_t) i * (M + 1) + k) * MD_THR_WORDS + (d - o * MD_THR_WORDS)] = ob[d];
       }
     }
     __syncthreads();
@@ -935,9 +1064,8 @@ k_md_rows(const DevProfile p, const MdJob *__restrict__ jobs, float *__restrict_
   const float xEmove = p.xfE_move, xEloop = p.xfE_loop, floop = p.xf_loop[L], fmove = p.xf_move[L];
   const float *mat = pool + J.area;
   const float *xmx = mat + (size_t) (Lr + 1) * 12 * Q;
-  double *thr = (double *) (pool + J.area + md_thr_at(M, Lr, J.segcap));
-  double *xthr = thr + (size_t) 5 * (Lr + 1) * (M + 1);
-  double *ecum = xthr + (size_t) 3 * (Lr + 1);
+  double *xthr = (double *) (pool + J.area + md_xthr_at(M, Lr, J.segcap));
+  double *ecum = (double *) (pool + J.area + md_ecum_at(M, Lr, J.segcap));
   __shared__ float4 tile[64 * 17];                         // [row][q][M, D halves], 17 float4 a row
   const int i = r0 + t;
   const bool row = (i >= 1 && i <= Lr);
@@ -986,11 +1114,11 @@ k_md_rows(const DevProfile p, const MdJob *__restrict__ jobs, float *__restrict_
 }
 
 // floats of one region's area in the pool: matrix, specials, residue sums,
-// endpoint counts, the ensemble, then the traces' thresholds (doubles)
+// endpoint counts, the ensemble, the traces' thresholds, the walk's log (and 64
+// entries past it, which the replay may read)
 int64_t md_area_floats(int M, int Lr, int segcap)
 {
-  const int64_t Q = md_q(M), R = (int64_t) Lr + 1;
-  const int64_t f = md_thr_at(M, Lr, segcap) + 2 * (5 * R * ((int64_t) M + 1) + 3 * R + md_ncp(Q) * R);
+  const int64_t f = md_log_at(M, Lr, segcap) + (md_log_entries(M, Lr) + 1) / 2 + 32;
   return (f + 63) & ~(int64_t) 63;
 }
 
@@ -999,16 +1127,15 @@ hipError_t launch_md_regions(const DevProfile &p, const uint8_t *res, const MdJo
                              hipEvent_t thr_done)
 {
   if (njobs <= 0) return hipSuccess;
-  const int acc_cap = md_acc_cap(max_lr);
-  const size_t lds = md_lds_bytes(p.M, segcap, acc_cap);
-  if (lds > P7G_LDS_MAX) return hipErrorInvalidValue;
-  hipError_t e = hipFuncSetAttribute((const void *) k_md_region, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
+  const size_t lds0 = md_fwd_lds(p.M), lds = md_replay_lds(p.M, segcap);
+  if (std::max(lds0, lds) > P7G_LDS_MAX) return hipErrorInvalidValue;
+  hipError_t e = hipFuncSetAttribute((const void *) k_md_fwd, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds0);
+  if (e == hipSuccess) e = hipFuncSetAttribute((const void *) k_md_replay, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
   if (e != hipSuccess) return e;
   // the Forward matrices (one wave per region, the Forward's LDS only), the
-  // thresholds (the whole device), then the traces and the clustering
+  // thresholds (the whole device), then the traces' walks and replays
   // (128 floats past the rows: the D->D chains read up to seven cells past q = Q - 1)
-  const size_t lds0 = (size_t) ((md_stage_t(p.M) ? md_stage_floats(p.M) : 0) + 32 * md_q(p.M) + 128) * 4;
-  hipLaunchKernelGGL(k_md_region, dim3(njobs), dim3(64), lds0, st, p, res, jobs, out, pool, nsamples, seed, 0, acc_cap);
+  hipLaunchKernelGGL(k_md_fwd, dim3(njobs), dim3(64), lds0, st, p, res, jobs, pool);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   for (int j0 = 0; j0 < njobs; j0 += 65535) {
     const int nj = std::min(njobs - j0, 65535);
@@ -1018,8 +1145,16 @@ hipError_t launch_md_regions(const DevProfile &p, const uint8_t *res, const MdJo
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   if (thr_done && (e = hipEventRecord(thr_done, st)) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_md_region, dim3(njobs), dim3(64), lds, st, p, res, jobs, out, pool, nsamples, seed, 1, acc_cap);
-  return hipGetLastError();
+  // as many launches as a region needs whose every trace fills its share of
+  // the log: one for M above some 150, and mostly the first does everything
+  const int passes = std::max(md_passes(p.M, max_lr, nsamples), md_passes(p.M, 1, nsamples));
+  for (int a = 0; a < passes; a++) {
+    hipLaunchKernelGGL(k_md_walk, dim3(njobs), dim3(64), 0, st, p, jobs, out, pool, nsamples, seed, (int) (a == 0));
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_md_replay, dim3(njobs), dim3(64 * md_replay_waves(p.M)), lds, st, p, res, jobs, out, pool, nsamples);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 // Residue copies of the envelopes the clusters define, from their regions'

@@ -1491,7 +1491,7 @@ md_start(Work &w, const DevProfile &p, const std::vector<int4> &rec, const std::
   for (int64_t k = 0; k < nregs; k++) if (rec[(size_t) k].w == 1 && vlen[(size_t) k] > 0) m.mdk.push_back(k);
   if (m.mdk.empty()) return p7G_OK;
   for (int64_t k : m.mdk) m.max_lr = std::max(m.max_lr, (int) vlen[(size_t) k]);
-  if (md_lds_bytes(p.M, MD_SEGCAP, md_acc_cap(m.max_lr)) > P7G_LDS_MAX) { p7g_set_error("model too long for multidomain regions (M=%d)", p.M); return p7G_EINVAL; }
+  if (md_lds_bytes(p.M, MD_SEGCAP) > P7G_LDS_MAX) { p7g_set_error("model too long for multidomain regions (M=%d)", p.M); return p7G_EINVAL; }
   m.voff.resize((size_t) nregs); m.eloop.resize((size_t) nregs); m.emove.resize((size_t) nregs);
   HIPCHK(hipMemcpyAsync(m.voff.data(), w.dout.v_off, 8 * (size_t) nregs, hipMemcpyDeviceToHost, w.st));
   HIPCHK(hipMemcpyAsync(m.eloop.data(), w.dout.env_loop, 4 * (size_t) nregs, hipMemcpyDeviceToHost, w.st));
@@ -3403,7 +3403,7 @@ p7_gpu_RegionTraceEnsemble(const uint8_t *dsq, int Lr, int Ltarget, const P7_GPU
   if ((status = check_dsq(dsq, Lr, om)) != p7G_OK) return status;
   if (segcap <= 0) segcap = MD_SEGCAP;
   if ((status = dev_profile(om, Ltarget, &p)) != p7G_OK) return status;
-  if (md_lds_bytes(p->M, segcap, md_acc_cap(Lr)) > P7G_LDS_MAX) { p7g_set_error("model too long for multidomain regions (M=%d)", p->M); return p7G_EINVAL; }
+  if (md_lds_bytes(p->M, segcap) > P7G_LDS_MAX) { p7g_set_error("model too long for multidomain regions (M=%d)", p->M); return p7G_EINVAL; }
   const int64_t Q = std::max(2, (p->M - 1) / 4 + 1);
   const int64_t area = md_area_floats(p->M, Lr, segcap);
   const size_t resb = ((size_t) Lr + 31) & ~(size_t) 15;
