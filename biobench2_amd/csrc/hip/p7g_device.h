@@ -65,6 +65,7 @@ struct DevProfile {
   // scalars
   int   tbm, tec, base, bias;
   float scale_b;
+  int   vf_free;         // every Viterbi row may close its D->D paths, and xB never falls (see k_vit)
   int   base_w, ddbound_w, xwE_move, xwE_loop, xwN_loop, xwC_loop, xwJ_loop;
   float scale_w;
   float xfE_move, xfE_loop;

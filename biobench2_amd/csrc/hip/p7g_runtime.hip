@@ -357,6 +357,18 @@ dev_profile_build(P7_GPU_OPROFILE *om, int Lmax_need, struct p7g_dev_profile_s *
   // ---- scalars ----
   p.tbm = om->tbm_b; p.tec = om->tec_b; p.base = om->base_b; p.bias = om->bias_b; p.scale_b = om->scale_b;
   p.base_w = om->base_w; p.ddbound_w = om->ddbound_w; p.scale_w = om->scale_w;
+  // Whether a Viterbi row may close its D->D paths without the lazy-F test:
+  // ddbound_w is at least every D(k-1) -> D(k) -> M(k+1) less B -> M(k+1)
+  // (D(1) is never reached), so that on rows that fail the test no such path
+  // wins an M; and every D->D score and the specials' loops are at most 0, the
+  // base not negative, so that xB does not fall.
+  p.vf_free = (om->xw[p7G_XN][p7G_LOOP] == 0 && om->xw[p7G_XC][p7G_LOOP] == 0 && om->xw[p7G_XJ][p7G_LOOP] == 0
+               && om->xw[p7G_XE][p7G_LOOP] <= 0 && om->xw[p7G_XE][p7G_MOVE] <= 0 && om->base_w >= 0);
+  for (int k = 2; k <= M; k++) {
+    const int dd = om->twv[(size_t) p7G_DD * M + k - 2];
+    if (dd > 0) p.vf_free = 0;
+    if (k > 2 && k < M && dd + om->twv[(size_t) p7G_DM * M + k] - om->twv[(size_t) p7G_BM * M + k] > om->ddbound_w) p.vf_free = 0;
+  }
   p.xwE_move = om->xw[p7G_XE][p7G_MOVE]; p.xwE_loop = om->xw[p7G_XE][p7G_LOOP];
   p.xwN_loop = om->xw[p7G_XN][p7G_LOOP]; p.xwC_loop = om->xw[p7G_XC][p7G_LOOP]; p.xwJ_loop = om->xw[p7G_XJ][p7G_LOOP];
   p.xfE_move = om->xf[p7G_XE][p7G_MOVE]; p.xfE_loop = om->xf[p7G_XE][p7G_LOOP];

@@ -54,3 +54,33 @@ def test_parser_rows_at_block_edges(gpu, tmp_path, M):
         for got, ref in ((fwd.xmx()[0], xmx), (bck.xmx()[0], bxmx)):
             np.testing.assert_allclose(got[:, 5], ref[:, 5], rtol=1e-5)
             np.testing.assert_allclose(got[:, :5], ref[:, :5], rtol=2e-4, atol=1e-30)
+
+
+@pytest.mark.parametrize("M", [1, 2, 127, 128, 129, 257, 640, 1023, 1281, 1535, 1536, 2046, 2047, 2559, 3071, 4095])
+@pytest.mark.parametrize("tables", ["converted", "lazy", "loops"])
+def test_viterbi_rows_bit_exact(gpu, tmp_path, M, tables):
+    """Every instance at its largest model and just past it (ND dwords per lane hold
+    128 ND - 1 positions), as converted (each row's D->D paths closed), and with a ddbound
+    that is no bound or loops that are not 0, which need the lazy test on every row."""
+    rng = np.random.default_rng([8, M])
+    h = synth.random_profile(M, rng, f"vit_M{M}")
+    h.stats = (-9.0, 0.6931, -9.5, 0.6931, -5.0, 0.6931)
+    path = str(tmp_path / "vit.hmm")
+    synth.write_hmm(path, [h])
+    om = gpu.OProfile.from_file(path)
+    core = synth.emit_homologs(synth.read_hmm_probs(path), 1, rng, indel_rich=True)[0]
+    seqs = random_seqs(rng, LENGTHS) + [core[:L] for L in (64, 129, 400)]
+    t = om.tables()
+    if tables == "lazy":
+        t["ddbound_w"] = t["ddbound_w"] - 4000
+    if tables == "loops":
+        t["xw"][1, 1] = t["xw"][2, 1] = t["xw"][3, 1] = -3
+    if tables != "converted":
+        om.load(t)
+    lm = oracle.LengthModel(t, max(len(s) for s in seqs) + 1)
+    sc, st = gpu.viterbi_batch(om, gpu.SeqDB.from_list(seqs))
+    for i, s in enumerate(seqs):
+        xw = t["xw"].copy()
+        xw[1, 0] = xw[2, 0] = xw[3, 0] = lm.xwmove[len(s)]
+        st0, sc0, _ = oracle.vit_filter(s, t, xw)
+        assert st0 == st[i] and (sc0 == sc[i] or (np.isinf(sc0) and np.isinf(sc[i]) and sc0 * sc[i] > 0)), (i, len(s), sc0, sc[i])
