@@ -26,7 +26,7 @@
 // when it holds the D->D closure is a max-plus prefix scan across the wave.
 // Forward/Backward parsers (fwdback.c:258-735): fp32, the D->D chain as an
 // affine prefix scan across the wave, sparse rescaling when xE > 1e4.
-#include "p7g_devfn.h"
+#include "p7g_list.h"
 
 /*****************************************************************
  * 2. MSV stage: per-target decision after the ungapped pass
@@ -58,7 +58,11 @@ __global__ void k_msv_classify(const DevProfile p, const int32_t *__restrict__ l
  * 3. MSV stage, full recurrence (one target per wave, 64 lanes)
  *****************************************************************/
 // LDS: the score table is staged in LDS; otherwise (models whose table does
-// not fit, ND >= 24) the rows are read from global memory.
+// not fit, ND >= 24) the rows are read from global memory. Bound by the row's
+// chain of a long target alone: residues come 64 rows at a time and the scores a
+// row ahead. Lists of 60,013 targets, M = 86: 95 us; 5,003 targets with longer
+// ones, M = 50: 88 us (217 and 205 us with both fetched in the row, the floor at
+// 0 as an instruction and a wave maximum every row).
 template <int ND, bool LDS>
 __global__ __launch_bounds__(512)
 void k_msv_full(const DevProfile p, const int *__restrict__ tbl, int tbl_dwords,
@@ -80,36 +84,44 @@ void k_msv_full(const DevProfile p, const int *__restrict__ tbl, int tbl_dwords,
     const int tjbm = ((lc.on ? lc.tjb : (int) p.tjb[L]) + p.tbm) & 0xff;
     int xJ = 0;
     int xB = max(p.base - tjbm, 0);
-    int mp[ND];
+    // Values are held as M - 32768 in int16, so that the floor at 0 is the
+    // saturation of the add. xJ (and so xB) only changes, and the overflow test
+    // only fires, when the row's xE exceeds min(xJ + tec, 254 - bias): a ballot
+    // on the lanes' packed maxima decides whether the wave maximum is needed.
+    int mp[ND], e[ND];
 #pragma unroll
-    for (int d = 0; d < ND; d++) mp[d] = 0;
+    for (int d = 0; d < ND; d++) mp[d] = (int) NEG_PAIR;
     bool overflow = false;
-    ResAsc rd;
-    if (L > 0) rd.init(sq);
-    for (int i = 0; i < L; i++) {
-      const int x = rd.at(i);
-      const int *row = rows + x * (ND * 64) + z;
-      const int s0 = shift_in<64>(mp[ND-1], 0);
-      const int xB2 = pair16(xB);
-      int E = 0;
+    int xB2 = pair16(xB - 32768), th2 = pair16(min(xJ + p.tec, 254 - p.bias) - 32768);
+    if (L > 0) {
+      RowRes<false> rr;
+      const int x0 = rr.init(sq, L, z, ND * 64);
 #pragma unroll
-      for (int d = ND-1; d >= 0; d--) {
-        int src = (d > 0) ? mp[d-1] : s0;
-        int tv = max2(src, xB2);
-        tv = adds2(tv, row[d * 64]);
-        tv = max2(tv, 0);
-        E  = max2(E, tv);
-        mp[d] = tv;
-      }
-      // xJ (and so xB) only changes, and the overflow test only fires, when
-      // the row's xE exceeds min(xJ + tec, 254 - bias): a ballot on the lanes'
-      // maxima decides whether the wave maximum is needed at all
-      const int el = max(lo16(E), hi16(E));
-      if (__ballot(el > min(xJ + p.tec, 254 - p.bias)) != 0ull) {
-        const int xE = uni(wave_max_i(el));
-        if (xE + p.bias >= 255) { overflow = true; break; }
-        xJ = max(xJ, max(xE - p.tec, 0));
-        xB = max(max(p.base, xJ) - tjbm, 0);
+      for (int d = 0; d < ND; d++) e[d] = rows[x0 + z + d * 64];
+      for (int i0 = 0; i0 < L && ! overflow; i0 += 64) {
+        const int cnt = min(64, L - i0);
+        for (int u = 0; u < cnt; u++) {
+          const int *en = rows + rr.ahead(u) + z;
+          const int s0 = shift_in<64>(mp[ND-1], (int) NEG_PAIR);
+          int E = (int) NEG_PAIR;
+#pragma unroll
+          for (int d = ND-1; d >= 0; d--) {
+            const int tv = adds2(max2(d > 0 ? mp[d-1] : s0, xB2), e[d]);
+            E = max2(E, tv);
+            mp[d] = tv;
+          }
+          // the next row's scores, a row ahead
+#pragma unroll
+          for (int d = 0; d < ND; d++) e[d] = en[d * 64];
+          if (__builtin_expect(__ballot(max2(E, th2) != th2) != 0ull, 0)) {
+            const int xE = uni(wave_max_i(max(lo16(E), hi16(E)))) + 32768;
+            if (xE + p.bias >= 255) { overflow = true; break; }
+            xJ = max(xJ, max(xE - p.tec, 0));
+            xB = max(max(p.base, xJ) - tjbm, 0);
+            xB2 = pair16(xB - 32768); th2 = pair16(min(xJ + p.tec, 254 - p.bias) - 32768);
+          }
+        }
+        rr.advance();
       }
     }
     if (z == 0) xj[slot] = (int16_t) (overflow ? -1 : xJ);
@@ -120,10 +132,12 @@ void k_msv_full(const DevProfile p, const int *__restrict__ tbl, int tbl_dwords,
 // dwords [w·ND/W, (w+1)·ND/W) of every lane. A slice's first dword takes the
 // previous row's last dword of the slice before it (slice 0: of the last
 // slice, joined across lanes as shift_in does) from LDS, double-buffered by
-// row parity, so one barrier per row orders the exchange. The waves' row
+// row parity, so one barrier per row orders the exchange. The lanes' row
 // maxima travel in the same buffers, and xJ and xB are updated from them at
 // the top of the next row (or after the last), in the same order as the
-// one-wave kernel; results are bit-identical.
+// one-wave kernel; results are bit-identical. Bound by the row's exchange;
+// M = 2600, a target of 35,000 residues: 3.1 ms, 5.4 ms with the maxima reduced
+// in every wave and residues and scores fetched in the row.
 template <int ND, int W>
 __global__ __launch_bounds__(64 * W)
 void k_msv_full_wg(const DevProfile p, const int *__restrict__ tbl, const uint8_t *__restrict__ res,
@@ -132,74 +146,81 @@ void k_msv_full_wg(const DevProfile p, const int *__restrict__ tbl, const uint8_
 {
   static_assert(ND % W == 0, "slices of equal width");
   constexpr int NW = ND / W;
-  __shared__ int sh_end[2][W][64];       // each slice's last dword, by row parity
-  __shared__ int sh_el[2][W];            // each wave's row maximum, by row parity
+  __shared__ int sh_end[2][W][65];       // each slice's last dword, by row parity; lane z at z + 1 (0: none)
+  __shared__ int sh_el[2][W][64];        // each wave's row maxima per lane, by row parity
   __shared__ int64_t sh_t;
   if ((int64_t) blockIdx.x >= *count) return;
-  const int wv = threadIdx.x >> 6, z = threadIdx.x & 63;
+  const int wv = uni(threadIdx.x >> 6), z = threadIdx.x & 63;
   const int d0 = wv * NW;
   const int64_t n = *count;
   int32_t *queue = (int32_t *) count + P7G_QOFF;
+  if (z == 0) sh_end[0][wv][0] = sh_end[1][wv][0] = (int) NEG_PAIR;
 
   for (;;) {
     if (threadIdx.x == 0) sh_t = (int64_t) atomicAdd(queue, 1);
     __syncthreads();
     const int64_t t = sh_t;
     if (t >= n) break;
-    const int slot = list[t];
-    const int L = len[slot];
+    const int slot = uni(list[t]);
+    const int L = uni(len[slot]);
     const uint8_t *sq = res + off[slot];
     const int tjbm = ((lc.on ? lc.tjb : (int) p.tjb[L]) + p.tbm) & 0xff;
     int xJ = 0;
     int xB = max(p.base - tjbm, 0);
-    int mp[NW];
+    // values as M - 32768, and the threshold of a change of xJ, as in k_msv_full
+    int mp[NW], e[NW];
 #pragma unroll
-    for (int j = 0; j < NW; j++) mp[j] = 0;
-    sh_end[1][wv][z] = 0;                              // row -1
+    for (int j = 0; j < NW; j++) mp[j] = (int) NEG_PAIR;
+    sh_end[1][wv][z + 1] = (int) NEG_PAIR;             // row -1
     bool overflow = false;
-    // the update of xJ and xB from the row maximum the waves left in buffer b
+    int xB2 = pair16(xB - 32768), th2 = pair16(min(xJ + p.tec, 254 - p.bias) - 32768);
+    // the update of xJ and xB when a row's maximum, left per lane in buffer b,
+    // exceeds the threshold
     auto update = [&](int b) {
-      int xE = sh_el[b][0];
+      int E = sh_el[b][0][z];
 #pragma unroll
-      for (int v = 1; v < W; v++) xE = max(xE, sh_el[b][v]);
-      if (xE > min(xJ + p.tec, 254 - p.bias)) {
-        if (xE + p.bias >= 255) { overflow = true; return; }
-        xJ = max(xJ, max(xE - p.tec, 0));
-        xB = max(max(p.base, xJ) - tjbm, 0);
-      }
+      for (int v = 1; v < W; v++) E = max2(E, sh_el[b][v][z]);
+      if (__builtin_expect(__ballot(max2(E, th2) != th2) == 0ull, 1)) return;
+      const int xE = uni(wave_max_i(max(lo16(E), hi16(E)))) + 32768;
+      if (xE + p.bias >= 255) { overflow = true; return; }
+      xJ = max(xJ, max(xE - p.tec, 0));
+      xB = max(max(p.base, xJ) - tjbm, 0);
+      xB2 = pair16(xB - 32768); th2 = pair16(min(xJ + p.tec, 254 - p.bias) - 32768);
     };
-    ResAsc rd;
-    if (L > 0) rd.init(sq);
-    for (int i = 0; i < L; i++) {
-      const int x = rd.at(i);
-      const int *row = tbl + (size_t) x * (ND * 64) + z;
-      const int pb = (i + 1) & 1;                      // the previous row's buffer
-      __syncthreads();                                 // the previous row's slice ends and maxima are written
-      if (i > 0) { update(pb); if (overflow) break; }
-      int s0;
-      if (wv > 0) s0 = sh_end[pb][wv-1][z];
-      else {
-        const int nb = (z > 0) ? sh_end[pb][W-1][z-1] : 0;
-        s0 = (int) __builtin_amdgcn_alignbit((unsigned) sh_end[pb][W-1][z], (unsigned) nb, 16);
-      }
-      const int xB2 = pair16(xB);
-      int E = 0;
+    if (L > 0) {
+      RowRes<false> rr;
+      const int x0 = rr.init(sq, L, z, ND * 64);
+      const int *tz = tbl + (size_t) d0 * 64 + z;
 #pragma unroll
-      for (int j = NW-1; j >= 0; j--) {
-        int src = j ? mp[j-1] : s0;
-        int tv = max2(src, xB2);
-        tv = adds2(tv, row[(size_t) (d0 + j) * 64]);
-        tv = max2(tv, 0);
-        E  = max2(E, tv);
-        mp[j] = tv;
+      for (int j = 0; j < NW; j++) e[j] = tz[x0 + j * 64];
+      for (int i0 = 0; i0 < L && ! overflow; i0 += 64) {
+        const int cnt = min(64, L - i0);
+        for (int u = 0; u < cnt; u++) {
+          const int q = u & 1;                         // 64 is even: the buffers alternate
+          lds_barrier();                               // the previous row's slice ends and maxima are written
+          int s0;
+          if (wv > 0) s0 = sh_end[q ^ 1][wv-1][z + 1];
+          else s0 = (int) __builtin_amdgcn_alignbit((unsigned) sh_end[q ^ 1][W-1][z + 1], (unsigned) sh_end[q ^ 1][W-1][z], 16);
+          if (i0 + u > 0) { update(q ^ 1); if (overflow) break; }
+          int E = (int) NEG_PAIR;
+#pragma unroll
+          for (int j = NW-1; j >= 0; j--) {
+            const int tv = adds2(max2(j ? mp[j-1] : s0, xB2), e[j]);
+            E = max2(E, tv);
+            mp[j] = tv;
+          }
+          const int *en = tz + rr.ahead(u);            // the next row's scores, a row ahead
+#pragma unroll
+          for (int j = 0; j < NW; j++) e[j] = en[j * 64];
+          sh_end[q][wv][z + 1] = mp[NW-1];
+          sh_el[q][wv][z] = E;
+        }
+        rr.advance();
       }
-      sh_end[i & 1][wv][z] = mp[NW-1];
-      const int el = wave_max_i(max(lo16(E), hi16(E)));
-      if (z == 0) sh_el[i & 1][wv] = el;
-    }
-    if (L > 0 && ! overflow) {
-      __syncthreads();
-      update((L - 1) & 1);
+      if (! overflow) {
+        lds_barrier();
+        update((L - 1) & 1);
+      }
     }
     if (threadIdx.x == 0) xj[slot] = (int16_t) (overflow ? -1 : xJ);
     __syncthreads();                                   // sh_t and the buffers are free for the next target

@@ -84,3 +84,30 @@ def test_viterbi_rows_bit_exact(gpu, tmp_path, M, tables):
         xw[1, 0] = xw[2, 0] = xw[3, 0] = lm.xwmove[len(s)]
         st0, sc0, _ = oracle.vit_filter(s, t, xw)
         assert st0 == st[i] and (sc0 == sc[i] or (np.isinf(sc0) and np.isinf(sc[i]) and sc0 * sc[i] > 0)), (i, len(s), sc0, sc[i])
+
+
+@pytest.mark.parametrize("M", [1, 127, 128, 129, 640, 1023, 1281, 2047, 2559, 3071, 4095])
+def test_msv_rows_bit_exact(gpu, tmp_path, M):
+    """The full MSV recurrence (targets whose J state matters) at block and instance edges:
+    segments of the model side by side, up to overflow."""
+    rng = np.random.default_rng([9, M])
+    h = synth.random_profile(M, rng, f"msv_M{M}")
+    h.stats = (-9.0, 0.6931, -9.5, 0.6931, -5.0, 0.6931)
+    path = str(tmp_path / "msv.hmm")
+    synth.write_hmm(path, [h])
+    om = gpu.OProfile.from_file(path)
+    core = synth.emit_homologs(synth.read_hmm_probs(path), 1, rng)[0]
+    piece = core[:min(len(core), 18)]
+    seqs = random_seqs(rng, LENGTHS)
+    for n in (1, 2, 3, 5, 8):
+        for L in (63, 64, 65, 129, 300):
+            s = random_seqs(rng, [L])[0]
+            for at in range(0, min(n * 37, L - len(piece)), 37):
+                s[at:at + len(piece)] = piece
+            seqs.append(s)
+    t = om.tables()
+    lm = oracle.LengthModel(t, max(len(s) for s in seqs) + 1)
+    sc, st = gpu.msv_batch(om, gpu.SeqDB.from_list(seqs))
+    for i, s in enumerate(seqs):
+        st0, sc0, _ = oracle.msv_filter(s, t, tjb=int(lm.tjb[len(s)]))
+        assert st0 == st[i] and (sc0 == sc[i] or (np.isinf(sc0) and np.isinf(sc[i]))), (i, len(s), sc0, sc[i])
