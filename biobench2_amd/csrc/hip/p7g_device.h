@@ -70,6 +70,7 @@ struct DevProfile {
   float scale_w;
   float xfE_move, xfE_loop;
   float nj;
+  int   bias_ok;         // the filter HMM's numbers are all in range of k_bias's division
   float ft1_0, ft1_1;     // filter HMM state-1 transitions
   float pi0, pi1;
   void *blob;             // single device allocation holding everything above

@@ -288,7 +288,7 @@ __global__ void k_msv_gate(const DevProfile p, const int32_t *__restrict__ len, 
  * 5. Bias-composition filter: 2-state HMM Forward with per-row max
  *    normalisation (easel/esl_hmm.c:351-409, HMMER/src/p7_bg.c:473-484).
  *    Float arithmetic in the reference's order, in two passes:
- *    k_bias runs the recurrence, one target per thread, and stores each
+ *    k_bias runs the recurrence, one target per pair of lanes, and stores each
  *    row's normaliser; k_bias_sum takes the logs of a target's normalisers
  *    on all lanes at once and adds them in row order, as the reference does.
  *    The log is off the recurrence's serial chain, which bounds the stage.
@@ -308,6 +308,25 @@ __device__ __forceinline__ void bias_finish(const DevProfile &p, DevResults &r, 
   }
 }
 
+// n / m, correctly rounded, for n <= m in the range that bias_ok and the length
+// model's test set up: no intermediate is subnormal, so that the residuals are
+// exact and no operand needs scaling. The quotient is corrected twice by its
+// exact residual (P. Markstein, Computation of elementary functions on the IBM
+// RISC System/6000, IBM J. Res. Dev. 34, 1990).
+__device__ __forceinline__ float div_in_range(float n, float m)
+{
+  float y = __builtin_amdgcn_rcpf(m);
+  y = __builtin_fmaf(__builtin_fmaf(-m, y, 1.0f), y, y);
+  float q = n * y;
+  q = __builtin_fmaf(__builtin_fmaf(-m, q, n), y, q);
+  return __builtin_fmaf(__builtin_fmaf(-m, q, n), y, q);
+}
+
+// Two lanes per target: the even lane holds state 0, the odd one state 1, and a
+// row takes the other state's value with a DPP operand. A target's rows are one
+// serial chain and a wave runs alone on its SIMD for most lists, so the stage is
+// bound by the instructions of a row, 15 here. A row of one target: 104 ns with
+// both states and both divisions in one lane, 47 ns now.
 __global__ __launch_bounds__(64)
 void k_bias(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *__restrict__ off,
             const int32_t *__restrict__ len, const int32_t *__restrict__ list, const int32_t *__restrict__ count,
@@ -315,14 +334,15 @@ void k_bias(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *
             float *__restrict__ rowmax, int64_t rowmax_size, unsigned long long *cursor, int64_t *__restrict__ defer_off)
 {
 #pragma clang fp contract(off)
+  constexpr int OTHER = 0xB1;                    // quad_perm [1, 0, 3, 2]: the pair's other lane
   // the two states' odds of every residue code, in LDS
-  __shared__ float2 eo2[P7G_NROWS];
-  for (int x = threadIdx.x; x < P7G_NROWS; x += blockDim.x) eo2[x] = make_float2(p.eo[2*x], p.eo[2*x + 1]);
+  __shared__ float eo2[2 * P7G_NROWS];
+  for (int x = threadIdx.x; x < 2 * P7G_NROWS; x += blockDim.x) eo2[x] = p.eo[x];
   __syncthreads();
   const int64_t n = *count;
-  const int lane = threadIdx.x & 63;
-  for (int64_t t0 = (int64_t) blockIdx.x * blockDim.x; t0 < n; t0 += (int64_t) gridDim.x * blockDim.x) {
-    const int64_t t = t0 + threadIdx.x;
+  const int lane = threadIdx.x & 63, s = lane & 1;
+  for (int64_t t0 = (int64_t) blockIdx.x * 32; t0 < n; t0 += (int64_t) gridDim.x * 32) {
+    const int64_t t = t0 + (lane >> 1);
     const bool valid = t < n;
     const int slot = valid ? list[t] : 0;
     const int L = valid ? len[slot] : 0;
@@ -331,7 +351,7 @@ void k_bias(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *
     if (rowmax) {
       // whole 16-row blocks and the closing sum, in 16-byte aligned pieces
       const int64_t need = valid ? 16 * (((int64_t) L + 15) >> 4) + 4 : 0;
-      int64_t incl = need;
+      int64_t incl = s ? 0 : need;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) { const int64_t v = __shfl_up(incl, o, 64); if (lane >= o) incl += v; }
       unsigned long long b0 = 0;
@@ -344,79 +364,93 @@ void k_bias(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *
     const uint8_t *sq = res + off[slot];
     const float p1  = lc.on ? lc.p1 : __fdiv_rn((float) L, (float) (L + 1));
     const float t00 = p1, t01 = lc.on ? lc.q1 : 1.0f - p1;
-    const float t10 = p.ft1_0, t11 = p.ft1_1;
+    // this state's transitions from itself and from the other state
+    const float ts = s ? p.ft1_1 : t00, to = s ? t01 : p.ft1_0;
     float *rm = (base >= 0) ? rowmax + base : nullptr;
     float logsc = 0.0f;
     // Row 0 runs the same arithmetic as the others with the identity for the
     // transitions and (pi0, pi1) for the previous row: ((0 + pi0*1) + pi1*0)
     // * e0 is exactly pi0 * e0, the reference's first row.
-    float d0 = p.pi0, d1 = p.pi1;
-    float T00 = 1.0f, T01 = 0.0f, T10 = 0.0f, T11 = 1.0f;
-    float f0 = d0, f1 = d1;                      // (d0, d1) after the target's last row
+    float d = s ? p.pi1 : p.pi0;
+    float Ts = 1.0f, To = 0.0f;
+    float fin = d;                               // d after the target's last row
+    float mx;
+    // a row in the reference's order for any odds
+    auto row_any = [&](float e) {
+      const float ds = d * Ts, dot = dppz<OTHER>(d) * To;
+      const float nn = ((0.0f + (s ? dot : ds)) + (s ? ds : dot)) * e;
+      const float no = dppz<OTHER>(nn), n0 = s ? no : nn, n1 = s ? nn : no;
+      mx = 0.0f; mx = (n0 > mx) ? n0 : mx; mx = (n1 > mx) ? n1 : mx;
+      d = __fdiv_rn(nn, mx);
+      Ts = ts; To = to;
+    };
+    // the same for odds and transitions in range, all positive, so that the
+    // values' bit patterns order as integers
+    auto row_fast = [&](float e) {
+      const float nn = (d * Ts + dppz<OTHER>(d) * To) * e;
+      const int ni = __float_as_int(nn);
+      mx = __int_as_float(max(ni, dppi<OTHER>(0, ni)));
+      d = div_in_range(nn, mx);
+    };
     const uint4 *pc = (const uint4 *) sq;
     const int nblk = (L + 15) >> 4;
-    if (rm) {
+    const bool ok = p.bias_ok && t00 >= 0x1p-2f && t00 <= 1.0f && t01 >= 0x1p-32f && t01 <= 1.0f;
+    if (rm && __all(ok)) {
       // Straight-line blocks of 16 rows, so that the compiler can count the
       // memory operations in flight. At the top of block bk every access in
       // flight was issued a whole block earlier: the block's residue chunk,
       // and the stores of block bk-2's normalisers. The block then reads its
-      // odds pairs from LDS, requests the next chunk, stores block bk-1's
+      // odds from LDS, requests the next chunk, stores block bk-1's
       // normalisers (block 0 writes its own slot, rewritten a block later),
       // and runs its rows. Rows past the end compute values no one reads,
       // into the target's own whole-block room.
       uint4 cn = pc[0];
+      const float *es = eo2 + s;
       float qp[16];
 #pragma unroll
       for (int u = 0; u < 16; u++) qp[u] = 0.0f;
-      for (int bk = 0; bk < nblk; bk++) {
-        float2 eb[16];
-#pragma unroll
-        for (int u = 0; u < 16; u++) eb[u] = eo2[chunk_byte(cn, u)];
-        cn = pc[min(bk + 1, nblk)];             // the chunk after the target is still readable
-        {
-          float4 *o = (float4 *) (rm + max(bk - 1, 0) * 16);
-          o[0] = make_float4(qp[0], qp[1], qp[2], qp[3]);     o[1] = make_float4(qp[4], qp[5], qp[6], qp[7]);
-          o[2] = make_float4(qp[8], qp[9], qp[10], qp[11]);   o[3] = make_float4(qp[12], qp[13], qp[14], qp[15]);
-        }
-#pragma unroll
-        for (int u = 0; u < 16; u++) {
-          const float2 e = eb[u];
-          float n0 = 0.0f, n1 = 0.0f, mx;
-          n0 += d0 * T00; n0 += d1 * T10; n0 *= e.x;
-          mx = 0.0f; mx = (n0 > mx) ? n0 : mx;
-          n1 += d0 * T01; n1 += d1 * T11; n1 *= e.y;
-          mx = (n1 > mx) ? n1 : mx;
-          d0 = __fdiv_rn(n0, mx); d1 = __fdiv_rn(n1, mx);
-          qp[u] = mx;
-          if (u == 0) { T00 = t00; T01 = t01; T10 = t10; T11 = t11; }
-          const bool last = (bk * 16 + u == L - 1);
-          f0 = last ? d0 : f0; f1 = last ? d1 : f1;
-        }
-      }
-      if (nblk > 0) {
-        float4 *o = (float4 *) (rm + (nblk - 1) * 16);
+      auto put = [&](int bk) {
+        if (s) return;
+        float4 *o = (float4 *) (rm + bk * 16);
         o[0] = make_float4(qp[0], qp[1], qp[2], qp[3]);     o[1] = make_float4(qp[4], qp[5], qp[6], qp[7]);
         o[2] = make_float4(qp[8], qp[9], qp[10], qp[11]);   o[3] = make_float4(qp[12], qp[13], qp[14], qp[15]);
+      };
+      auto block = [&](int bk, auto last) {
+        float eb[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) eb[u] = es[2 * chunk_byte(cn, u)];
+        cn = pc[min(bk + 1, nblk)];             // the chunk after the target is still readable
+        put(max(bk - 1, 0));
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+          row_fast(eb[u]);
+          qp[u] = mx;
+          if (u == 0) { Ts = ts; To = to; }
+          if (decltype(last)::value) fin = (bk * 16 + u == L - 1) ? d : fin;
+        }
+      };
+      for (int bk = 0; bk < nblk - 1; bk++) block(bk, std::false_type());
+      if (nblk > 0) { block(nblk - 1, std::true_type()); put(nblk - 1); }
+    } else if (rm) {
+      // odds out of range: row by row
+      for (int i = 0; i < L; i++) {
+        row_any(eo2[2 * chunk_byte(pc[i >> 4], i) + s]);
+        if (! s) rm[i] = mx;
       }
+      fin = d;
     } else {
       // no room for the normalisers (pool exhausted): their logs are summed here
       for (int i = 0; i < L; i++) {
-        const float2 e = eo2[chunk_byte(pc[i >> 4], i)];
-        float n0 = 0.0f, n1 = 0.0f, mx;
-        n0 += d0 * T00; n0 += d1 * T10; n0 *= e.x;
-        mx = 0.0f; mx = (n0 > mx) ? n0 : mx;
-        n1 += d0 * T01; n1 += d1 * T11; n1 *= e.y;
-        mx = (n1 > mx) ? n1 : mx;
-        d0 = __fdiv_rn(n0, mx); d1 = __fdiv_rn(n1, mx);
+        row_any(eo2[2 * chunk_byte(pc[i >> 4], i) + s]);
         logsc += (float) log((double) mx);
-        T00 = t00; T01 = t01; T10 = t10; T11 = t11;
       }
-      f0 = d0; f1 = d1;
+      fin = d;
     }
-    d0 = f0; d1 = f1;
     // the closing sum; an empty target scores log(pi_end) = log(0) (esl_hmm.c:360-364)
+    const float fo = dppz<OTHER>(fin);
     float sfin = 0.0f;
-    if (L > 0) { sfin += d0 * 1.0f; sfin += d1 * 1.0f; }
+    if (L > 0) { sfin += (s ? fo : fin) * 1.0f; sfin += (s ? fin : fo) * 1.0f; }
+    if (s) continue;
     if (rm) {
       rm[L] = sfin;                            // after the block stores of the same lane
       defer_off[slot] = base;                  // k_bias_log + k_bias_sum finish it
@@ -438,17 +472,20 @@ void k_bias_log(float *__restrict__ rowmax, const unsigned long long *__restrict
 }
 
 // One target per wave: its L+1 logs added in row order, as esl_hmm_Forward
-// sums sc[1..L+1] (esl_hmm.c:403-405). The wave loads 64 terms at a time
-// (coalesced) and the sum takes them lane by lane, so the order of the float
-// additions is the reference's; a long target no longer waits on its own
-// dependent loads, one per four terms.
+// sums sc[1..L+1] (esl_hmm.c:403-405), so the order of the float additions is the
+// reference's and their latency bounds a long target. The wave loads 256 terms
+// ahead and passes them through LDS 64 at a time, from which every lane reads
+// them back four at a time and adds them all: an addition and a quarter of a
+// read per term. 35,000 terms: 121 us, 661 us with each term taken out of its
+// lane by v_readlane.
 __global__ __launch_bounds__(256)
 void k_bias_sum(const DevProfile p, const int32_t *__restrict__ len, const int32_t *__restrict__ list,
                 const int32_t *__restrict__ count, DevResults r, GateThresh g, int gating, LenCfg lc,
                 const float *__restrict__ rowmax, const int64_t *__restrict__ defer_off)
 {
 #pragma clang fp contract(off)
-  const int lane = threadIdx.x & 63;
+  __shared__ __attribute__((aligned(16))) float sh[4][2][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int64_t n = *count;
   for (int64_t t = wave_id(); t < n; t += wave_cnt()) {
     const int slot = uni(list[t]);
@@ -457,18 +494,31 @@ void k_bias_sum(const DevProfile p, const int32_t *__restrict__ len, const int32
     if (o < 0) continue;                       // finished in the first pass
     const int L = uni(len[slot]);
     const int nv = L + 1;                      // L row terms and the closing sum
+    const float *rw = rowmax + o;
     float logsc = 0.0f;
-    float v = (lane < nv) ? rowmax[o + lane] : 0.0f;
-    for (int base = 0; base < nv; base += 64) {
-      const float nxt = (base + 64 + lane < nv) ? rowmax[o + base + 64 + lane] : 0.0f;    // the next block in flight
-      const int cnt = min(64, nv - base);
-      int k = 0;
-      for (; k + 8 <= cnt; k += 8) {
+    float v[4], nx[4];
 #pragma unroll
-        for (int u = 0; u < 8; u++) logsc += readlanef(v, k + u);
+    for (int j = 0; j < 4; j++) v[j] = rw[min(64 * j + lane, L)];
+    for (int base = 0; base < nv; base += 256) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) nx[j] = rw[min(base + 256 + 64 * j + lane, L)];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int cnt = min(64, nv - base - 64 * j);
+        float *w = sh[wv][j & 1];
+        w[lane] = v[j];
+        // a wave's LDS operations complete in order: only the compiler is held
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        if (cnt == 64) {
+          float x[64];
+#pragma unroll
+          for (int k = 0; k < 64; k++) x[k] = w[k];
+#pragma unroll
+          for (int k = 0; k < 64; k++) logsc += x[k];
+        } else
+          for (int k = 0; k < cnt; k++) logsc += readlanef(v[j], k);
+        v[j] = nx[j];
       }
-      for (; k < cnt; k++) logsc += readlanef(v, k);
-      v = nxt;
     }
     if (lane == 0) bias_finish(p, r, g, gating, lc, slot, L, logsc);
   }
@@ -903,7 +953,7 @@ hipError_t launch_bias(const DevProfile &p, const DevSeqs &s, const int32_t *lis
                        float *rowmax, int64_t rowmax_size, int64_t *defer_off, hipStream_t st)
 {
   if (maxn <= 0) return hipSuccess;
-  unsigned grid = (unsigned) ((maxn + 63) / 64); if (grid > 8192) grid = 8192;
+  unsigned grid = (unsigned) ((maxn + 31) / 32); if (grid > 8192) grid = 8192;
   hipLaunchKernelGGL(k_bias, dim3(grid), dim3(64), 0, st, p, s.res, s.off, s.len, list, count, r, g, gating, lc,
                      rowmax, rowmax_size, l.cursor, defer_off);
   hipError_t e = hipGetLastError();

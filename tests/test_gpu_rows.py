@@ -111,3 +111,38 @@ def test_msv_rows_bit_exact(gpu, tmp_path, M):
     for i, s in enumerate(seqs):
         st0, sc0, _ = oracle.msv_filter(s, t, tjb=int(lm.tjb[len(s)]))
         assert st0 == st[i] and (sc0 == sc[i] or (np.isinf(sc0) and np.isinf(sc[i]))), (i, len(s), sc0, sc[i])
+
+
+@pytest.mark.parametrize("compo", ["converted", "steep", "tiny"])
+def test_bias_rows_bit_exact(gpu, tmp_path, compo):
+    """The bias filter around its blocks of 16 rows and of 64 and 256 summed terms, in batches
+    (pairs of lanes, a last wave part full) and as single targets (the row pool from 65
+    residues on), with odds in and out of the division's range."""
+    h = synth.random_profile(40, np.random.default_rng(10), "bias")
+    h.stats = (-9.0, 0.6931, -9.5, 0.6931, -5.0, 0.6931)
+    path = str(tmp_path / "bias.hmm")
+    synth.write_hmm(path, [h])
+    om = gpu.OProfile.from_file(path)
+    t = om.tables()
+    if compo != "converted":
+        c = t["compo"].copy()
+        c[:20] = 1e-3
+        c[0] = 1 - 19e-3
+        if compo == "tiny":
+            c[1:20] = 1e-12
+        t["compo"] = c
+        om.load(t)
+        t = om.tables()
+    rng = np.random.default_rng(11)
+    seqs = random_seqs(rng, [1, 2, 15, 16, 17, 31, 32, 33, 62, 63, 64, 65, 127, 128, 255, 256, 257, 319, 320, 511, 512, 1000] * 2)
+    seqs.append(np.zeros(300, np.uint8))                   # one residue only: the odds' ends
+    bh = oracle.bias_hmm(t)
+    got = gpu.filter_score_batch(om, gpu.SeqDB.from_list(seqs))
+    bg = gpu.Background(gpu.AMINO)
+    bg.set_filter(t["M"], t["compo"])
+    for i, s in enumerate(seqs):
+        p1 = np.float32(len(s)) / np.float32(len(s) + 1)
+        ref = oracle.filter_score(s, bh["eo"], p1, np.float32(1) - p1, bh["t10"], bh["t11"], bh["pi0"], bh["pi1"], p1)
+        assert ref == got[i], (i, len(s), ref, got[i])
+        bg.set_length(len(s))
+        assert bg.filter_score(s) == ref, (i, len(s))
