@@ -16,7 +16,8 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
            const float *__restrict__ fwd_xmx, float *__restrict__ xmx_out, LenCfg lc, DomBufs dom, DevLists l)
 {
   constexpr bool PIN = (TM == TM_LDS || TM == TM_PIN);
-  if ((int64_t) blockIdx.x * (blockDim.x >> 6) >= *count) return;
+  const int lw = list_waves(*count);
+  if ((int64_t) blockIdx.x * lw >= *count) return;
   extern __shared__ float ldsf[];
   const size_t rowf = (size_t) 64 * B;
   const float *tbl = p.fb_tbl;                           // emission rows
@@ -46,7 +47,9 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
   const float eMove = ENV ? 1.0f : p.xfE_move, eLoop = ENV ? 0.0f : p.xfE_loop;
 
   int32_t *queue = (int32_t *) count + P7G_QOFF;
+  if ((int) (threadIdx.x >> 6) >= lw) return;
   for (int64_t t = queue_next(queue, 1); t < n; t = queue_next(queue, 1)) {
+    list_prio(t);
     const int slot = uni(list[t]);
     const int L = uni(len[slot]);
     const uint8_t *sq = res + off[slot];
@@ -524,7 +527,7 @@ hipError_t launch_bck(const DevProfile &p, const DevSeqs &s, const int32_t *list
     default: return hipErrorInvalidValue;
   }
   const size_t lds = fb_lds(p, tm);
-  const unsigned grid = grid_for_waves_blk(k, maxn, lds, nthr / 64);
+  const unsigned grid = list_grid(k, maxn, lds, nthr / 64);
   void *args[] = { (void *) &p, (void *) &s.res, (void *) &s.off, (void *) &s.len, (void *) &list, (void *) &count,
                    &r, (void *) &scale_pool, (void *) &scale_off, (void *) &fwd_xmx, &xmx_out, &lc, (void *) &dom, &l };
   return launch(k, grid, nthr, args, lds, st);

@@ -263,7 +263,8 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
            DomBufs dom)
 {
   constexpr bool PIN = (TM == TM_LDS || TM == TM_PIN);
-  if ((int64_t) blockIdx.x * (blockDim.x >> 6) >= *count) return;
+  const int lw = list_waves(*count);
+  if ((int64_t) blockIdx.x * lw >= *count) return;
   extern __shared__ float ldsf[];
   const size_t rowf = (size_t) 64 * B;
   const float *tbl = p.fb_tbl;                           // emission rows
@@ -296,7 +297,9 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
   const float eMove = ENV ? 1.0f : p.xfE_move, eLoop = ENV ? 0.0f : p.xfE_loop;
 
   int32_t *queue = (int32_t *) count + P7G_QOFF;
+  if ((int) (threadIdx.x >> 6) >= lw) return;
   for (int64_t t = queue_next(queue, 1); t < n; t = queue_next(queue, 1)) {
+    list_prio(t);
     const int slot = uni(list[t]);
     const int L = uni(len[slot]);
     const uint8_t *sq = res + off[slot];
@@ -842,7 +845,7 @@ hipError_t launch_fwd(const DevProfile &p, const DevSeqs &s, const int32_t *list
   // them fits on a compute unit beside a multidomain region's wave
   if (dom.env_loop && dom.n2mode == 2) nthr = std::min(nthr, 256);
   const size_t lds = fb_lds(p, tm);
-  const unsigned grid = grid_for_waves_blk(k, maxn, lds, nthr / 64);
+  const unsigned grid = list_grid(k, maxn, lds, nthr / 64);
   void *args[] = { (void *) &p, (void *) &s.res, (void *) &s.off, (void *) &s.len, (void *) &list, (void *) &count,
                    &r, &l, &g, &gating, &lc, &scale_pool, &pool_size, &scale_off, &xmx_out, (void *) &dom };
   return launch(k, grid, nthr, args, lds, st);

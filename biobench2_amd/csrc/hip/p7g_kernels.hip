@@ -69,7 +69,8 @@ void k_msv_full(const DevProfile p, const int *__restrict__ tbl, int tbl_dwords,
                 const uint8_t *__restrict__ res, const int64_t *__restrict__ off, const int32_t *__restrict__ len,
                 const int32_t *__restrict__ list, const int32_t *__restrict__ count, int16_t *__restrict__ xj, LenCfg lc)
 {
-  if ((int64_t) blockIdx.x * (blockDim.x >> 6) >= *count) return;
+  const int lw = list_waves(*count);
+  if ((int64_t) blockIdx.x * lw >= *count) return;
   extern __shared__ int lds[];
   const int *rows = tbl;
   if (LDS) { stage_table(lds, tbl, (size_t) tbl_dwords); rows = lds; }
@@ -77,7 +78,9 @@ void k_msv_full(const DevProfile p, const int *__restrict__ tbl, int tbl_dwords,
   const int64_t n = *count;
   int32_t *queue = (int32_t *) count + P7G_QOFF;
 
+  if ((int) (threadIdx.x >> 6) >= lw) return;
   for (int64_t t = queue_next(queue, 1); t < n; t = queue_next(queue, 1)) {
+    list_prio(t);
     const int slot = uni(list[t]);
     const int L = uni(len[slot]);
     const uint8_t *sq = res + off[slot];
@@ -932,7 +935,7 @@ hipError_t launch_msv_full(const DevProfile &p, const DevSeqs &s, const int32_t 
     default: return hipErrorInvalidValue;
   }
   const size_t lds = (p.mf_ND <= 20) ? p.mf_dwords * 4 : 0;
-  const unsigned grid = grid_for_waves_blk(k, maxn, lds, LIST_BLOCK / 64);
+  const unsigned grid = list_grid(k, maxn, lds, LIST_BLOCK / 64);
   int tbl_dwords = (int) p.mf_dwords;
   void *args[] = { (void *) &p, (void *) &p.mf_tbl, &tbl_dwords, (void *) &s.res, (void *) &s.off, (void *) &s.len,
                    (void *) &list, (void *) &count, &xj, &lc };

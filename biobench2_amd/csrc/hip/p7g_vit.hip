@@ -150,7 +150,8 @@ void k_vit(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
 #pragma clang fp contract(off)
   static_assert(TM == TM_LDS || TM == TM_TLDS, "Viterbi tables are in LDS, whole or transitions only");
   constexpr bool PIN = (TM == TM_LDS), PMDS = (ND < 10 && ND != 6);
-  if ((int64_t) blockIdx.x * (blockDim.x >> 6) >= *count) return;
+  const int lw = list_waves(*count);
+  if ((int64_t) blockIdx.x * lw >= *count) return;
   extern __shared__ int lds[];
   const size_t rowd = (size_t) 64 * ND;
   const int *tbl = p.vf_tbl;                             // emission rows
@@ -172,7 +173,9 @@ void k_vit(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
   const int64_t n = *count;
 
   int32_t *queue = (int32_t *) count + P7G_QOFF;
+  if ((int) (threadIdx.x >> 6) >= lw) return;
   for (int64_t t = queue_next(queue, 1); t < n; t = queue_next(queue, 1)) {
+    list_prio(t);
     const int slot = uni(list[t]);
     const int L = uni(len[slot]);
     const uint8_t *sq = res + off[slot];
@@ -618,7 +621,7 @@ hipError_t launch_vit(const DevProfile &p, const DevSeqs &s, const int32_t *list
     VIT_CASE(20, TM_TLDS) VIT_CASE(24, TM_TLDS) VIT_CASE(32, TM_TLDS) VIT_CASE(40, TM_TLDS)
     default: return hipErrorInvalidValue;
   }
-  const unsigned grid = grid_for_waves_blk(k, maxn, lds, nthr / 64);
+  const unsigned grid = list_grid(k, maxn, lds, nthr / 64);
   void *args[] = { (void *) &p, (void *) &s.res, (void *) &s.off, (void *) &s.len, (void *) &list, (void *) &count,
                    &r, &l, &g, &gating, &lc };
   return launch(k, grid, nthr, args, lds, st);

@@ -146,3 +146,22 @@ def test_bias_rows_bit_exact(gpu, tmp_path, compo):
         assert ref == got[i], (i, len(s), ref, got[i])
         bg.set_length(len(s))
         assert bg.filter_score(s) == ref, (i, len(s))
+
+
+@pytest.mark.parametrize("n", [1, 5, 4500, 12000])
+def test_lists_give_every_target_its_score(gpu, tmp_path, n):
+    """Short lists run on four waves of a workgroup, long ones on all, by falling priority:
+    each target's scores are those of a list of its own few."""
+    rng = np.random.default_rng(12)
+    h = synth.random_profile(30, rng, "lists")
+    h.stats = (-9.0, 0.6931, -9.5, 0.6931, -5.0, 0.6931)
+    path = str(tmp_path / "lists.hmm")
+    synth.write_hmm(path, [h])
+    om = gpu.OProfile.from_file(path)
+    seqs = random_seqs(rng, rng.integers(1, 60, n))
+    db = gpu.SeqDB.from_list(seqs)
+    for batch in (gpu.viterbi_batch, gpu.forward_batch, gpu.backward_batch):
+        sc, st = batch(om, db)
+        for i in sorted({0, n // 2, n - 1, *rng.integers(0, n, 6).tolist()}):
+            one, st1 = batch(om, gpu.SeqDB.from_list([seqs[i]]))
+            assert st[i] == st1[0] and sc[i] == one[0], (i, sc[i], one[0])
