@@ -216,7 +216,12 @@ __host__ __device__ inline int md_ncp(int64_t Q) { return (int) ((8 * Q + 63) / 
 // LDS, in floats: the transitions staged for the Forward (10 rows of M + 2)
 // and the Forward's rows
 __host__ __device__ inline int64_t md_stage_floats(int M) { return (10 * ((int64_t) M + 2) + 3) & ~(int64_t) 3; }
-__host__ __device__ inline bool md_stage_t(int M) { return (md_stage_floats(M) + 32 * md_q(M)) * 4 <= P7G_LDS_MAX; }
+// the Forward's row buffers: lanes' q padded to whole 8-step chunks, 8 rows of
+// cells (512 where a wave's registers hold a row's constants), a zero cell, odds of 1
+__host__ __device__ inline int md_qs(int M) { return (int) (md_q(M) + 7) & ~7; }
+__host__ __device__ inline int64_t md_row_floats(int M)
+{ return 4 * md_qs(M) <= 512 ? 8 * 512 + 4 + md_qs(M) : 32 * (int64_t) md_qs(M) + (md_qs(M) > md_q(M) ? 0 : 4); }
+__host__ __device__ inline bool md_stage_t(int M) { return (md_stage_floats(M) + md_row_floats(M)) * 4 <= P7G_LDS_MAX; }
 // the replay's: 64 domains' null2 odds (32 codes each) and records, then per
 // wave a domain's counts (4Q), then, when they fit beside one wave's counts,
 // the emission odds of 20 residues in striped order ([x][q][r])

@@ -124,13 +124,27 @@ __device__ __forceinline__ bool md_linked(const MdSeg &a, const MdSeg &b)
 
 struct MdSig { int c, i, j, k, m; float prob; };
 
+// The region's Forward matrix, one wave per region. The cells' M and I run on all
+// lanes; what the reference's operation order makes serial along q runs on lanes
+// 0..3 (its four SSE lanes), 10 cycles a step: the first D->D pass, beside which
+// lanes 4..7 take the M sum, then each later pass's carries, and the row's D sum.
+// Rows are kept per buffer in model order (cell (q, r) at r*QS + q), four steps to
+// an LDS access. A later pass only adds its carries to the cells, which all lanes
+// do; and where every D->D odds is at most 1 a pass is left out whose first
+// carry is too small to change any cell, for then none of its carries does.
+// 60 regions of up to 600 residues: M = 86 0.50 ms, M = 400 2.6 ms; with every
+// pass run in full by four lanes, cell by cell between LDS waits, 1.15 and 5.9 ms.
+// NU: models of up to 512 positions, NU cells per lane (c = 64 u + z), whose
+// transitions, places and odds are in registers; a step over them loads all
+// cells' operands before it stores any. 0: larger models, cell by cell.
+template <int NU>
 __global__ __launch_bounds__(64) void
 k_md_fwd(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__restrict__ jobs, float *__restrict__ pool)
 {
-  extern __shared__ float lds[];
+  extern __shared__ __attribute__((aligned(16))) float lds[];
   const int z = threadIdx.x;
   const MdJob J = jobs[blockIdx.x];
-  const int M = p.M, Q = max(2, (M - 1) / 4 + 1), Lr = J.Lr, L = J.Ltarget;
+  const int M = p.M, Q = max(2, (M - 1) / 4 + 1), QS = (Q + 7) & ~7, Lr = J.Lr, L = J.Ltarget;
   const int TR = p.nrows;                                  // first transition row of the table
   const float xEmove = p.xfE_move, xEloop = p.xfE_loop, floop = p.xf_loop[L], fmove = p.xf_move[L];
   const uint8_t *dsq = res + J.res_off;                    // residue i (1-based) at dsq[i-1]
@@ -151,192 +165,241 @@ k_md_fwd(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__res
   };
   enum { T_BM = 0, T_MM, T_IM, T_DM, T_MDS, T_DDS, T_MI, T_II, T_MD, T_DD };
 
-  // ---------------- 1. the region's Forward matrix ----------------
-  float *prev = ph, *cur = ph + 12 * Q, *tdd = ph + 24 * Q, *erow = ph + 28 * Q;   // erow: 4Q emissions
+  // two rows of M, D, I; the D->D odds; a scratch row (odds of models above 512
+  // positions; the carries of a pass); a zero cell, what precedes k = 1
+  constexpr bool pre = NU > 0;
+  constexpr int NC = pre ? NU : 1;
+  const int N = pre ? 512 : 4 * QS;                        // a buffer's cells
+  float *prev = ph, *cur = ph + 3 * N, *tdd = ph + 6 * N, *scr = ph + 7 * N;
+  const int zero = (QS > Q && ! pre) ? 6 * N + Q : 8 * N;   // index in ph (md_row_floats): the odds' padding, or a cell of its own
+  auto cell_k = [&](int c, int &q, int &r) { r = (c >= QS) + (c >= 2 * QS) + (c >= 3 * QS); q = c - r * QS; return r * Q + q + 1; };
   __syncthreads();
-  for (int c = z; c < 12 * Q; c += 64) { prev[c] = 0.0f; mat[c] = 0.0f; }
-  for (int c = z; c < 4 * Q; c += 64) tdd[c] = tv(T_DD, min((c & 3) * Q + (c >> 2) + 1, M + 1));
+  for (int c = z; c < 3 * N; c += 64) prev[c] = cur[c] = 0.0f;
+  for (int c = z; c < 12 * Q; c += 64) mat[c] = 0.0f;
+  if (z == 0 && zero == 8 * N) ph[zero] = 0.0f;
+  if (pre) for (int c = z; c < QS; c += 64) ph[8 * N + 4 + c] = 1.0f;      // odds of 1, for the M sum
+  bool le1 = true;
+  for (int c = z; c < N; c += 64) {
+    int q, r;
+    const int k = cell_k(c, q, r);
+    const float t = (q < Q) ? tv(T_DD, min(k, M + 1)) : 0.0f;
+    tdd[c] = t;
+    scr[c] = 0.0f;
+    // no odds above 1, and none out of the model's end into the cells behind it
+    le1 = le1 && t >= 0.0f && t <= 1.0f && (k < M || t == 0.0f);
+  }
+  const bool skips = __all(le1);
   float xN = 1.0f, xJ = 0.0f, xB = fmove, xC = 0.0f, xE = 0.0f;
   if (z == 0) { xmx[0] = 0.0f; xmx[1] = xN; xmx[2] = xJ; xmx[3] = xB; xmx[4] = xC; xmx[5] = 1.0f; }
   __syncthreads();
-  // a row's odds in striped order, eight per lane: loaded one row ahead
-  // while the row before is computed (models up to M = 512; larger ones load
-  // theirs at the row)
-  const bool pre = 4 * Q <= 64 * 8;
-  float enext[8];
+  // the residues 64 rows at a time; a row's odds one row ahead
+  const size_t xrow = (size_t) 64 * p.fb_B;
+  float enext[NC], ecur[NC], tBMr[NC], tMMr[NC], tIMr[NC], tDMr[NC], tMIr[NC], tIIr[NC], tMDr[NC];
+  int kr[NC], pr[NC], eo[NC], q0m = 0, xcur = 0;           // q0m: bit u where q = 0
+  int ro[3 * NC];                                          // what the row's [q][s][r] copy takes from
   auto load_row = [&](int i1) {
-    const int x = dsq[i1 - 1];
+    const int s = (i1 - 1) & 63;
+    if (s == 0) xcur = dsq[min(i1 - 1 + z, Lr - 1)];
+    const float *er = p.fb_tbl + (size_t) __builtin_amdgcn_readlane(xcur, s) * xrow;
 #pragma unroll
-    for (int u = 0; u < 8; u++) { const int c = u * 64 + z; enext[u] = md_tv(p, x, (c & 3) * Q + (c >> 2) + 1); }
+    for (int u = 0; u < NC; u++) enext[u] = er[eo[u]];
   };
-  // with the row's odds in registers (pre), lane z's cells are c = 64 u + z
-  // for u < 8, and their transitions are the row loop's constants: in
-  // registers too
-  float ecur[8], tBMr[8], tMMr[8], tIMr[8], tDMr[8], tMIr[8], tIIr[8], tMDr[8];
   if (pre) {
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int c = u * 64 + z, q = c >> 2, r = c & 3, k = r * Q + q + 1, kk = min(k, M + 1);
-      const bool in = c < 4 * Q;
+    for (int u = 0; u < NC; u++) {
+      const int c = u * 64 + z;
+      int q, r;
+      const int k = cell_k(c, q, r), kk = min(k, M + 1);
+      const bool in = q < Q;
+      kr[u] = in ? k : 0;
+      // model position k in the device table (past M: any, not used)
+      const int kz = min(max(k, 1), M) - 1, zl = kz / p.fb_B;
+      eo[u] = (kz - zl * p.fb_B) * 64 + zl;
+      q0m |= (int) (q == 0) << u;
+      // row i-1's predecessor, as an index from prev (none: far out, see cells)
+      pr[u] = (q > 0) ? c - 1 : (r > 0) ? (r - 1) * QS + Q - 1 : -1;
       tBMr[u] = in ? tv(T_BM, kk) : 0.0f; tMMr[u] = in ? tv(T_MM, kk) : 0.0f;
       tIMr[u] = in ? tv(T_IM, kk) : 0.0f; tDMr[u] = in ? tv(T_DM, kk) : 0.0f;
       tMIr[u] = in ? tv(T_MI, kk) : 0.0f; tIIr[u] = in ? tv(T_II, kk) : 0.0f;
-      tMDr[u] = in ? tv(T_MD, min(k - 1, M + 1)) : 0.0f;
+      tMDr[u] = (in && q > 0) ? tv(T_MD, min(k - 1, M + 1)) : 0.0f;
+    }
+#pragma unroll
+    for (int v = 0; v < 3 * NC; v++) {
+      const int c = min(v * 64 + z, 12 * Q - 1), q = c / 12, s = (c - 12 * q) >> 2;
+      ro[v] = s * N + (c & 3) * QS + q;
     }
     load_row(1);
   }
+  // M and I of a cell from row i-1 (esl_sse_rightshift_ps at q = 0)
+  auto cell_m = [&](float mp, float dp, float ip, float e, float bm, float mm, float im, float dm) {
+    float sv = __fmul_rn(xB, bm);
+    sv = __fadd_rn(sv, __fmul_rn(mp, mm));
+    sv = __fadd_rn(sv, __fmul_rn(ip, im));
+    sv = __fadd_rn(sv, __fmul_rn(dp, dm));
+    return __fmul_rn(sv, e); };
+  auto cell_i = [&](float m, float i, float mi, float ii) { return __fadd_rn(__fmul_rn(m, mi), __fmul_rn(i, ii)); };
+  // A chain along q over one or two arrays, eight steps' values loaded while the
+  // eight before run. f(q, u, a, b): the step, from a = A[q], b = T[q]; what it
+  // returns goes to dst[q] where there is one.
+  auto chain = [&](const float *A, const float *T, float *dst, auto f) {
+    auto ld = [&](const float *x, int q, float (&v)[8]) {
+      const float4 *w = (const float4 *) (x + q);
+      const float4 w0 = w[0], w1 = w[1];
+      v[0] = w0.x; v[1] = w0.y; v[2] = w0.z; v[3] = w0.w; v[4] = w1.x; v[5] = w1.y; v[6] = w1.z; v[7] = w1.w; };
+    auto run = [&](int q, const float (&a)[8], const float (&b)[8]) {
+      float o[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) o[u] = f(a[u], T ? b[u] : 0.0f);
+      if (dst) {
+        float4 *w = (float4 *) (dst + q);
+        w[0] = make_float4(o[0], o[1], o[2], o[3]); w[1] = make_float4(o[4], o[5], o[6], o[7]);
+      } };
+    auto tail = [&](int q, const float (&a)[8], const float (&b)[8]) {
+#pragma unroll
+      for (int u = 0; u < 7; u++)
+        if (q + u < Q) { const float o = f(a[u], T ? b[u] : 0.0f); if (dst) dst[q + u] = o; } };
+    float a0[8], b0[8], a1[8], b1[8];
+    ld(A, 0, a0); if (T) ld(T, 0, b0);
+    int q = 0;
+    for (; q + 16 <= Q; q += 16) {
+      ld(A, q + 8, a1); if (T) ld(T, q + 8, b1);
+      run(q, a0, b0);
+      const int qn = min(q + 16, QS - 8);
+      ld(A, qn, a0); if (T) ld(T, qn, b0);
+      run(q + 8, a1, b1);
+    }
+    if (q + 8 <= Q) {
+      const int qn = min(q + 8, QS - 8);
+      ld(A, qn, a1); if (T) ld(T, qn, b1);
+      run(q, a0, b0);
+      tail(q + 8, a1, b1);
+    } else tail(q, a0, b0);
+  };
   for (int i = 1; i <= Lr; i++) {
     if (pre) {
 #pragma unroll
-      for (int u = 0; u < 8; u++) ecur[u] = enext[u];
+      for (int u = 0; u < NC; u++) ecur[u] = ((unsigned) (kr[u] - 1) < (unsigned) M) ? enext[u] : 0.0f;
       if (i < Lr) load_row(i + 1);
-    } else {
-      const int x = dsq[i - 1];
-      for (int c0 = 0; c0 < 4 * Q; c0 += 64 * 8) {         // this residue's odds, striped order
-        float e[8];
+      md_sync();
+      float mp[NC], dp[NC], ip[NC], m0[NC], i0[NC];
 #pragma unroll
-        for (int u = 0; u < 8; u++) { const int c = c0 + u * 64 + z; e[u] = md_tv(p, x, (c & 3) * Q + (c >> 2) + 1); }
-#pragma unroll
-        for (int u = 0; u < 8; u++) { const int c = c0 + u * 64 + z; if (c < 4 * Q) erow[c] = e[u]; }
+      for (int u = 0; u < NC; u++) {
+        const float *P = (pr[u] >= 0) ? prev + pr[u] : ph + zero;
+        const int dn = (pr[u] >= 0) ? N : 0;
+        mp[u] = P[0]; dp[u] = P[dn]; ip[u] = P[2 * dn]; m0[u] = prev[u * 64 + z]; i0[u] = prev[2 * N + u * 64 + z];
       }
-    }
-    md_sync();
-    if (pre) {
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int c = u * 64 + z, q = c >> 2, r = c & 3;
-        if (c < 4 * Q) {
-          float mp = 0.0f, dp = 0.0f, ip = 0.0f;       // row i-1 at k-1 (esl_sse_rightshift_ps at q = 0)
-          if (q > 0)      { mp = prev[((q-1)*3+0)*4 + r]; dp = prev[((q-1)*3+1)*4 + r]; ip = prev[((q-1)*3+2)*4 + r]; }
-          else if (r > 0) { mp = prev[((Q-1)*3+0)*4 + r-1]; dp = prev[((Q-1)*3+1)*4 + r-1]; ip = prev[((Q-1)*3+2)*4 + r-1]; }
-          float sv = __fmul_rn(xB, tBMr[u]);
-          sv = __fadd_rn(sv, __fmul_rn(mp, tMMr[u]));
-          sv = __fadd_rn(sv, __fmul_rn(ip, tIMr[u]));
-          sv = __fadd_rn(sv, __fmul_rn(dp, tDMr[u]));
-          sv = __fmul_rn(sv, ecur[u]);
-          cur[(q*3+0)*4 + r] = sv;
-          cur[(q*3+2)*4 + r] = __fadd_rn(__fmul_rn(prev[(q*3+0)*4 + r], tMIr[u]),
-                                         __fmul_rn(prev[(q*3+2)*4 + r], tIIr[u]));
-        }
+      for (int u = 0; u < NC; u++) {
+        m0[u] = cell_i(m0[u], i0[u], tMIr[u], tIIr[u]);
+        mp[u] = cell_m(mp[u], dp[u], ip[u], ecur[u], tBMr[u], tMMr[u], tIMr[u], tDMr[u]);
       }
+#pragma unroll
+      for (int u = 0; u < NC; u++) { cur[u * 64 + z] = mp[u]; cur[2 * N + u * 64 + z] = m0[u]; }
       md_sync();
       // D before the D->D passes: cell q holds M(q-1)·tMD (the q loop's dcv); q = 0 holds 0
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int c = u * 64 + z, q = c >> 2, r = c & 3;
-        if (c < 4 * Q) cur[(q*3+1)*4 + r] = q ? __fmul_rn(cur[((q-1)*3+0)*4 + r], tMDr[u]) : 0.0f;
-      }
+      for (int u = 0; u < NC; u++) mp[u] = cur[max(pr[u], 0)];
+#pragma unroll
+      for (int u = 0; u < NC; u++) cur[N + u * 64 + z] = (((q0m >> u) & 1) || kr[u] == 0) ? 0.0f : __fmul_rn(mp[u], tMDr[u]);
     } else {
-    for (int c = z; c < 4 * Q; c += 64) {
-      const int q = c >> 2, r = c & 3, k = r * Q + q + 1, kk = min(k, M + 1);
-      float mp = 0.0f, dp = 0.0f, ip = 0.0f;           // row i-1 at k-1 (esl_sse_rightshift_ps at q = 0)
-      if (q > 0)      { mp = prev[((q-1)*3+0)*4 + r]; dp = prev[((q-1)*3+1)*4 + r]; ip = prev[((q-1)*3+2)*4 + r]; }
-      else if (r > 0) { mp = prev[((Q-1)*3+0)*4 + r-1]; dp = prev[((Q-1)*3+1)*4 + r-1]; ip = prev[((Q-1)*3+2)*4 + r-1]; }
-      float sv = __fmul_rn(xB, tv(T_BM, kk));
-      sv = __fadd_rn(sv, __fmul_rn(mp, tv(T_MM, kk)));
-      sv = __fadd_rn(sv, __fmul_rn(ip, tv(T_IM, kk)));
-      sv = __fadd_rn(sv, __fmul_rn(dp, tv(T_DM, kk)));
-      sv = __fmul_rn(sv, erow[c]);
-      cur[(q*3+0)*4 + r] = sv;
-      cur[(q*3+2)*4 + r] = __fadd_rn(__fmul_rn(prev[(q*3+0)*4 + r], tv(T_MI, kk)),
-                                     __fmul_rn(prev[(q*3+2)*4 + r], tv(T_II, kk)));
+      const int x = dsq[i - 1];
+      for (int c0 = 0; c0 < N; c0 += 64 * 8) {             // this residue's odds
+        float e[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) { const int c = c0 + u * 64 + z; int q, r; const int k = cell_k(c, q, r); e[u] = md_tv(p, x, (c < N && q < Q) ? k : 0); }
+#pragma unroll
+        for (int u = 0; u < 8; u++) { const int c = c0 + u * 64 + z; if (c < N) scr[c] = e[u]; }
+      }
+      md_sync();
+      for (int c = z; c < N; c += 64) {
+        int q, r;
+        const int k = cell_k(c, q, r), kk = min(k, M + 1), pc = (q > 0) ? c - 1 : (r > 0) ? (r - 1) * QS + Q - 1 : -1;
+        if (q < Q) {
+          const float *P = (pc >= 0) ? prev + pc : ph + zero;
+          const int dn = (pc >= 0) ? N : 0;
+          const float m = cell_m(P[0], P[dn], P[2 * dn], scr[c], tv(T_BM, kk), tv(T_MM, kk), tv(T_IM, kk), tv(T_DM, kk));
+          cur[2 * N + c] = cell_i(prev[c], prev[2 * N + c], tv(T_MI, kk), tv(T_II, kk));
+          cur[c] = m;
+        }
+      }
+      md_sync();
+      for (int c = z; c < N; c += 64) {
+        int q, r;
+        const int k = cell_k(c, q, r);
+        if (q < Q) cur[N + c] = q ? __fmul_rn(cur[c - 1], tv(T_MD, min(k - 1, M + 1))) : 0.0f;
+      }
     }
     md_sync();
-    // D before the D->D passes: cell q holds M(q-1)·tMD (the q loop's dcv); q = 0 holds 0
-    for (int c = z; c < 4 * Q; c += 64) {
-      const int q = c >> 2, r = c & 3, k = r * Q + q + 1;
-      cur[(q*3+1)*4 + r] = q ? __fmul_rn(cur[((q-1)*3+0)*4 + r], tv(T_MD, min(k - 1, M + 1))) : 0.0f;
+    const int r4 = z & 3;
+    float dcv = 0.0f, xm;
+    if (z < 8) {
+      // lanes 0..3: D(q) = dcv + D0(q), dcv = D(q)·tDD(q); lanes 4..7: the M sum
+      // in the same steps, with odds of 1, its partial sums to the scratch row
+      const bool dl = z < 4;
+      const float end = __fmul_rn(cur[r4 * QS + Q - 1], tv(T_MD, min(r4 * Q + Q, M + 1)));
+      const float sh = __shfl(end, (z + 3) & 3, 4);
+      float acc = (dl && r4) ? sh : 0.0f;
+      chain(cur + (dl ? N : 0) + r4 * QS, (dl || ! pre) ? tdd + r4 * QS : ph + 8 * N + 4, (dl ? cur + N : scr) + r4 * QS, [&](float d, float t) {
+        const float o = __fadd_rn(acc, d);
+        acc = __fmul_rn(o, (pre || dl) ? t : 1.0f);
+        return o; });
+      dcv = acc;
     }
-    }
+    xm = __shfl(dcv, 4 + r4, 64);                          // lane r: the M sum of its lane
     md_sync();
+    for (int pass = 1; pass < 4; pass++) {
+      const float sh = __shfl(dcv, (z + 3) & 3, 4);
+      dcv = (z < 4 && r4) ? sh : 0.0f;
+      if (skips && pass > 1) {
+        // the carry against the smallest D of the cells it can reach (positive
+        // values, whose bit patterns order as integers)
+        int big = 0;
+        auto take = [&](int k, float d) { if (k > Q && k <= M) big = max(big, 0x7f800000 - __float_as_int(d)); };
+        if (pre) {
+          float d[NC];
+#pragma unroll
+          for (int u = 0; u < NC; u++) d[u] = cur[N + u * 64 + z];
+#pragma unroll
+          for (int u = 0; u < NC; u++) take(kr[u], d[u]);
+        } else
+          for (int c = z; c < N; c += 64) { int q, r; const int k = cell_k(c, q, r); if (q < Q) take(k, cur[N + c]); }
+        const float dmin = __int_as_float(0x7f800000 - uni(wave_max_i(big)));
+        if (__all(dcv == 0.0f || (dcv > 0.0f && dcv < dmin * 0x1p-26f && dmin >= 0x1p-90f && dmin < INFINITY))) break;
+      }
+      if (z < 4) {
+        float acc = dcv;
+        chain(tdd + z * QS, nullptr, scr + z * QS, [&](float t, float) { const float o = acc; acc = __fmul_rn(acc, t); return o; });
+        dcv = acc;
+      }
+      md_sync();
+      bool changed = false;
+      if (pre) {
+        float d[NC], g[NC];
+#pragma unroll
+        for (int u = 0; u < NC; u++) { d[u] = cur[N + u * 64 + z]; g[u] = scr[u * 64 + z]; }
+#pragma unroll
+        for (int u = 0; u < NC; u++) {
+          const float dd = (kr[u] > 0) ? __fadd_rn(g[u], d[u]) : 0.0f;
+          changed = changed || dd > d[u];
+          cur[N + u * 64 + z] = dd;
+        }
+      } else
+        for (int c = z; c < N; c += 64) {
+          int q, r;
+          (void) cell_k(c, q, r);
+          if (q < Q) {
+            const float d = cur[N + c], dd = __fadd_rn(scr[c], d);
+            changed = changed || dd > d;
+            cur[N + c] = dd;
+          }
+        }
+      md_sync();
+      if (M >= 100 && ! __any(changed)) break;
+    }
     float xe = 0.0f;
-    if (z < 4) {                                         // lane z is SSE lane r
-      // The row's sums along q and its D->D passes, each a chain in q order
-      // (esl_sse_hsum_ps's lanes, fwdback.c's D passes): M(q) at cm[12 q],
-      // D(q) at cd[12 q], tDD(q) at tq[4 q]. Eight cells at a time, the next
-      // eight's loads issued before this eight's chain. The M sum and the
-      // first pass are independent chains and run together; every later
-      // pass also sums its new D values onto the M sum, so that the last
-      // pass leaves the row's total (its D values are the final ones).
-      const int r = z;
-      float *cm = cur + r, *cd = cur + 4 + r;
-      const float *tq = tdd + r;
-      float dcv = __fmul_rn(cur[((Q-1)*3+0)*4 + r], tv(T_MD, min(r * Q + Q, M + 1)));
-      float sh = __shfl(dcv, (z + 3) & 3, 4);
-      dcv = r ? sh : 0.0f;
-      // Reads past the row's last q stay inside the phase's LDS (the next
-      // buffers) and feed no result.
-      float xm = 0.0f;
-      {
-        // two chunk buffers in turn: the next chunk loads into one while
-        // the other's chain runs
-        float am[8], ad[8], at[8], bm[8], bd[8], bt[8];
-        auto ld = [&](int q0, float (&m)[8], float (&d)[8], float (&t)[8]) {
-#pragma unroll
-          for (int u = 0; u < 8; u++) { m[u] = cm[12*(q0+u)]; d[u] = cd[12*(q0+u)]; t[u] = tq[4*(q0+u)]; }
-        };
-        auto run = [&](int q0, const float (&m)[8], const float (&d)[8], const float (&t)[8]) {
-          auto step = [&](int u) {
-            xm = __fadd_rn(xm, m[u]);
-            const float dd = __fadd_rn(dcv, d[u]);
-            dcv = __fmul_rn(dd, t[u]);
-            cd[12*(q0+u)] = dd;
-          };
-          if (q0 + 8 <= Q) {
-#pragma unroll
-            for (int u = 0; u < 8; u++) step(u);
-          } else {
-#pragma unroll
-            for (int u = 0; u < 8; u++) if (q0 + u < Q) step(u);
-          }
-        };
-        ld(0, am, ad, at);
-        for (int q0 = 0; q0 < Q; q0 += 16) {
-          if (q0 + 8 < Q) ld(q0 + 8, bm, bd, bt);
-          run(q0, am, ad, at);
-          if (q0 + 8 >= Q) break;
-          if (q0 + 16 < Q) ld(q0 + 16, am, ad, at);
-          run(q0 + 8, bm, bd, bt);
-        }
-      }
-      for (int pass = 1; pass < 4; pass++) {
-        sh = __shfl(dcv, (z + 3) & 3, 4);
-        dcv = r ? sh : 0.0f;
-        int changed = 0;
-        float xd = xm;
-        float ad[8], at[8], bd[8], bt[8];
-        auto ld = [&](int q0, float (&d)[8], float (&t)[8]) {
-#pragma unroll
-          for (int u = 0; u < 8; u++) { d[u] = cd[12*(q0+u)]; t[u] = tq[4*(q0+u)]; }
-        };
-        auto run = [&](int q0, const float (&d)[8], const float (&t)[8]) {
-          auto step = [&](int u) {
-            const float dd = __fadd_rn(dcv, d[u]);
-            changed |= (dd > d[u]);
-            dcv = __fmul_rn(dcv, t[u]);
-            xd = __fadd_rn(dd, xd);
-            cd[12*(q0+u)] = dd;
-          };
-          if (q0 + 8 <= Q) {
-#pragma unroll
-            for (int u = 0; u < 8; u++) step(u);
-          } else {
-#pragma unroll
-            for (int u = 0; u < 8; u++) if (q0 + u < Q) step(u);
-          }
-        };
-        ld(0, ad, at);
-        for (int q0 = 0; q0 < Q; q0 += 16) {
-          if (q0 + 8 < Q) ld(q0 + 8, bd, bt);
-          run(q0, ad, at);
-          if (q0 + 8 >= Q) break;
-          if (q0 + 16 < Q) ld(q0 + 16, ad, at);
-          run(q0 + 8, bd, bt);
-        }
-        xe = xd;
-        const bool any = (__ballot(changed) & 0xfull) != 0ull;
-        if (M >= 100 && ! any) break;
-      }
+    if (z < 4) {                                           // the row's sum: the M sum, then D in q order
+      xe = xm;
+      chain(cur + N + z * QS, nullptr, nullptr, [&](float d, float) { xe = __fadd_rn(d, xe); return 0.0f; });
     }
     // esl_sse_hsum_ps: (e0 + e1) + (e2 + e3)
     xE = __fadd_rn(__fadd_rn(readlanef(xe, 0), readlanef(xe, 1)), __fadd_rn(readlanef(xe, 2), readlanef(xe, 3)));
@@ -349,13 +412,23 @@ k_md_fwd(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__res
     if (xE > 1.0e4f) {
       xN = __fdiv_rn(xN, xE); xC = __fdiv_rn(xC, xE); xJ = __fdiv_rn(xJ, xE); xB = __fdiv_rn(xB, xE);
       const float inv = (float) (1.0 / (double) xE);
-      for (int c = z; c < 12 * Q; c += 64) cur[c] = __fmul_rn(cur[c], inv);
+      for (int c = z; c < 3 * N; c += 64) cur[c] = __fmul_rn(cur[c], inv);
       scale = xE;
       xE = 1.0f;
       md_sync();
     }
     float *row = mat + (size_t) i * 12 * Q;
-    for (int c = z; c < 12 * Q; c += 64) row[c] = cur[c];
+    if (pre) {                                             // [q][s][r]
+      float v[3 * NC];
+#pragma unroll
+      for (int j = 0; j < 3 * NC; j++) v[j] = cur[ro[j]];
+#pragma unroll
+      for (int j = 0; j < 3 * NC; j++) if (j * 64 + z < 12 * Q) row[j * 64 + z] = v[j];
+    } else
+      for (int c = z; c < 12 * Q; c += 64) {
+        const int q = c / 12, s = (c - 12 * q) >> 2;
+        row[c] = cur[s * N + (c & 3) * QS + q];
+      }
     if (z == 0) {
       float *xr = xmx + (size_t) i * 6;
       xr[0] = xE; xr[1] = xN; xr[2] = xJ; xr[3] = xB; xr[4] = xC; xr[5] = scale;
@@ -925,7 +998,7 @@ k_md_replay(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__
 // LDS of one region's workgroup: the Forward's two rows and D->D odds, the
 // replay's odds and counts, or the clustering's stacks
 static size_t md_fwd_lds(int M)
-{ return (size_t) ((md_stage_t(M) ? md_stage_floats(M) : 0) + 32 * md_q(M) + 128) * 4; }
+{ return (size_t) ((md_stage_t(M) ? md_stage_floats(M) : 0) + md_row_floats(M)) * 4; }
 static size_t md_replay_lds(int M, int segcap)
 {
   const size_t clu = (size_t) 2 * segcap * 4 + (size_t) (segcap + 63) / 64 * 8 + (size_t) MD_MAXSIG * sizeof(MdSig);
@@ -1129,14 +1202,24 @@ hipError_t launch_md_regions(const DevProfile &p, const uint8_t *res, const MdJo
   if (njobs <= 0) return hipSuccess;
   const size_t lds0 = md_fwd_lds(p.M), lds = md_replay_lds(p.M, segcap);
   if (std::max(lds0, lds) > P7G_LDS_MAX) return hipErrorInvalidValue;
-  hipError_t e = hipFuncSetAttribute((const void *) k_md_fwd, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds0);
+  void *kf;
+  switch (4 * md_qs(p.M) <= 512 ? (4 * md_qs(p.M) + 63) / 64 : 0) {
+    case 1: kf = (void *) k_md_fwd<1>; break;
+    case 2: kf = (void *) k_md_fwd<2>; break;
+    case 3: case 4: kf = (void *) k_md_fwd<4>; break;
+    case 5: case 6: kf = (void *) k_md_fwd<6>; break;
+    case 7: case 8: kf = (void *) k_md_fwd<8>; break;
+    default: kf = (void *) k_md_fwd<0>; break;
+  }
+  hipError_t e = hipFuncSetAttribute((const void *) kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds0);
   if (e == hipSuccess) e = hipFuncSetAttribute((const void *) k_md_replay, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
   if (e != hipSuccess) return e;
   // the Forward matrices (one wave per region, the Forward's LDS only), the
   // thresholds (the whole device), then the traces' walks and replays
-  // (128 floats past the rows: the D->D chains read up to seven cells past q = Q - 1)
-  hipLaunchKernelGGL(k_md_fwd, dim3(njobs), dim3(64), lds0, st, p, res, jobs, pool);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
+  {
+    void *args[] = { (void *) &p, (void *) &res, (void *) &jobs, (void *) &pool };
+    if ((e = hipLaunchKernel(kf, dim3(njobs), dim3(64), args, lds0, st)) != hipSuccess) return e;
+  }
   for (int j0 = 0; j0 < njobs; j0 += 65535) {
     const int nj = std::min(njobs - j0, 65535);
     hipLaunchKernelGGL(k_md_thr, dim3(32, nj), dim3(MD_THR_NT), md_thr_tl_bytes(p.M) + MD_THR_LDS_OUT, st, p, jobs + j0, pool);

@@ -3,7 +3,8 @@
 A trace's domains go to a log of runs that is read 64 entries at a time and
 holds all 200 traces of a region only from about M = 150 on; below, several
 passes fill it in turn. Covered: one-node, smallest and one-pass models, M at
-the edges of 4 striped lanes and 64, regions of one residue, around 64 residues
+the edges of 4 striped lanes and of 64 cells (the region's Forward holds up to
+eight per lane, M = 512, in registers), regions of one residue, around 64 residues
 and of several domains, and 1, 3 and 200 traces. The sampled domains and the
 clusters equal the oracle's exactly; the residues' null2 scores differ by logf's
 last bit per residue (1e-6 nats, as for the regions of whole searches).
@@ -17,7 +18,7 @@ from biobench2_amd import synth
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M", [1, 4, 5, 63, 64, 65, 149, 160, 400])
+@pytest.mark.parametrize("M", [1, 4, 5, 32, 33, 63, 64, 65, 128, 129, 149, 160, 256, 257, 384, 385, 400, 512, 513, 700])
 def test_traces_equal_the_oracle_at_log_and_region_edges(gpu, tmp_path, M):
     rng = np.random.default_rng([11, M])
     h = synth.random_profile(M, rng, f"traces_M{M}")
