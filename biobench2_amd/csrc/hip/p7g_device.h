@@ -345,6 +345,12 @@ int ssv_chunk_built(int ND);
 // launchers (p7g_kernels.hip)
 // p[0..nwords) = v, as a kernel (so that a captured graph holds no memset node)
 hipError_t launch_fill32(void *p, uint32_t v, int64_t nwords, hipStream_t st);
+// a single-target call's start and end (src, dst of 16-byte words; list null: no list)
+struct SingleIn  { const void *src1; void *dst1; int64_t n1; const void *src2; void *dst2; int64_t n2;
+                   int64_t *off; int32_t *len; int32_t L, which; int32_t *list, *counts; unsigned long long *cursor; };
+struct SingleOut { const float *src; float *dst; int64_t n; const void *w0; const int32_t *w1; int32_t *words; int half; };
+hipError_t launch_single_in(const SingleIn &a, hipStream_t st);
+hipError_t launch_single_out(const SingleOut &a, hipStream_t st);
 // dst[0..nwords) = src[0..nwords), device to device, as a kernel
 hipError_t launch_copy32(void *dst, const void *src, int64_t nwords, hipStream_t st);
 // With slots == NULL (every slot) targets that need the full recurrence are

@@ -711,6 +711,49 @@ hipError_t launch_fill32(void *p, uint32_t v, int64_t nwords, hipStream_t st)
   return hipGetLastError();
 }
 
+// The start of a single-target call, one launch in place of seven copies and
+// fills with a synchronisation among them: its residues and, when given, a second
+// array, read from pinned host memory in 16-byte words; the target's offset and
+// length; the cleared counts and cursor; and the stage's list of slot 0. The
+// single targets' fixed cost is the launches and copies around their stages:
+// five calls of 350 residues at M = 86 took 690 us, and 384 us with these kernels.
+__global__ __launch_bounds__(256)
+void k_single_in(SingleIn a)
+{
+  const int64_t i0 = (int64_t) blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t) gridDim.x * blockDim.x;
+  for (int64_t i = i0; i < a.n1; i += step) ((uint4 *) a.dst1)[i] = ((const uint4 *) a.src1)[i];
+  for (int64_t i = i0; i < a.n2; i += step) ((uint4 *) a.dst2)[i] = ((const uint4 *) a.src2)[i];
+  if (i0 < 16) {
+    a.counts[i0] = (a.list && i0 == a.which) ? 1 : 0;
+    ((uint32_t *) a.cursor)[i0] = 0u;
+  }
+  if (i0 == 0) {
+    *a.off = 0; *a.len = a.L;
+    if (a.list) a.list[0] = 0;
+  }
+}
+// Its end: two result words and, when given, rows of floats, to pinned host memory.
+__global__ __launch_bounds__(256)
+void k_single_out(SingleOut a)
+{
+  const int64_t i0 = (int64_t) blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t) gridDim.x * blockDim.x;
+  for (int64_t i = i0; i < a.n; i += step) a.dst[i] = a.src[i];
+  if (i0 == 0) { a.words[0] = a.half ? (int32_t) *(const int16_t *) a.w0 : *(const int32_t *) a.w0; a.words[1] = a.w1 ? *a.w1 : 0; }
+}
+
+hipError_t launch_single_in(const SingleIn &a, hipStream_t st)
+{
+  const unsigned grid = (unsigned) std::min<int64_t>((std::max(a.n1, a.n2) + 255) / 256 + 1, 64);
+  hipLaunchKernelGGL(k_single_in, dim3(grid), dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+hipError_t launch_single_out(const SingleOut &a, hipStream_t st)
+{
+  const unsigned grid = (unsigned) std::min<int64_t>(a.n / 256 + 1, 64);
+  hipLaunchKernelGGL(k_single_out, dim3(grid), dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_copy32(void *dst, const void *src, int64_t nwords, hipStream_t st)
 {
   if (nwords <= 0) return hipSuccess;

@@ -3134,32 +3134,77 @@ p7_gpu_tune_Load(const char *path)
 struct Single {
   uint8_t *res = nullptr; int64_t cap = 0;
   int64_t *off = nullptr; int32_t *len = nullptr;
-  float   *xmx = nullptr; int64_t xcap = 0;     // two (L+1)*6 buffers: forward, backward
+  float   *xmx = nullptr; int64_t xcap = 0;     // two (L+1)*6 buffers, each of whole 16-byte words: forward, backward
+  float   *eo = nullptr;                        // the bias filter's odds
+  uint8_t *pin = nullptr; int64_t pcap = 0;     // pinned host memory (single_pin)
 };
 static Single g_one;
 
+// The pinned buffer single targets pass through: 64 bytes of result words, then
+// an array of rows (or the bias filter's odds), then the residues. Kept between
+// calls up to SINGLE_PIN_KEEP bytes; a longer target's buffer is given back when
+// its call ends. All single-target calls hold g_lock.
+#define SINGLE_PIN_KEEP (8 << 20)
 static int
-single_stage(const uint8_t *dsq, int L, DevSeqs *s)
+single_pin(int64_t bytes)
 {
   Single &o = g_one;
+  if (bytes <= o.pcap) return p7G_OK;
+  if (o.pin) (void) hipHostFree(o.pin);
+  o.pin = nullptr; o.pcap = 0;
+  const int64_t cap = std::max<int64_t>(bytes, 1 << 18);
+  HIPCHK(hipHostMalloc((void **) &o.pin, (size_t) cap, hipHostMallocDefault));
+  o.pcap = cap;
+  return p7G_OK;
+}
+
+// Stages a target (and `rows`, nrows floats, to d_rows) and clears the counts,
+// with counts[which] = 1 and slot 0 in `list` when there is one. The pinned
+// buffer also has room for the rows the call returns.
+static int
+single_stage(const uint8_t *dsq, int L, DevSeqs *s, int32_t *list, int which, const float *rows, float *d_rows, int64_t nrows)
+{
+  Single &o = g_one;
+  int status;
   const int64_t need = (((int64_t) L + 15) & ~(int64_t) 15) + 16;
   if (need > o.cap) {
     if (o.res) (void) hipFree(o.res);
-    o.res = nullptr;
+    o.res = nullptr; o.cap = 0;
     HIPCHK(hipMalloc((void **) &o.res, (size_t) need));
     o.cap = need;
   }
   if (! o.off) { HIPCHK(hipMalloc((void **) &o.off, 64)); HIPCHK(hipMalloc((void **) &o.len, 64)); }
-  std::vector<uint8_t> h((size_t) need, P7G_PADCODE);
-  for (int i = 0; i < L; i++) h[i] = dsq[i + 1];
-  int64_t zero = 0;
-  HIPCHK(hipMemcpyAsync(o.res, h.data(), (size_t) need, hipMemcpyHostToDevice, g_stream));
-  HIPCHK(hipMemcpyAsync(o.off, &zero, sizeof(zero), hipMemcpyHostToDevice, g_stream));
-  HIPCHK(hipMemcpyAsync(o.len, &L, sizeof(int32_t), hipMemcpyHostToDevice, g_stream));
-  // the work buffers' stream-ordered use keeps `h` alive until the copies complete
-  HIPCHK(hipStreamSynchronize(g_stream));
+  const int64_t rbytes = (nrows * 4 + 15) & ~(int64_t) 15;
+  if ((status = single_pin(64 + rbytes + need)) != p7G_OK) return status;
+  uint8_t *pr = o.pin + 64, *ps = pr + rbytes;
+  if (rows) memcpy(pr, rows, (size_t) nrows * 4);
+  memcpy(ps, dsq + 1, (size_t) L);
+  memset(ps + L, P7G_PADCODE, (size_t) (need - L));
+  SingleIn a;
+  a.src1 = ps; a.dst1 = o.res; a.n1 = need / 16;
+  a.src2 = pr; a.dst2 = d_rows; a.n2 = rows ? rbytes / 16 : 0;
+  a.off = o.off; a.len = o.len; a.L = L; a.which = which;
+  a.list = list; a.counts = g_work.l.counts; a.cursor = g_work.l.cursor;
+  HIPCHK(launch_single_in(a, g_stream));
   s->res = o.res; s->off = o.off; s->len = o.len; s->nslot = 1;
   s->perm = nullptr; s->seg = nullptr; s->nseg = 0; s->nseg_slots = 0;
+  return p7G_OK;
+}
+
+// Waits for the call's results: two words (the first an int16 when half) and n
+// floats of rows.
+static int
+single_result(const void *w0, bool half, const int32_t *w1, int32_t out[2], const float *d_rows, float *rows, int64_t n)
+{
+  Single &o = g_one;
+  SingleOut a;
+  a.src = d_rows; a.dst = (float *) (o.pin + 64); a.n = n;
+  a.w0 = w0; a.w1 = w1; a.words = (int32_t *) o.pin; a.half = half ? 1 : 0;
+  HIPCHK(launch_single_out(a, g_stream));
+  HIPCHK(hipStreamSynchronize(g_stream));
+  memcpy(out, o.pin, 8);
+  if (n) memcpy(rows, o.pin + 64, (size_t) n * 4);
+  if (o.pcap > SINGLE_PIN_KEEP) { (void) hipHostFree(o.pin); o.pin = nullptr; o.pcap = 0; }
   return p7G_OK;
 }
 
@@ -3192,20 +3237,17 @@ single_msv(const uint8_t *dsq, int L, const P7_GPU_OPROFILE *om, int *ret_xj)
   if ((status = dev_profile(om, L, &p)) != p7G_OK) return status;
   if ((status = work_reserve(g_work, 1, 0)) != p7G_OK) return status;
   DevSeqs s;
-  if ((status = single_stage(dsq, L, &s)) != p7G_OK) return status;
+  if ((status = single_stage(dsq, L, &s, nullptr, 0, nullptr, nullptr, 0)) != p7G_OK) return status;
   Work &w = g_work;
   LenCfg lc = lencfg_of(om);
-  if ((status = reset_counts(g_work)) != p7G_OK) return status;
   if ((status = work_bnd(w, *p, g_one.cap)) != p7G_OK) return status;
   HIPCHK(launch_ssv_chosen(*p, s, nullptr, 1, w.r.zmax, &w.l.counts[P7G_Q_SSV], w.bnd, w.bnd_cap, g_stream));
   HIPCHK(launch_msv_classify(*p, s, nullptr, 1, w.r.zmax, w.r.xj, w.l.full, &w.l.counts[0], lc, g_stream));
   HIPCHK(launch_compact_i16(w.r.xj, -2, 1, w.l.full, &w.l.counts[0], w.tilecnt, g_stream));
   HIPCHK(launch_msv_full(*p, s, w.l.full, &w.l.counts[0], 1, w.r.xj, lc, g_stream));
-  int16_t xj; int32_t nfull;
-  HIPCHK(hipMemcpyAsync(&xj, w.r.xj, sizeof(xj), hipMemcpyDeviceToHost, g_stream));
-  HIPCHK(hipMemcpyAsync(&nfull, &w.l.counts[0], sizeof(nfull), hipMemcpyDeviceToHost, g_stream));
-  HIPCHK(hipStreamSynchronize(g_stream));
-  *ret_xj = (xj < 0) ? -1 : (nfull ? 1000 + xj : xj);
+  int32_t res[2];                                          // xJ, and whether the full recurrence ran
+  if ((status = single_result(w.r.xj, true, &w.l.counts[0], res, nullptr, nullptr, 0)) != p7G_OK) return status;
+  *ret_xj = (res[0] < 0) ? -1 : (res[1] ? 1000 + res[0] : res[0]);
   return p7G_OK;
 }
 
@@ -3256,27 +3298,22 @@ p7_gpu_ViterbiFilter(const uint8_t *dsq, int L, const P7_GPU_OPROFILE *om, P7_GP
   if ((status = dev_profile(om, L, &p)) != p7G_OK) return status;
   if ((status = work_reserve(g_work, 1, 0)) != p7G_OK) return status;
   DevSeqs s;
-  if ((status = single_stage(dsq, L, &s)) != p7G_OK) return status;
   Work &w = g_work;
   GateThresh g; memset(&g, 0, sizeof(g));
-  if ((status = reset_counts(g_work)) != p7G_OK) return status;
-  int32_t zero = 0, one = 1;
-  HIPCHK(hipMemcpyAsync(w.l.vit, &zero, sizeof(zero), hipMemcpyHostToDevice, g_stream));
-  HIPCHK(hipMemcpyAsync(&w.l.counts[2], &one, sizeof(one), hipMemcpyHostToDevice, g_stream));
+  if ((status = single_stage(dsq, L, &s, w.l.vit, 2, nullptr, nullptr, 0)) != p7G_OK) return status;
   HIPCHK(launch_vit(*p, s, w.l.vit, &w.l.counts[2], 1, w.r, w.l, g, 0, lencfg_of(om), g_stream));
-  float sc; int vst;
-  HIPCHK(hipMemcpyAsync(&sc, w.r.vfsc, sizeof(sc), hipMemcpyDeviceToHost, g_stream));
-  HIPCHK(hipMemcpyAsync(&vst, w.r.vstatus, sizeof(vst), hipMemcpyDeviceToHost, g_stream));
-  HIPCHK(hipStreamSynchronize(g_stream));
-  *ret_sc = sc;
-  return vst == 16 ? p7G_ERANGE : p7G_OK;
+  int32_t res[2];
+  if ((status = single_result(w.r.vfsc, false, w.r.vstatus, res, nullptr, nullptr, 0)) != p7G_OK) return status;
+  memcpy(ret_sc, &res[0], sizeof(float));
+  return res[1] == 16 ? p7G_ERANGE : p7G_OK;
 }
 
+static int64_t single_rows(int L) { return ((int64_t) (L + 1) * 6 + 3) & ~(int64_t) 3; }
 static int
 single_xmx(int L)
 {
   Single &o = g_one;
-  const int64_t need = (int64_t) (L + 1) * 6 * 2;
+  const int64_t need = single_rows(L) * 2;
   if (need > o.xcap) {
     if (o.xmx) (void) hipFree(o.xmx);
     o.xmx = nullptr;
@@ -3307,19 +3344,15 @@ p7_gpu_ForwardParser(const uint8_t *dsq, int L, const P7_GPU_OPROFILE *om, P7_GP
   if ((status = work_reserve(g_work, 1, 0)) != p7G_OK) return status;
   if ((status = single_xmx(L)) != p7G_OK) return status;
   DevSeqs s;
-  if ((status = single_stage(dsq, L, &s)) != p7G_OK) return status;
   Work &w = g_work;
   GateThresh g; memset(&g, 0, sizeof(g));
-  if ((status = reset_counts(g_work)) != p7G_OK) return status;
-  int32_t zero = 0, one = 1;
-  HIPCHK(hipMemcpyAsync(w.l.fwd, &zero, sizeof(zero), hipMemcpyHostToDevice, g_stream));
-  HIPCHK(hipMemcpyAsync(&w.l.counts[3], &one, sizeof(one), hipMemcpyHostToDevice, g_stream));
+  const int64_t nx = (int64_t) (L + 1) * 6;
+  if ((status = single_stage(dsq, L, &s, w.l.fwd, 3, nullptr, nullptr, nx)) != p7G_OK) return status;
   HIPCHK(launch_fwd(*p, s, w.l.fwd, &w.l.counts[3], 1, w.r, w.l, g, 0, lencfg_of(om), nullptr, 0, nullptr, g_one.xmx, g_stream));
-  float sc; int fst;
-  HIPCHK(hipMemcpyAsync(&sc, w.r.fwdsc, sizeof(sc), hipMemcpyDeviceToHost, g_stream));
-  HIPCHK(hipMemcpyAsync(&fst, w.r.fstatus, sizeof(fst), hipMemcpyDeviceToHost, g_stream));
-  HIPCHK(hipMemcpyAsync(fwd->xmx, g_one.xmx, sizeof(float) * (size_t) (L + 1) * 6, hipMemcpyDeviceToHost, g_stream));
-  HIPCHK(hipStreamSynchronize(g_stream));
+  int32_t res[2];
+  if ((status = single_result(w.r.fwdsc, false, w.r.fstatus, res, g_one.xmx, fwd->xmx, nx)) != p7G_OK) return status;
+  float sc; const int fst = res[1];
+  memcpy(&sc, &res[0], sizeof(sc));
   double ts = 0.0;
   for (int i = 1; i <= L; i++) { float sf = fwd->xmx[i*6 + 5]; if (sf != 1.0f) ts = (float) (ts + log((double) sf)); }
   fwd->totscale = (float) ts;
@@ -3345,20 +3378,15 @@ p7_gpu_BackwardParser(const uint8_t *dsq, int L, const P7_GPU_OPROFILE *om, cons
   if ((status = work_reserve(g_work, 1, 0)) != p7G_OK) return status;
   if ((status = single_xmx(L)) != p7G_OK) return status;
   DevSeqs s;
-  if ((status = single_stage(dsq, L, &s)) != p7G_OK) return status;
   Work &w = g_work;
-  if ((status = reset_counts(g_work)) != p7G_OK) return status;
-  int32_t zero = 0, one = 1;
-  float *d_fx = g_one.xmx, *d_bx = g_one.xmx + (size_t) (L + 1) * 6;
-  HIPCHK(hipMemcpyAsync(d_fx, fwd->xmx, sizeof(float) * (size_t) (L + 1) * 6, hipMemcpyHostToDevice, g_stream));
-  HIPCHK(hipMemcpyAsync(w.l.bck, &zero, sizeof(zero), hipMemcpyHostToDevice, g_stream));
-  HIPCHK(hipMemcpyAsync(&w.l.counts[4], &one, sizeof(one), hipMemcpyHostToDevice, g_stream));
+  const int64_t nx = (int64_t) (L + 1) * 6;
+  float *d_fx = g_one.xmx, *d_bx = g_one.xmx + single_rows(L);
+  if ((status = single_stage(dsq, L, &s, w.l.bck, 4, fwd->xmx, d_fx, nx)) != p7G_OK) return status;
   HIPCHK(launch_bck(*p, s, w.l.bck, &w.l.counts[4], 1, w.r, nullptr, nullptr, d_fx, d_bx, lencfg_of(om), g_stream));
-  float sc; int fst;
-  HIPCHK(hipMemcpyAsync(&sc, w.r.bcksc, sizeof(sc), hipMemcpyDeviceToHost, g_stream));
-  HIPCHK(hipMemcpyAsync(&fst, w.r.fstatus, sizeof(fst), hipMemcpyDeviceToHost, g_stream));
-  HIPCHK(hipMemcpyAsync(bck->xmx, d_bx, sizeof(float) * (size_t) (L + 1) * 6, hipMemcpyDeviceToHost, g_stream));
-  HIPCHK(hipStreamSynchronize(g_stream));
+  int32_t res[2];
+  if ((status = single_result(w.r.bcksc, false, w.r.fstatus, res, d_bx, bck->xmx, nx)) != p7G_OK) return status;
+  float sc; const int fst = res[1];
+  memcpy(&sc, &res[0], sizeof(sc));
   bck->has_own_scales = (fst & 0x100) ? 1 : 0;
   {
     double ts = log((double) bck->xmx[(size_t) L * 6 + 5]);
@@ -3390,29 +3418,24 @@ p7_gpu_bg_FilterScore(P7_GPU_BG *bg, const uint8_t *dsq, int L, float *ret_sc)
     DevProfile p; memset(&p, 0, sizeof(p));
     std::vector<float> eo(64, 1.0f);
     for (int x = 0; x < bg->abc->Kp; x++) { eo[x*2] = bg->eo[x][0]; eo[x*2+1] = bg->eo[x][1]; }
-    float *d_eo = nullptr;
-    HIPCHK(hipMalloc((void **) &d_eo, sizeof(float) * 64));
-    HIPCHK(hipMemcpyAsync(d_eo, eo.data(), sizeof(float) * 64, hipMemcpyHostToDevice, g_stream));
-    p.eo = d_eo; p.ft1_0 = bg->ft[1][0]; p.ft1_1 = bg->ft[1][1]; p.pi0 = bg->pi[0]; p.pi1 = bg->pi[1];
+    if (! g_one.eo) HIPCHK(hipMalloc((void **) &g_one.eo, sizeof(float) * 64));
+    p.eo = g_one.eo; p.ft1_0 = bg->ft[1][0]; p.ft1_1 = bg->ft[1][1]; p.pi0 = bg->pi[0]; p.pi1 = bg->pi[1];
     p.bias_ok = bias_in_range(eo.data(), bg->abc->Kp, p);
-    if ((status = work_reserve(g_work, 1, 0)) != p7G_OK) { (void) hipFree(d_eo); return status; }
+    if ((status = work_reserve(g_work, 1, 0)) != p7G_OK) return status;
     DevSeqs s;
-    if ((status = single_stage(dsq, L, &s)) != p7G_OK) { (void) hipFree(d_eo); return status; }
     Work &w = g_work;
+    if ((status = single_stage(dsq, L, &s, w.l.bias, 1, eo.data(), g_one.eo, 64)) != p7G_OK) return status;
     GateThresh g; memset(&g, 0, sizeof(g));
     LenCfg lc; memset(&lc, 0, sizeof(lc)); lc.on = 1; lc.p1 = bg->ft[0][0]; lc.q1 = bg->ft[0][1];
-    int32_t zero = 0, one = 1;
-    HIPCHK(hipMemcpyAsync(w.l.bias, &zero, sizeof(zero), hipMemcpyHostToDevice, g_stream));
-    HIPCHK(hipMemcpyAsync(&w.l.counts[1], &one, sizeof(one), hipMemcpyHostToDevice, g_stream));
     // The normalisers' logs are taken by kernels of their own where the rows
     // gain more than those launches cost (about 12 us): a row with its log in the
     // chain takes 390 ns, else 47 ns.
     const bool pool = (L > 64);
     HIPCHK(launch_bias(p, s, w.l.bias, &w.l.counts[1], 1, w.r, w.l, g, 0, lc, pool ? w.pool : nullptr, pool ? w.pool_size : 0,
                        pool ? w.scale_off : nullptr, g_stream));
-    HIPCHK(hipMemcpyAsync(&logsc, w.r.filtersc, sizeof(float), hipMemcpyDeviceToHost, g_stream));
-    HIPCHK(hipStreamSynchronize(g_stream));
-    (void) hipFree(d_eo);
+    int32_t res[2];
+    if ((status = single_result(w.r.filtersc, false, nullptr, res, nullptr, nullptr, 0)) != p7G_OK) return status;
+    memcpy(&logsc, &res[0], sizeof(float));
   }
   *ret_sc = logsc + (float) L * logf(bg->p1) + logf(1.-bg->p1);
   return p7G_OK;

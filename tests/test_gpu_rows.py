@@ -165,3 +165,34 @@ def test_lists_give_every_target_its_score(gpu, tmp_path, n):
         for i in sorted({0, n // 2, n - 1, *rng.integers(0, n, 6).tolist()}):
             one, st1 = batch(om, gpu.SeqDB.from_list([seqs[i]]))
             assert st[i] == st1[0] and sc[i] == one[0], (i, sc[i], one[0])
+
+
+@pytest.mark.parametrize("L", [1, 15, 16, 17, 4967, 360000])
+def test_single_targets_pass_through_the_pinned_buffer(gpu, tmp_path, L):
+    """Single-target calls of every size, up to rows past what the buffer keeps (8 MB), leave
+    each other's results alone and agree with the batched stages (Forward's two instances
+    may round differently: 1e-5 relative)."""
+    rng = np.random.default_rng([13, L])
+    h = synth.random_profile(20, rng, "single")
+    h.stats = (-9.0, 0.6931, -9.5, 0.6931, -5.0, 0.6931)
+    path = str(tmp_path / "single.hmm")
+    synth.write_hmm(path, [h])
+    om = gpu.OProfile.from_file(path)
+    small, s = random_seqs(rng, [33, L])
+
+    def calls(x):
+        om.reconfig_length(x.size)
+        f = gpu.forward_parser(x, om)
+        b = gpu.backward_parser(x, om, f[2])
+        return (gpu.msv_filter(x, om), gpu.viterbi_filter(x, om), f[:2], b[:2]), f[2].xmx()[0], b[2].xmx()[0]
+
+    first = calls(small)
+    got = calls(s)
+    again = calls(small)
+    assert first[0] == again[0] and np.array_equal(first[1], again[1]) and np.array_equal(first[2], again[2])
+    db = gpu.SeqDB.from_list([s])
+    (mst, m), (vst, v), (fst, f), (bst, b) = got[0]
+    for (sc, st), one, st1, tol in ((gpu.msv_batch(om, db), m, mst, 0), (gpu.viterbi_batch(om, db), v, vst, 0),
+                                    (gpu.forward_batch(om, db), f, fst, 1e-5), (gpu.backward_batch(om, db), b, bst, 1e-5)):
+        assert st[0] == st1 and abs(sc[0] - one) <= tol * max(1.0, abs(one)), (sc[0], one)
+    assert got[1].shape == (L + 1, 6) and np.isfinite(got[1]).all() and np.isfinite(got[2]).all()
