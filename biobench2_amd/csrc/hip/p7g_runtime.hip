@@ -1481,7 +1481,7 @@ stats_accumulate(P7_GPU_STATS &tot, const P7_GPU_STATS &one, bool first_of_call)
 }
 
 // Multidomain regions (p7_domaindef.c:431-476): each region's sampled traces
-// and clusters (k_md_region), in batches whose areas fit the multidomain pool.
+// and clusters (k_md_fwd to k_md_replay), in batches whose areas fit the multidomain pool.
 // Every cluster becomes a record of its own after the nregs regions (w = 2):
 // its residues copied from the region's copy, its envelope score computed as
 // the regions' were; its correction is the sum of the region's sampled null2
@@ -3442,7 +3442,7 @@ p7_gpu_bg_FilterScore(P7_GPU_BG *bg, const uint8_t *dsq, int L, float *ret_sc)
 }
 
 // region_trace_ensemble for one region (p7_domaindef.c:600-690, as
-// p7_domaindef_ByPosteriorHeuristics calls it at :440-446): k_md_region over
+// p7_domaindef_ByPosteriorHeuristics calls it at :440-446): the regions' kernels over
 // residues dsq[1..Lr] of a target of Ltarget residues.
 extern "C" int
 p7_gpu_RegionTraceEnsemble(const uint8_t *dsq, int Lr, int Ltarget, const P7_GPU_OPROFILE *om, int nsamples,
