@@ -236,15 +236,22 @@ void k_vit(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
             M[d] = adds2(max2(part[d], adds2(d ? D[d-1] : ds0, tDM[d])), e[d]);
             xE = max2(xE, M[d]);
           }
+          // M -> D scores that are not pinned come before the next row's odds:
+          // LDS answers in order
+          int md[PMDS ? 1 : ND];
+          if (! PMDS) {
+            const int *trr = tr + opaque_zero();
+#pragma unroll
+            for (int d = 0; d < ND; d++) md[d] = trr[VT_MDS*rowd + d*64];
+          }
           const int *en = tbl + rr.ahead(u) + z;
 #pragma unroll
           for (int d = 0; d < ND; d++) e[d] = en[d * 64];
-          const int *trr = tr + opaque_zero();
           const unsigned long long hit = __ballot(max2(xE, th2) != th2);
           nbM = dppi<WAVE_SHR1>(nbM, M[ND-1]);
           ms0 = (int) __builtin_amdgcn_alignbit((unsigned) M[ND-1], (unsigned) nbM, 16);
 #pragma unroll
-          for (int d = 0; d < ND; d++) D[d] = adds2(d ? M[d-1] : ms0, PMDS ? tMDS[d] : trr[VT_MDS*rowd + d*64]);
+          for (int d = 0; d < ND; d++) D[d] = adds2(d ? M[d-1] : ms0, PMDS ? tMDS[d] : md[d]);
           ahead();
           ds0 = dd_closure_max<ND>(D, ddc);
           if (__builtin_expect(hit != 0ull, 0)) {
