@@ -132,7 +132,7 @@ struct MdSig { int c, i, j, k, m; float prob; };
 // an LDS access. A later pass only adds its carries to the cells, which all lanes
 // do; and where every D->D odds is at most 1 a pass is left out whose first
 // carry is too small to change any cell, for then none of its carries does.
-// 60 regions of up to 600 residues: M = 86 0.50 ms, M = 400 2.6 ms; with every
+// Regions of up to 240 and 487 residues: M = 86 0.50 ms, M = 400 2.6 ms; with every
 // pass run in full by four lanes, cell by cell between LDS waits, 1.15 and 5.9 ms.
 // NU: models of up to 512 positions, NU cells per lane (c = 64 u + z), whose
 // transitions, places and odds are in registers; a step over them loads all
@@ -462,7 +462,7 @@ enum { MD_NAN_M = 5, MD_NAN_D = 6, MD_NAN_I = 7 };         // flag bits: the cel
 // left to k_md_replay, for which each run goes to the log: bits 0-6 the
 // repeats, 7-9 the state it leads to (0: the run goes on), 10 whether that I
 // or D state steps back to M at once; a domain starts with its last node and
-// state. 60 regions of up to 600 residues, walk + replay: M = 86 3.3 + 1.7 ms,
+// state. Regions of up to 240 and 487 residues, walk + replay: M = 86 3.1 + 1.7 ms,
 // M = 400 6.2 + 1.2 ms; with the steps' bookkeeping and the null2 sums of each
 // domain in the walk's chain, one wave a region, it was 9.1 and 13.7 ms.
 __global__ __launch_bounds__(64) void
@@ -557,9 +557,16 @@ k_md_walk(const DevProfile p, const MdJob *__restrict__ jobs, MdOut *__restrict_
           const int j = 64 * c + z, q = j >> 3;
           const float u = (j < 8 * Q) ? __fmul_rn(mat[((size_t) i * Q + q) * 12 + (j & 7)], nf) : 0.0f;
           double sum = c ? cp[c - 1] : 0.0;
-          for (int l = 0; l < 64; l++) {
-            sum = sum + (double) readlanef(u, l);
-            if (roll < sum) { found = 64 * c + l; break; }
+          // eight sums to a test (they do not fall: a roll under one of them is
+          // under the last, unless that is no number)
+          for (int l0 = 0; l0 < 64 && found < 0; l0 += 8) {
+            double s8[8];
+#pragma unroll
+            for (int l = 0; l < 8; l++) { sum = sum + (double) readlanef(u, l0 + l); s8[l] = sum; }
+            if (! (roll >= s8[7])) {
+#pragma unroll
+              for (int l = 7; l >= 0; l--) if (roll < s8[l]) found = 64 * c + l0 + l;
+            }
           }
         }
         if (found >= 0) {
