@@ -30,7 +30,6 @@ __device__ __forceinline__ int   pair16(int v) { return (int)(((unsigned)v & 0xf
 __device__ __forceinline__ int wave_shr1(int v, int fill) { return __builtin_amdgcn_update_dpp(fill, v, 0x138, 0xf, 0xf, false); }
 __device__ __forceinline__ int wave_shl1(int v, int fill) { return __builtin_amdgcn_update_dpp(fill, v, 0x130, 0xf, 0xf, false); }
 __device__ __forceinline__ int row_shr1(int v, int fill)  { return __builtin_amdgcn_update_dpp(fill, v, 0x111, 0xf, 0xf, false); }
-__device__ __forceinline__ float wave_shr1f(float v) { return __builtin_bit_cast(float, wave_shr1(__builtin_bit_cast(int, v), 0)); }
 __device__ __forceinline__ float wave_shl1f(float v) { return __builtin_bit_cast(float, wave_shl1(__builtin_bit_cast(int, v), 0)); }
 
 // Row shift of a packed block: the dword that becomes the new position pair 0.
@@ -170,18 +169,6 @@ struct ResAsc {                       // i = 0, 1, 2, ...
   __device__ __forceinline__ int at(int i)
   {
     if ((i >> 4) != c) { c = i >> 4; cur = uni4(nxt); nxt = p[c + 1]; }
-    return chunk_byte(cur, i);
-  }
-};
-struct ResDesc {                      // i = L-1, L-2, ..., 0
-  const uint4 *p; uint4 cur, nxt; int c;
-  __device__ __forceinline__ void init(const uint8_t *sq, int L)
-  {
-    p = (const uint4 *) sq; c = (L - 1) >> 4; cur = uni4(p[c]); nxt = p[c > 0 ? c - 1 : 0];
-  }
-  __device__ __forceinline__ int at(int i)
-  {
-    if ((i >> 4) != c) { c = i >> 4; cur = uni4(nxt); nxt = p[c > 0 ? c - 1 : 0]; }
     return chunk_byte(cur, i);
   }
 };

@@ -208,7 +208,6 @@ struct DomOut {
 #define MD_TSEG   512     // sampled domains in one trace
 #define MD_MAXSIG 64      // significant clusters of one region
 #define MD_MAXC   32      // envelopes one region may give
-#define MD_ACC_LDS 8192   // regions up to this many residues + 1 sum their odds, and keep their residues, in LDS
 __host__ __device__ inline int64_t md_q(int M) { return (M - 1) / 4 + 1 < 2 ? 2 : (M - 1) / 4 + 1; }
 // checkpoints per row of the E state's running sum over the 8Q M and D
 // cells (one at the end of every 64 of them, and the last)
@@ -342,7 +341,7 @@ hipError_t launch_ssv_chunked(const DevProfile &p, const DevSeqs &s, const int32
 // 1 if a kernel of this shape is built
 int ssv_shape_built(int G, int ND);
 int ssv_chunk_built(int ND);
-// launchers (p7g_kernels.hip)
+// launchers
 // p[0..nwords) = v, as a kernel (so that a captured graph holds no memset node)
 hipError_t launch_fill32(void *p, uint32_t v, int64_t nwords, hipStream_t st);
 // a single-target call's start and end (src, dst of 16-byte words; list null: no list)
