@@ -41,7 +41,7 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
     aff_bck_setup<B>(akc, tdd);
   }
 #define BTR(A, T, j) (PIN ? A[j] : trr[(T) * rowf + (j) * 64])
-  constexpr bool DOM = (MODE == 1), ENV = (MODE == 2), PF = (B <= 24);
+  constexpr bool DOM = (MODE == 1), ENV = (MODE == 2), STREAM = (TM == TM_GLOB), PF = ! STREAM;
   constexpr bool FI = (B == 1 || (B >= 6 && B <= 8)), FM = (B == 1 || (B >= 7 && B <= 8));
   const int64_t n = ENV ? min((int64_t) *count, dom.env_cap) : (int64_t) *count;
   const float eMove = ENV ? 1.0f : p.xfE_move, eLoop = ENV ? 0.0f : p.xfE_loop;
@@ -94,8 +94,8 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
     for (int j = 0; j < B; j++) { M[j] = xE; D[j] = xE; I[j] = 0.0f; }
     {
       const float *trr = tr + (PIN ? 0 : opaque_zero());
-      affine_bck_scan<B>(D, [&](int j) { return BTR(tDD, FT_DD, j); }, akc, z);
-      const float dS = wave_shl1f(D[0]);
+      affine_bck_scan<B>(D, [&](int j) { return BTR(tDD, FT_DD, j); }, akc);
+      const float dS = dppz<WAVE_SHL1>(D[0]);
 #pragma unroll
       for (int j = 0; j < B; j++) M[j] = M[j] + (j < B-1 ? D[j+1] : dS) * BTR(tMD, FT_MD, j);
     }
@@ -125,43 +125,66 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
     // leave 64 rows at a time. A row of one target alone, M = 20 | 86 | 400 |
     // 803: 190 | 218 | 320 | 497 ns (before 367 | 392 | 468 | 684 ns).
     float bE = 0.0f, bN = 0.0f, bJ = 0.0f, bB = 0.0f, bC = 0.0f, bS = 0.0f;
-    float e[PF ? B : 1];
+    float e[B];
     auto row = [&](int xoff, int xnext, float fs, int i, int u) {
       const float *er = tbl + xoff + z;
       const float *trr = tr + (PIN ? 0 : opaque_zero());
-#define EM(j) (PF ? e[PF ? (j) : 0] : er[(j) * 64])
-      // mn(j) = M(j) * e(j), formed one position ahead of the update that
-      // overwrites M(j); xBl sums mn(j) * tBM(j) in increasing j
-      float mn = M[0] * EM(0);
       float xBl = 0.0f;
-      xBl = __builtin_fmaf(mn, BTR(tBM, VT_BM, 0), xBl);
-      const float mS = wave_shl1f(mn);
+      if constexpr (STREAM) {
+        // M(j) * e(j), its share of the B sum, then the update
+        stream_tables<B, 2, 32, false>({ er, trr + VT_BM*rowf }, [&](int j, const float (&x)[2]) {
+          M[j] = M[j] * x[0];
+          xBl = __builtin_fmaf(M[j], x[1], xBl); });
+        const float mS = dppz<WAVE_SHL1>(M[0]);
+        stream_tables<B, 4, 16, false>({ trr + VT_II*rowf, trr + FT_IMN*rowf, trr + VT_MI*rowf, trr + FT_MMN*rowf },
+                                       [&](int j, const float (&x)[4]) {
+          const float ms = (j < B-1) ? M[j < B-1 ? j+1 : 0] : mS, ip = I[j];
+          I[j] = fma2<FI>(ip, x[0], ms, x[1]);
+          D[j] = ms;
+          M[j] = fma2<FM>(ip, x[2], ms, x[3]); });
+      } else {
+        // mn(j) = M(j) * e(j), formed one position ahead of the update that
+        // overwrites M(j); xBl sums mn(j) * tBM(j) in increasing j
+        const float mn = M[0] * e[0];
+        xBl = __builtin_fmaf(mn, BTR(tBM, VT_BM, 0), xBl);
+        const float mS = dppz<WAVE_SHL1>(mn);
 #pragma unroll
-      for (int j = 0; j < B; j++) {
-        float ms = mS;
-        if (j < B-1) { ms = M[j+1] * EM(j+1); xBl = __builtin_fmaf(ms, BTR(tBM, VT_BM, j+1), xBl); }
-        const float ip = I[j];
-        I[j] = fma2<FI>(ip, BTR(tII, VT_II, j), ms, BTR(tIMN, FT_IMN, j));
-        D[j] = ms;
-        M[j] = fma2<FM>(ip, BTR(tMI, VT_MI, j), ms, BTR(tMMN, FT_MMN, j));
-      }
-#undef EM
-      if (PF) {
+        for (int j = 0; j < B; j++) {
+          float ms = mS;
+          if (j < B-1) { ms = M[j+1] * e[j+1]; xBl = __builtin_fmaf(ms, BTR(tBM, VT_BM, j+1), xBl); }
+          const float ip = I[j];
+          I[j] = fma2<FI>(ip, BTR(tII, VT_II, j), ms, BTR(tIMN, FT_IMN, j));
+          D[j] = ms;
+          M[j] = fma2<FM>(ip, BTR(tMI, VT_MI, j), ms, BTR(tMMN, FT_MMN, j));
+        }
         const float *el = tbl + xnext + z;
 #pragma unroll
-        for (int j = 0; j < (PF ? B : 1); j++) e[j] = el[j * 64];
+        for (int j = 0; j < B; j++) e[j] = el[j * 64];
       }
       xB = wave_sum_f(xBl);
       xC = xC * floop;
       xJ = fma2<true>(xB, fmove, xJ, floop);
       xN = fma2<true>(xB, fmove, xN, floop);
       xE = fma2<false>(xC, eMove, xJ, eLoop);
+      if constexpr (STREAM) {
+        float C = 0.0f, mdl = 0.0f;
+        stream_tables<B, 2, 32, true>({ trr + FT_DMN*rowf, trr + FT_DD*rowf }, [&](int j, const float (&x)[2]) {
+          D[j] = __builtin_fmaf(D[j], x[0], xE);
+          C = (j == B-1) ? D[j] : __builtin_fmaf(x[1], C, D[j]); });
+        float cur = lane_carry_bck(C, akc);
+        stream_tables<B, 2, 32, true>({ trr + FT_DD*rowf, trr + FT_MD*rowf }, [&](int j, const float (&x)[2]) {
+          if (j < B-1) M[j] = __builtin_fmaf(D[j < B-1 ? j+1 : 0], x[1], M[j] + xE);
+          else mdl = x[1];
+          D[j] = cur = __builtin_fmaf(x[0], cur, D[j]); });
+        M[B-1] = __builtin_fmaf(dppz<WAVE_SHL1>(D[0]), mdl, M[B-1] + xE);
+      } else {
 #pragma unroll
-      for (int j = 0; j < B; j++) D[j] = __builtin_fmaf(D[j], BTR(tDMN, FT_DMN, j), xE);
-      affine_bck_scan<B>(D, [&](int j) { return BTR(tDD, FT_DD, j); }, akc, z);
-      const float dS = wave_shl1f(D[0]);
+        for (int j = 0; j < B; j++) D[j] = __builtin_fmaf(D[j], BTR(tDMN, FT_DMN, j), xE);
+        affine_bck_scan<B>(D, [&](int j) { return BTR(tDD, FT_DD, j); }, akc);
+        const float dS = dppz<WAVE_SHL1>(D[0]);
 #pragma unroll
-      for (int j = 0; j < B; j++) M[j] = __builtin_fmaf(j < B-1 ? D[j+1] : dS, BTR(tMD, FT_MD, j), M[j] + xE);
+        for (int j = 0; j < B; j++) M[j] = __builtin_fmaf(j < B-1 ? D[j+1] : dS, BTR(tMD, FT_MD, j), M[j] + xE);
+      }
       const int xBbits = uni(__float_as_int(xB));
       if (gt_bits(xBbits, BITS_1E16)) own = 1;
       if (__builtin_expect(own, 0)) fs = (xB > 1.0e4f) ? xB : 1.0f;
@@ -190,7 +213,7 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
       xoff = rr.init(sq, L, z, (int) rowf);
       if (PF) {
 #pragma unroll
-        for (int j = 0; j < (PF ? B : 1); j++) e[j] = tbl[xoff + z + j * 64];
+        for (int j = 0; j < B; j++) e[j] = tbl[xoff + z + j * 64];
       }
       // Forward's scale factors of the block's rows: lane u holds row L-1-s0-u's
       auto scales = [&](int s0) { return fsc[(size_t) max(L - 1 - s0 - z, 0) * fstride]; };
@@ -243,24 +266,6 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
 // every wave updates the special states by itself.
 // Bound by the row's chain of dependent steps; M = 2600 (B = 48, W = 4): 760 ns
 // a row, where four barriers and odds loaded in the row made it 1250 ns.
-__device__ __forceinline__ float lane_carry_bck(float C, const AffConst &k, int z)
-{
-  // C: the lane's map constant (carry-in 0 from the right); returns D at the
-  // first position of lane z+1
-  C = C + k.w1 * dppz<ROW_SHL1>(C);
-  C = C + k.w2 * dppz<ROW_SHL2>(C);
-  C = C + k.w4 * dppz<ROW_SHL4>(C);
-  C = C + k.w8 * dppz<ROW_SHL8>(C);
-  {
-    const float c2 = readlanef(C, 48);
-    const float c1 = k.pa * c2 + readlanef(C, 32);
-    const float c0 = k.pb * c1 + readlanef(C, 16);
-    const float rc = lane_sel(lane_sel(lane_sel(0.0f, c2, LANES_ROW(2)), c1, LANES_ROW(1)), c0, LANES_ROW(0));
-    C = C + k.prow * rc;
-  }
-  return dppz<WAVE_SHL1>(C);
-}
-
 __device__ __forceinline__ void aff_setup_lane_bck(AffConst &k, float P)
 {
   k.w1 = P; P = P * dppf<ROW_SHL1>(1.0f, P);
@@ -338,7 +343,7 @@ void k_bck_wg(const DevProfile p, const uint8_t *__restrict__ res, const int64_t
     float Cl = 0.0f;
 #pragma unroll
     for (int v = W-1; v >= 0; v--) Cl = __builtin_fmaf(Pv[v], Cl, cv[v]);
-    float c = lane_carry_bck(Cl, akl, z);
+    float c = lane_carry_bck(Cl, akl);
 #pragma unroll
     for (int v = W-1; v > 0; v--) if (v > wv) c = __builtin_fmaf(Pv[v], c, cv[v]);
     float cur = c;

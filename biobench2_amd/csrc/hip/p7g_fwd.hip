@@ -243,6 +243,10 @@ __device__ __forceinline__ void oa_row(const DevProfile &p, int z, int i,
 #undef OTR
 }
 
+// The null2 pass (MODE 3) runs in workgroups of four waves, one per SIMD, whose
+// waves may hold 512 registers; with 256 the rows of B > 12 spilled up to 1100
+// of them (null2 pass of M = 1500 | 2600: 34 | 215 ms, now 15 | 140 ms).
+#define NULL2_THREADS 256
 // MODE 0: the parser. MODE 1: the special-state rows also go to the caller's
 // matrix (one target) or to the domain decoding pool (a separate instance, so
 // that the plain parser keeps its register budget).
@@ -255,7 +259,7 @@ __device__ __forceinline__ void oa_row(const DevProfile &p, int z, int i,
 // (p7_Null2_ByExpectation, impl_sse/null2.c:59-118) and the envelope's
 // correction sum_pos logf(null2[x_pos]) (p7_domaindef.c:925-931).
 template <int B, int TM, int MODE>
-__global__ __launch_bounds__(FWD_THREADS(B))
+__global__ __launch_bounds__(MODE == 3 && B > 12 ? NULL2_THREADS : FWD_THREADS(B))
 void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *__restrict__ off,
            const int32_t *__restrict__ len, const int32_t *__restrict__ list, const int32_t *__restrict__ count,
            DevResults r, DevLists l, GateThresh g, int gating, LenCfg lc,
@@ -283,9 +287,9 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
   // PF: a row's emission odds are loaded a row ahead (not where the positions
   // of a large model, or the alignment's state, already fill the registers).
   // PIND: the D->D odds are pinned too.
-  constexpr bool FI = false, FP = (B == 1 && MODE != 3);
+  constexpr bool FP = (B == 1 && MODE != 3);
   constexpr int EG = (MODE == 3) ? 8 : 16;
-  constexpr bool PF = (MODE != 3 && B <= 28), PIND = (PIN && MODE != 3 && B <= 4);
+  constexpr bool STREAM = (TM == TM_GLOB && MODE != 3), PF = (MODE != 3 && B <= 28), PIND = (PIN && MODE != 3 && B <= 4);
   AffConst akc;
   float tDDP[B];
 #pragma unroll
@@ -408,39 +412,56 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
 #define FTR(A, T, j) (PIN ? A[j] : trr[(T) * rowf + (j) * 64])
       const float iL = dppz<WAVE_SHR1>(I[B-1]), dL = dppz<WAVE_SHR1>(D[B-1]);
       float xEl = 0.0f;
-      float eg[EG];                              // without PF the odds come EG positions at a time
-#pragma unroll
-      for (int j = B-1; j >= 0; j--) {
-        const float mp = j ? M[j-1] : mL, ip = j ? I[j-1] : iL, dp = j ? D[j-1] : dL;
-        const float In = fma2<FI>(M[j], FTR(tMI, VT_MI, j), I[j], FTR(tII, VT_II, j));
-        float sv = fma2<FP>(xB, FTR(tBM, VT_BM, j), mp, FTR(tMM, VT_MM, j));
-        sv = __builtin_fmaf(ip, FTR(tIM, VT_IM, j), sv);
-        sv = __builtin_fmaf(dp, FTR(tDM, VT_DM, j), sv);
-        if (! PF && (B - 1 - j) % EG == 0) {
-#pragma unroll
-          for (int v = 0; v < EG; v++) if (j - v >= 0) eg[v] = er[(j - v) * 64];
-        }
-        const float ej = PF ? e[PF ? j : 0] : eg[(B - 1 - j) % EG];
+      auto cell = [&](int j, float ej, float bm, float mm, float im, float dm, float mi, float ii) {
+        const float mp = j ? M[j ? j-1 : 0] : mL, ip = j ? I[j ? j-1 : 0] : iL, dp = j ? D[j ? j-1 : 0] : dL;
+        const float In = fma2<false>(M[j], mi, I[j], ii);
+        float sv = fma2<FP>(xB, bm, mp, mm);
+        sv = __builtin_fmaf(ip, im, sv);
+        sv = __builtin_fmaf(dp, dm, sv);
         M[j] = sv * ej; I[j] = In;
-        xEl = __builtin_fmaf(sv, ej, xEl);
-      }
-      if (PF) {
-        const float *el = tbl + xnext + z;
+        xEl = (B > 1 && j == B-1) ? M[j] : __builtin_fmaf(sv, ej, xEl);   // B = 1: no product left to fuse with D
+      };
+      if constexpr (STREAM) {
+        stream_tables<B, 7, 8, true>({ er, trr + VT_BM*rowf, trr + VT_MM*rowf, trr + VT_IM*rowf, trr + VT_DM*rowf,
+                                        trr + VT_MI*rowf, trr + VT_II*rowf },
+                                      [&](int j, const float (&x)[7]) { cell(j, x[0], x[1], x[2], x[3], x[4], x[5], x[6]); });
+        mL = dppz<WAVE_SHR1>(M[B-1]);
+        float C = 0.0f;
+        stream_tables<B, 2, 32, false>({ trr + VT_MDS*rowf, trr + VT_DDS*rowf }, [&](int j, const float (&x)[2]) {
+          D[j] = (j ? M[j ? j-1 : 0] : mL) * x[0];
+          C = j ? __builtin_fmaf(x[1], C, D[j]) : D[j]; });
+        float cur = lane_carry_fwd(C, akc);
+        stream_tables<B, 1, 32, false>({ trr + VT_DDS*rowf }, [&](int j, const float (&x)[1]) {
+          D[j] = cur = __builtin_fmaf(x[0], cur, D[j]); });
+      } else {
+        float eg[EG];                            // without PF the odds come EG positions at a time
 #pragma unroll
-        for (int j = 0; j < (PF ? B : 1); j++) e[j] = el[j * 64];
-      }
-      const float mS = dppz<WAVE_SHR1>(M[B-1]);
+        for (int j = B-1; j >= 0; j--) {
+          if (! PF && (B - 1 - j) % EG == 0) {
 #pragma unroll
-      for (int j = 0; j < B; j++) D[j] = (j ? M[j-1] : mS) * FTR(tMDS, VT_MDS, j);
+            for (int v = 0; v < EG; v++) if (j - v >= 0) eg[v] = er[(j - v) * 64];
+          }
+          cell(j, PF ? e[PF ? j : 0] : eg[(B - 1 - j) % EG], FTR(tBM, VT_BM, j), FTR(tMM, VT_MM, j), FTR(tIM, VT_IM, j),
+               FTR(tDM, VT_DM, j), FTR(tMI, VT_MI, j), FTR(tII, VT_II, j));
+        }
+        if (PF) {
+          const float *el = tbl + xnext + z;
+#pragma unroll
+          for (int j = 0; j < (PF ? B : 1); j++) e[j] = el[j * 64];
+        }
+        mL = dppz<WAVE_SHR1>(M[B-1]);
+#pragma unroll
+        for (int j = 0; j < B; j++) D[j] = (j ? M[j-1] : mL) * FTR(tMDS, VT_MDS, j);
 #undef FTR
-      if (PIND) affine_fwd_scan<B>(D, tDDP, akc, z);
-      else {
-        // the D->D odds are read per row, not pinned in registers: this keeps
-        // the kernel at 128 VGPRs, four waves per SIMD
-        float tDDS[B];
+        if (PIND) affine_fwd_scan<B>(D, tDDP, akc);
+        else {
+          // the D->D odds are read per row, not pinned in registers: this keeps
+          // the kernel at 128 VGPRs, four waves per SIMD
+          float tDDS[B];
 #pragma unroll
-        for (int j = 0; j < B; j++) tDDS[j] = trr[VT_DDS*rowf + j*64];
-        affine_fwd_scan<B>(D, tDDS, akc, z);
+          for (int j = 0; j < B; j++) tDDS[j] = trr[VT_DDS*rowf + j*64];
+          affine_fwd_scan<B>(D, tDDS, akc);
+        }
       }
 #pragma unroll
       for (int j = 0; j < B; j++) xEl += D[j];
@@ -455,6 +476,7 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
         const float inv = (float) (1.0 / (double) xE);
 #pragma unroll
         for (int j = 0; j < B; j++) { M[j] *= inv; D[j] *= inv; I[j] *= inv; }
+        mL *= inv;
         scale = xE;
         sbuf = (z == u) ? xE : sbuf;
         totscale = (float) ((double) totscale + log((double) xE));
@@ -470,7 +492,6 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
           }
         }
       }
-      mL = dppz<WAVE_SHR1>(M[B-1]);
       if (DOM) {
         const bool me = (z == u);
         bE = me ? xE : bE; bN = me ? xN : bN; bJ = me ? xJ : bJ; bB = me ? xB : bB; bC = me ? xC : bC;
@@ -565,24 +586,6 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
 // wave updates the special states and rescales by itself, from the same sum.
 // Bound by the row's chain of dependent steps; M = 2600 (B = 48, W = 4): 820 ns
 // a row, where four barriers and odds loaded in the row made it 1083 ns.
-template <int B>
-__device__ __forceinline__ float lane_carry_fwd(float C, const AffConst &k, int z)
-{
-  // C: the lane's map constant (carry-in 0); returns D at the end of lane z-1
-  C = C + k.w1 * dppz<ROW_SHR1>(C);
-  C = C + k.w2 * dppz<ROW_SHR2>(C);
-  C = C + k.w4 * dppz<ROW_SHR4>(C);
-  C = C + k.w8 * dppz<ROW_SHR8>(C);
-  {
-    const float c1 = readlanef(C, 15);
-    const float c2 = k.pa * c1 + readlanef(C, 31);
-    const float c3 = k.pb * c2 + readlanef(C, 47);
-    const float rc = lane_sel(lane_sel(lane_sel(0.0f, c1, LANES_ROW(1)), c2, LANES_ROW(2)), c3, LANES_ROW(3));
-    C = C + k.prow * rc;
-  }
-  return dppz<WAVE_SHR1>(C);
-}
-
 __device__ __forceinline__ void aff_setup_lane(AffConst &k, float P)
 {
   k.w1 = P; P = P * dppf<ROW_SHR1>(1.0f, P);
@@ -730,7 +733,7 @@ void k_fwd_wg(const DevProfile p, const uint8_t *__restrict__ res, const int64_t
             float Cl = 0.0f;
 #pragma unroll
             for (int v = 0; v < W; v++) Cl = __builtin_fmaf(Pv[v], Cl, cv[v]);
-            float c = lane_carry_fwd<B>(Cl, akl, z);
+            float c = lane_carry_fwd(Cl, akl);
 #pragma unroll
             for (int v = 0; v < W - 1; v++) if (v < wv) c = __builtin_fmaf(Pv[v], c, cv[v]);
             float cur = c;
@@ -843,7 +846,7 @@ hipError_t launch_fwd(const DevProfile &p, const DevSeqs &s, const int32_t *list
   }
   // the null2 pass in workgroups of four waves (one per SIMD), so that one of
   // them fits on a compute unit beside a multidomain region's wave
-  if (dom.env_loop && dom.n2mode == 2) nthr = std::min(nthr, 256);
+  if (dom.env_loop && dom.n2mode == 2) nthr = std::min(nthr, NULL2_THREADS);
   const size_t lds = fb_lds(p, tm);
   const unsigned grid = list_grid(k, maxn, lds, nthr / 64);
   void *args[] = { (void *) &p, (void *) &s.res, (void *) &s.off, (void *) &s.len, (void *) &list, (void *) &count,

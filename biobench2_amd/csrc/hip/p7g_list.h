@@ -157,13 +157,10 @@ __device__ __forceinline__ void aff_bck_setup(AffConst &k, const float (&a)[B])
   k.prow = P; k.pa = readlanef(P, 32); k.pb = readlanef(P, 16);
 }
 
-template <int B>
-__device__ __forceinline__ void affine_fwd_scan(float (&D)[B], const float (&a)[B], const AffConst &k, int z)
+// C: the lane's map constant (carry-in 0); returns D at the end of lane z-1,
+// resp. (towards smaller k) at the first position of lane z+1.
+__device__ __forceinline__ float lane_carry_fwd(float C, const AffConst &k)
 {
-  // D(j) = D0(j) + a(j) * D(j-1), carried across lanes in increasing k
-  float C = 0.0f;
-#pragma unroll
-  for (int j = 0; j < B; j++) C = D[j] + a[j] * C;
   C = C + k.w1 * dppz<ROW_SHR1>(C);
   C = C + k.w2 * dppz<ROW_SHR2>(C);
   C = C + k.w4 * dppz<ROW_SHR4>(C);
@@ -175,21 +172,11 @@ __device__ __forceinline__ void affine_fwd_scan(float (&D)[B], const float (&a)[
     const float rc = lane_sel(lane_sel(lane_sel(0.0f, c1, LANES_ROW(1)), c2, LANES_ROW(2)), c3, LANES_ROW(3));
     C = C + k.prow * rc;
   }
-  const float cin = dppz<WAVE_SHR1>(C);
-  float cur = cin;
-#pragma unroll
-  for (int j = 0; j < B; j++) { cur = D[j] + a[j] * cur; D[j] = cur; }
+  return dppz<WAVE_SHR1>(C);
 }
 
-// a(j) gives the D->D odds of the lane's position j (read twice per call, so
-// that large models need not hold them in registers through the scan).
-template <int B, typename A>
-__device__ __forceinline__ void affine_bck_scan(float (&D)[B], A a, const AffConst &k, int z)
+__device__ __forceinline__ float lane_carry_bck(float C, const AffConst &k)
 {
-  // D(j) = c(j) + a(j) * D(j+1), carried across lanes in decreasing k
-  float C = 0.0f;
-#pragma unroll
-  for (int j = B-1; j >= 0; j--) C = D[j] + a(j) * C;
   C = C + k.w1 * dppz<ROW_SHL1>(C);
   C = C + k.w2 * dppz<ROW_SHL2>(C);
   C = C + k.w4 * dppz<ROW_SHL4>(C);
@@ -201,10 +188,67 @@ __device__ __forceinline__ void affine_bck_scan(float (&D)[B], A a, const AffCon
     const float rc = lane_sel(lane_sel(lane_sel(0.0f, c2, LANES_ROW(2)), c1, LANES_ROW(1)), c0, LANES_ROW(0));
     C = C + k.prow * rc;
   }
-  const float cin = dppz<WAVE_SHL1>(C);
-  float cur = cin;
+  return dppz<WAVE_SHL1>(C);
+}
+
+template <int B>
+__device__ __forceinline__ void affine_fwd_scan(float (&D)[B], const float (&a)[B], const AffConst &k)
+{
+  // D(j) = D0(j) + a(j) * D(j-1), carried across lanes in increasing k
+  float C = 0.0f;
+#pragma unroll
+  for (int j = 0; j < B; j++) C = D[j] + a[j] * C;
+  float cur = lane_carry_fwd(C, k);
+#pragma unroll
+  for (int j = 0; j < B; j++) { cur = D[j] + a[j] * cur; D[j] = cur; }
+}
+
+// a(j) gives the D->D odds of the lane's position j (read twice per call, so
+// that large models need not hold them in registers through the scan).
+template <int B, typename A>
+__device__ __forceinline__ void affine_bck_scan(float (&D)[B], A a, const AffConst &k)
+{
+  // D(j) = c(j) + a(j) * D(j+1), carried across lanes in decreasing k
+  float C = 0.0f;
+#pragma unroll
+  for (int j = B-1; j >= 0; j--) C = D[j] + a(j) * C;
+  float cur = lane_carry_bck(C, k);
 #pragma unroll
   for (int j = B-1; j >= 0; j--) { cur = D[j] + a(j) * cur; D[j] = cur; }
+}
+
+// The values of NT tables at a lane's B positions, read from memory where a row
+// needs them (DESC: from the last position down), for models too large to hold
+// or stage them: G positions at a time, the next group requested before this
+// one is used. Bound by the latency of these loads: left to itself the compiler
+// loads one position's values, waits and goes on. Decoding of 40 targets of
+// M = 3500: Forward 18.9 ms, Backward 19.0 ms; position by position 70 and 120 ms.
+template <int B, int NT, int G, bool DESC, typename F>
+__device__ __forceinline__ void stream_tables(const float *const (&src)[NT], F f)
+{
+  constexpr int NG = (B + G - 1) / G;
+  float v[2][NT][G];
+  auto load = [&](int g) {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int u = 0; u < G; u++)
+        if (g * G + u < B) v[g & 1][t][u] = src[t][(DESC ? B - 1 - (g * G + u) : g * G + u) * 64];
+  };
+  load(0);
+#pragma unroll
+  for (int g = 0; g < NG; g++) {
+    if (g + 1 < NG) load(g + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < G; u++)
+      if (g * G + u < B) {
+        float x[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) x[t] = v[g & 1][t][u];
+        f(DESC ? B - 1 - (g * G + u) : g * G + u, x);
+      }
+  }
 }
 
 // Forward/Backward: the whole table in LDS up to B = 12 (150 KB); B = 14 reads
