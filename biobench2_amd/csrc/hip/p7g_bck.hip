@@ -8,8 +8,9 @@
 // MODE 0: the parser. MODE 1: the special-state rows also go to the caller's
 // matrix (one target) or to the domain decoding pool (a separate instance, so
 // that the plain parser keeps its register budget). MODE 2: envelopes.
+// At B <= 2 six waves per SIMD (80 registers) leave room for a third workgroup.
 template <int B, int TM, int MODE>
-__global__ __launch_bounds__(BCK_THREADS(B)) __attribute__((amdgpu_waves_per_eu((B) <= 7 ? 4 : 1)))
+__global__ __launch_bounds__(BCK_THREADS(B)) __attribute__((amdgpu_waves_per_eu((B) <= 2 ? 6 : (B) <= 7 ? 4 : 1)))
 void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *__restrict__ off,
            const int32_t *__restrict__ len, const int32_t *__restrict__ list, const int32_t *__restrict__ count,
            DevResults r, const float *__restrict__ pool, const int64_t *__restrict__ scale_off,
@@ -126,7 +127,7 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
     // 803: 190 | 218 | 320 | 497 ns (before 367 | 392 | 468 | 684 ns).
     float bE = 0.0f, bN = 0.0f, bJ = 0.0f, bB = 0.0f, bC = 0.0f, bS = 0.0f;
     float e[B];
-    auto row = [&](int xoff, int xnext, float fs, int i, int u) {
+    auto row = [&](int xoff, int xnext, int fsbits, int i, int u) {
       const float *er = tbl + xoff + z;
       const float *trr = tr + (PIN ? 0 : opaque_zero());
       float xBl = 0.0f;
@@ -153,9 +154,10 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
           float ms = mS;
           if (j < B-1) { ms = M[j+1] * e[j+1]; xBl = __builtin_fmaf(ms, BTR(tBM, VT_BM, j+1), xBl); }
           const float ip = I[j];
-          I[j] = fma2<FI>(ip, BTR(tII, VT_II, j), ms, BTR(tIMN, FT_IMN, j));
+          M[j] = fma2<FM>(ip, BTR(tMI, VT_MI, j), ms, BTR(tMMN, FT_MMN, j));   // before I: ip in place, no copy
+          if (FI || ! PIN) I[j] = fma2<FI>(ip, BTR(tII, VT_II, j), ms, BTR(tIMN, FT_IMN, j));
+          else fma_onto(I[j], BTR(tII, VT_II, j), ms * BTR(tIMN, FT_IMN, j));
           D[j] = ms;
-          M[j] = fma2<FM>(ip, BTR(tMI, VT_MI, j), ms, BTR(tMMN, FT_MMN, j));
         }
         const float *el = tbl + xnext + z;
 #pragma unroll
@@ -185,16 +187,18 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
 #pragma unroll
         for (int j = 0; j < B; j++) M[j] = __builtin_fmaf(j < B-1 ? D[j+1] : dS, BTR(tMD, FT_MD, j), M[j] + xE);
       }
+      // the row's scale: Forward's, or its own; bits in scalar registers
       const int xBbits = uni(__float_as_int(xB));
       if (gt_bits(xBbits, BITS_1E16)) own = 1;
-      if (__builtin_expect(own, 0)) fs = (xB > 1.0e4f) ? xB : 1.0f;
-      if (gt_bits(uni(__float_as_int(fs)), BITS_ONE)) {
+      if (own) fsbits = gt_bits(xBbits, BITS_1E4) ? xBbits : BITS_ONE;
+      const float fs = __int_as_float(fsbits);
+      if (gt_bits(fsbits, BITS_ONE)) {
         const float s = fs;
         xE /= s; xN /= s; xJ /= s; xB /= s; xC /= s;
         const float inv = (float) (1.0 / (double) s);
 #pragma unroll
         for (int j = 0; j < B; j++) { M[j] *= inv; D[j] *= inv; I[j] *= inv; }
-        totscale = (float) ((double) totscale + log((double) s));
+        if (MODE == 0) bS = (z == u) ? s : bS;
       }
       if (MODE != 0) {
         const bool me = (z == u);
@@ -219,12 +223,14 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
       auto scales = [&](int s0) { return fsc[(size_t) max(L - 1 - s0 - z, 0) * fstride]; };
       float sc0 = scales(0), sc1 = scales(64);
       for (int s0 = 0; s0 < L - 1; s0 += 64) {
-        const int cnt = min(64, L - 1 - s0), i0 = L - 1 - s0;
+        const int cnt = uni(min(64, L - 1 - s0)), i0 = L - 1 - s0;
+        bS = 1.0f;
         for (int u = 0; u < cnt; u++) {
           const int xnext = rr.ahead(u);
-          row(xoff, xnext, readlanef(sc0, u), i0 - u, u);
+          row(xoff, xnext, __builtin_amdgcn_readlane(__float_as_int(sc0), u), i0 - u, u);
           xoff = xnext;
         }
+        add_scales(totscale, bS);
         if (MODE != 0 && xo && z < cnt) {
           float *xr = xo + (size_t) (i0 - z) * 6;
           xr[0] = bE; xr[1] = bN; xr[2] = bJ; xr[3] = bB; xr[4] = bC; xr[5] = bS;

@@ -53,6 +53,24 @@ __device__ __forceinline__ bool gt_bits(int xbits, int limbits)
 #define BITS_1E16 0x5a0e1bca      // 1.0e16f
 #define BITS_ONE  0x3f800000      // 1.0f
 
+// Adds the logs of a block's row scales (lane u: row u's, 1 where the row was not
+// rescaled) to totscale in row order. Once per 64 rows: with its logarithm in
+// the row loop a parser held some twenty registers less for its rows (Backward's
+// B = 5..7 spilled up to 23 of them, and B = 2 had five waves per SIMD for six).
+__device__ __forceinline__ void add_scales(float &totscale, float s)
+{
+  unsigned long long m = __ballot(s > 1.0f);
+  if (__builtin_expect(m != 0ull, 0)) {
+    const double lg = log((double) s);
+    const int lo = (int) __double2loint(lg), hi = (int) __double2hiint(lg);
+    do {
+      const int l = (int) __ffsll((long long) m) - 1;
+      totscale = (float) ((double) totscale + __hiloint2double(__builtin_amdgcn_readlane(hi, l), __builtin_amdgcn_readlane(lo, l)));
+      m &= m - 1;
+    } while (m);
+  }
+}
+
 // A workgroup barrier that orders LDS alone: global loads in flight (the next
 // row's odds) stay in flight, where __syncthreads would wait for them.
 __device__ __forceinline__ void lds_barrier()
@@ -107,6 +125,15 @@ __device__ __forceinline__ float fma2(float a, float b, float c, float d)
 {
 #pragma clang fp contract(off)
   return SW ? __builtin_fmaf(c, d, a * b) : __builtin_fmaf(a, b, c * d);
+}
+
+// x = x * a + t, fused, in x's own register: left to itself the compiler adds onto
+// t's and copies the sum back at the end of the row. What is left of t keeps it
+// from that.
+__device__ __forceinline__ void fma_onto(float &x, float a, float t)
+{
+  x = __builtin_fmaf(x, a, t);
+  asm("" :: "v"(t));
 }
 
 // v where the lane's bit of a constant mask is set, else w: one v_cndmask. The
@@ -195,9 +222,9 @@ template <int B>
 __device__ __forceinline__ void affine_fwd_scan(float (&D)[B], const float (&a)[B], const AffConst &k)
 {
   // D(j) = D0(j) + a(j) * D(j-1), carried across lanes in increasing k
-  float C = 0.0f;
+  float C = D[0];
 #pragma unroll
-  for (int j = 0; j < B; j++) C = D[j] + a[j] * C;
+  for (int j = 1; j < B; j++) C = D[j] + a[j] * C;
   float cur = lane_carry_fwd(C, k);
 #pragma unroll
   for (int j = 0; j < B; j++) { cur = D[j] + a[j] * cur; D[j] = cur; }
@@ -209,9 +236,9 @@ template <int B, typename A>
 __device__ __forceinline__ void affine_bck_scan(float (&D)[B], A a, const AffConst &k)
 {
   // D(j) = c(j) + a(j) * D(j+1), carried across lanes in decreasing k
-  float C = 0.0f;
+  float C = D[B-1];
 #pragma unroll
-  for (int j = B-1; j >= 0; j--) C = D[j] + a(j) * C;
+  for (int j = B-2; j >= 0; j--) C = D[j] + a(j) * C;
   float cur = lane_carry_bck(C, k);
 #pragma unroll
   for (int j = B-1; j >= 0; j--) { cur = D[j] + a(j) * cur; D[j] = cur; }

@@ -56,6 +56,39 @@ def test_parser_rows_at_block_edges(gpu, tmp_path, M):
             np.testing.assert_allclose(got[:, :5], ref[:, :5], rtol=2e-4, atol=1e-30)
 
 
+@pytest.mark.parametrize("M", [64, 86, 250, 448, 512])
+@pytest.mark.parametrize("own", [False, True])
+def test_row_scales_across_blocks(gpu, tmp_path, M, own):
+    """Targets of several homologs, whose rows rescale many times over the blocks of 64: the
+    scales' logs add up in row order. own: Backward is given a Forward matrix without scales
+    and goes over to its own from the first row above 1e16. Scores: half a unit in the last
+    place of the score per scale added, or 1e-4; scales as the special rows above."""
+    rng = np.random.default_rng([15, M])
+    h = synth.random_profile(M, rng, f"scales_M{M}")
+    h.stats = (-9.0, 0.6931, -9.5, 0.6931, -5.0, 0.6931)
+    path = str(tmp_path / "scales.hmm")
+    synth.write_hmm(path, [h])
+    om = gpu.OProfile.from_file(path)
+    cores = synth.emit_homologs(synth.read_hmm_probs(path), 6 + 600 // M, rng)
+    s = np.concatenate([x for c in cores for x in (c, random_seqs(rng, [7])[0])])
+    om.reconfig_length(len(s))
+    t = om.tables()
+    st, sc, xmx, _ = oracle.fwd_parser(s, t)
+    st1, one, fwd = gpu.forward_parser(s, om)
+    n = int((xmx[:, 5] > 1).sum())
+    tol = max(1e-4, n * 2.0 ** -24 * abs(sc))
+    assert st == st1 == 0 and n >= 6 and abs(one - sc) <= tol
+    np.testing.assert_allclose(fwd.xmx()[0][:, 5], xmx[:, 5], rtol=2e-4)
+    if own:
+        xmx[:, 5] = 1.0
+        p = p7gpu.lib.p7_gpu_omx_Xmx(fwd.h, None, None, None)
+        np.ctypeslib.as_array(p, ((len(s) + 1) * 6,))[5::6] = 1.0
+    st2, sc2, bxmx, bown = oracle.bck_parser(s, t, xmx)
+    st3, one2, bck = gpu.backward_parser(s, om, fwd)
+    assert st2 == st3 == 0 and abs(one2 - sc2) <= tol and bool(bown) == own
+    np.testing.assert_allclose(bck.xmx()[0][:, 5], bxmx[:, 5], rtol=2e-4)
+
+
 @pytest.mark.parametrize("M", [1, 2, 127, 128, 129, 257, 640, 1023, 1281, 1535, 1536, 2046, 2047, 2559, 3071, 4095])
 @pytest.mark.parametrize("tables", ["converted", "lazy", "loops"])
 def test_viterbi_rows_bit_exact(gpu, tmp_path, M, tables):
