@@ -349,7 +349,7 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
       opp   = (uint8_t *) (area + n2_pp_at(L, B));
       if (z == 0) orow[0] = 1u << OA_BBIT;        // B(0) comes from N(0)
     }
-    if (pool) {
+    if (MODE != 3 && pool) {
       unsigned long long a64 = 0;
       if (z == 0) a64 = atomicAdd(l.cursor, (unsigned long long) (L + 1));
       const int64_t at = ((int64_t) (unsigned) uni((int) (a64 >> 32)) << 32) | (unsigned) uni((int) a64);
@@ -390,7 +390,7 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
     float bE = 0.0f, bN = 0.0f, bJ = 0.0f, bB = 0.0f, bC = 0.0f;
     float e[PF ? B : 1];
     auto row = [&](int xoff, int xnext, int i, int u) {
-      const float *er = tbl + xoff + z;
+      const float *er = (const float *) ((const char *) tbl + xoff) + z;
       const float *trr = tr + (PIN ? 0 : opaque_zero());
       const float pxN = xN, pxJ = xJ, pxC = xC;          // row i-1
       // null2 (MODE 3): Backward's specials and, for up to eight positions
@@ -445,7 +445,7 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
                FTR(tDM, VT_DM, j), FTR(tMI, VT_MI, j), FTR(tII, VT_II, j));
         }
         if (PF) {
-          const float *el = tbl + xnext + z;
+          const float *el = (const float *) ((const char *) tbl + xnext) + z;
 #pragma unroll
           for (int j = 0; j < (PF ? B : 1); j++) e[j] = el[j * 64];
         }
@@ -467,8 +467,8 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
       for (int j = 0; j < B; j++) xEl += D[j];
       xE = wave_sum_f(xEl);
       xN = xN * floop;
-      xC = fma2<false>(xC, floop, xE, eMove);
-      xJ = fma2<false>(xJ, floop, xE, eLoop);
+      fma_onto(xC, floop, xE * eMove);
+      fma_onto(xJ, floop, xE * eLoop);
       xB = fma2<true>(xJ, fmove, xN, fmove);
       float scale = 1.0f;
       if (gt_bits(uni(__float_as_int(xE)), BITS_1E4)) {
@@ -478,8 +478,10 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
         for (int j = 0; j < B; j++) { M[j] *= inv; D[j] *= inv; I[j] *= inv; }
         mL *= inv;
         scale = xE;
-        sbuf = (z == u) ? xE : sbuf;
-        totscale = (float) ((double) totscale + log((double) xE));
+        if (MODE != 3) {
+          sbuf = (z == u) ? xE : sbuf;
+          totscale = (float) ((double) totscale + log((double) xE));
+        }
         xE = 1.0f;
         if (TM == TM_LDS && MODE != 3) {
           // the pinned odds are read again, so that they need no registers
@@ -516,15 +518,20 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
                                 oaN, oaJ, oaB, oaC, obits, orow, opp);
       }
     };
-    if (L > 0) {
+    if constexpr (MODE == 3) {
+      // long rows that keep many registers: a scalar residue each, no row ahead
+      ResAsc rd;
+      rd.init(sq);
+      for (int i = 1; i <= L; i++) row(rd.at(i - 1) * (int) rowf * 4, 0, i, 0);
+    } else if (L > 0) {
       RowRes<false> rr;
-      int xoff = rr.init(sq, L, z, (int) rowf);
+      int xoff = rr.init(sq, L, z, (int) rowf * 4);      // in bytes: one instruction a row less
       if (PF) {
 #pragma unroll
-        for (int j = 0; j < (PF ? B : 1); j++) e[j] = tbl[xoff + z + j * 64];
+        for (int j = 0; j < (PF ? B : 1); j++) e[j] = ((const float *) ((const char *) tbl + xoff))[z + j * 64];
       }
       for (int i0 = 0; i0 < L; i0 += 64) {
-        const int cnt = min(64, L - i0);
+        const int cnt = uni(min(64, L - i0));
         sbuf = 1.0f;
         for (int u = 0; u < cnt; u++) {
           const int xnext = rr.ahead(u);
