@@ -23,6 +23,7 @@
 #include "p7_gpu.h"
 #include "p7g_internal.h"
 #include "p7g_device.h"
+#include "p7g_keep.h"
 
 extern "C" const char *p7g_host_error(void);
 
@@ -2648,9 +2649,10 @@ batch_reserve(Batch &b, int nprof, int64_t n, unsigned mask)
 {
   if (nprof <= b.nprof_cap && n <= b.n_cap && (mask & ~b.mask_cap) == 0) return p7G_OK;
   batch_drop_graph(b);
-  if (b.mem) { (void) hipFree(b.mem); b.mem = nullptr; }
   const int64_t np = std::max(nprof, b.nprof_cap), nn = std::max(n, b.n_cap);
   mask |= b.mask_cap;
+  if (b.mem) { (void) hipFree(b.mem); b.mem = nullptr; }
+  b.nprof_cap = 0; b.n_cap = 0; b.mask_cap = 0;            // until the new buffer is there
   size_t o = 0;
   auto take = [&](size_t bytes) { size_t at = o; o += (bytes + 255) & ~(size_t) 255; return at; };
   const size_t ozm = take(2 * (size_t) (np * nn)), oq = take(4 * (1 + P7G_SSV_MAXCHUNK) * (size_t) np),
@@ -3140,6 +3142,9 @@ struct Single {
 };
 static Single g_one;
 
+static void dev_free(void *p) { (void) hipFree(p); }
+template <typename T> static hipError_t dev_alloc(T **p, int64_t n) { return hipMalloc((void **) p, sizeof(T) * (size_t) n); }
+
 // The pinned buffer single targets pass through: 64 bytes of result words, then
 // an array of rows (or the bias filter's odds), then the residues. Kept between
 // calls up to SINGLE_PIN_KEEP bytes; a longer target's buffer is given back when
@@ -3149,12 +3154,8 @@ static int
 single_pin(int64_t bytes)
 {
   Single &o = g_one;
-  if (bytes <= o.pcap) return p7G_OK;
-  if (o.pin) (void) hipHostFree(o.pin);
-  o.pin = nullptr; o.pcap = 0;
-  const int64_t cap = std::max<int64_t>(bytes, 1 << 18);
-  HIPCHK(hipHostMalloc((void **) &o.pin, (size_t) cap, hipHostMallocDefault));
-  o.pcap = cap;
+  HIPCHK(keep_at_least(o.pin, o.pcap, bytes, std::max<int64_t>(bytes, 1 << 18), [](void *q) { (void) hipHostFree(q); },
+                       [](uint8_t **q, int64_t n) { return hipHostMalloc((void **) q, (size_t) n, hipHostMallocDefault); }));
   return p7G_OK;
 }
 
@@ -3167,12 +3168,7 @@ single_stage(const uint8_t *dsq, int L, DevSeqs *s, int32_t *list, int which, co
   Single &o = g_one;
   int status;
   const int64_t need = (((int64_t) L + 15) & ~(int64_t) 15) + 16;
-  if (need > o.cap) {
-    if (o.res) (void) hipFree(o.res);
-    o.res = nullptr; o.cap = 0;
-    HIPCHK(hipMalloc((void **) &o.res, (size_t) need));
-    o.cap = need;
-  }
+  HIPCHK(keep_at_least(o.res, o.cap, need, need, dev_free, dev_alloc<uint8_t>));
   if (! o.off) { HIPCHK(hipMalloc((void **) &o.off, 64)); HIPCHK(hipMalloc((void **) &o.len, 64)); }
   const int64_t rbytes = (nrows * 4 + 15) & ~(int64_t) 15;
   if ((status = single_pin(64 + rbytes + need)) != p7G_OK) return status;
@@ -3314,12 +3310,7 @@ single_xmx(int L)
 {
   Single &o = g_one;
   const int64_t need = single_rows(L) * 2;
-  if (need > o.xcap) {
-    if (o.xmx) (void) hipFree(o.xmx);
-    o.xmx = nullptr;
-    HIPCHK(hipMalloc((void **) &o.xmx, sizeof(float) * (size_t) need));
-    o.xcap = need;
-  }
+  HIPCHK(keep_at_least(o.xmx, o.xcap, need, need, dev_free, dev_alloc<float>));
   return p7G_OK;
 }
 
