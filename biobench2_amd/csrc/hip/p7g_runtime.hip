@@ -1072,7 +1072,8 @@ p7_gpu_MSVFilterBatch(const P7_GPU_OPROFILE *om, const P7_GPU_SEQDB *db, const i
   if (db->maxcode >= om->abc->Kp) { p7g_set_error("database holds residue codes outside the model alphabet"); return p7G_EINCOMPAT; }
   if ((status = dev_profile(om, db->Lmax, &p)) != p7G_OK) return status;
   if (idx == nullptr) n = db->nseq;
-  if ((status = work_reserve(g_work, db->nseq, 0)) != p7G_OK) return status;
+  // lists hold n targets, an index any number of times; results one per slot
+  if ((status = work_reserve(g_work, std::max(n, db->nseq), 0)) != p7G_OK) return status;
   std::vector<int32_t> slots;
   if ((status = slots_from_idx(db, idx, n, slots)) != p7G_OK) return status;
   DevSeqs s = seqs_of(db);
@@ -1181,7 +1182,7 @@ run_list_stage(int which, const P7_GPU_OPROFILE *om, const P7_GPU_SEQDB *db, con
   if ((status = slots_from_idx(db, idx, n, slots)) != p7G_OK) return status;
   int64_t poolneed = 0;
   if (which == ST_BCK) for (int64_t t = 0; t < n; t++) poolneed += db->h_len[slots[t]] + 1;
-  if ((status = work_reserve(g_work, db->nseq, poolneed)) != p7G_OK) return status;
+  if ((status = work_reserve(g_work, std::max(n, db->nseq), poolneed)) != p7G_OK) return status;   // an index may repeat
   for (int64_t t = 0; t < n; t++) if (db->h_len[slots[t]] == 0) { p7g_set_error("zero-length target in a batched stage"); return p7G_EINVAL; }
   DevSeqs s = seqs_of(db);
   Work &w = g_work;

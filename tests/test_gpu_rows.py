@@ -200,6 +200,24 @@ def test_lists_give_every_target_its_score(gpu, tmp_path, n):
             assert st[i] == st1[0] and sc[i] == one[0], (i, sc[i], one[0])
 
 
+def test_an_index_may_name_targets_more_often_than_the_database_holds(gpu, tmp_path):
+    """A list longer than the database: every entry has its target's score."""
+    rng = np.random.default_rng(17)
+    h = synth.random_profile(40, rng, "again")
+    h.stats = (-9.0, 0.6931, -9.5, 0.6931, -5.0, 0.6931)
+    path = str(tmp_path / "again.hmm")
+    synth.write_hmm(path, [h])
+    om = gpu.OProfile.from_file(path)
+    db = gpu.SeqDB.from_list(random_seqs(rng, [30, 200, 64, 1, 77]))
+    idx = rng.integers(0, 5, 6000).astype(np.int64)
+    for batch in (gpu.msv_batch, gpu.viterbi_batch, gpu.forward_batch, gpu.backward_batch, gpu.filter_score_batch):
+        each, many = batch(om, db), batch(om, db, idx)
+        if batch is gpu.filter_score_batch:
+            each, many = (each,), (many,)
+        for a, b in zip(each, many):
+            assert np.array_equal(a[idx], b)
+
+
 @pytest.mark.parametrize("L", [1, 15, 16, 17, 4967, 360000])
 def test_single_targets_pass_through_the_pinned_buffer(gpu, tmp_path, L):
     """Single-target calls of every size, up to rows past what the buffer keeps (8 MB), leave
