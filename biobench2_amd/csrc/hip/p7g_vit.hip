@@ -145,13 +145,13 @@ template <int ND, int TM>
 __global__ __launch_bounds__(VIT_THREADS(ND))
 void k_vit(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *__restrict__ off,
            const int32_t *__restrict__ len, const int32_t *__restrict__ list, const int32_t *__restrict__ count,
-           DevResults r, DevLists l, GateThresh g, int gating, LenCfg lc)
+           DevResults r, DevLists l, GateThresh g, int gating, LenCfg lc, int32_t above)
 {
 #pragma clang fp contract(off)
   static_assert(TM == TM_LDS || TM == TM_TLDS, "Viterbi tables are in LDS, whole or transitions only");
   constexpr bool PIN = (TM == TM_LDS), PMDS = (ND < 10 && ND != 6);
   const int lw = list_waves(*count);
-  if ((int64_t) blockIdx.x * lw >= *count) return;
+  if (*count <= above || (int64_t) blockIdx.x * lw >= *count) return;
   extern __shared__ int lds[];
   const size_t rowd = (size_t) 64 * ND;
   const int *tbl = p.vf_tbl;                             // emission rows
@@ -362,7 +362,7 @@ template <int ND>
 __global__ __launch_bounds__(64 * VIT_W)
 void k_vit_wg(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *__restrict__ off,
               const int32_t *__restrict__ len, const int32_t *__restrict__ list, const int32_t *__restrict__ count,
-              DevResults r, DevLists l, GateThresh g, int gating, LenCfg lc)
+              DevResults r, DevLists l, GateThresh g, int gating, LenCfg lc, int32_t upto)
 {
 #pragma clang fp contract(off)
   constexpr int W = VIT_W, NW = ND / W;
@@ -373,7 +373,7 @@ void k_vit_wg(const DevProfile p, const uint8_t *__restrict__ res, const int64_t
   __shared__ int4 sh_f[2][64];           // lanes whose M exceeds the specials' threshold
   __shared__ int sh_e[W];
   __shared__ int64_t sh_t;
-  if ((int64_t) blockIdx.x >= *count) return;
+  if (*count > upto || (int64_t) blockIdx.x >= *count) return;
   const int wv = uni(threadIdx.x >> 6), z = threadIdx.x & 63;
   const int d0 = wv * NW;
   const size_t rowd = (size_t) 64 * ND;
@@ -581,14 +581,19 @@ void k_vit_wg(const DevProfile p, const uint8_t *__restrict__ res, const int64_t
 
 // Viterbi: the whole table in LDS while it fits (ND <= 16 at 160 KB), else the
 // transitions in LDS and emission rows from global memory.
-// The cooperative kernel takes models of ND >= 20, and of ND = 12 and 16 when few
-// targets are expected (VIT_WG_FEW: all of a plain list, about one in 32 behind
-// the gates): its row is the shorter one (M = 1500 383 against 595 ns, 2000 416
-// against 930 ns), but its waves repeat the scan, and a full chip does less
-// (us for 512 | 4096 targets of 350, M = 2000: 320 | 1514 against 550 | 1072).
-// At ND = 8 the row gains little (350 against 386 ns). P7G_VIT_WG=0 selects the
-// one-wave kernel (for comparisons).
+// The cooperative kernel takes models of ND >= 20, and of ND = 12 and 16 short
+// lists: its row is the shorter one (M = 1500 383 against 595 ns, 2000 416 against
+// 930 ns), but its waves repeat the scan, and a full chip does less (us for 512 |
+// 4096 targets of 350, M = 2000: 320 | 1514 against 550 | 1072). Lists given by a
+// caller: up to VIT_WG_FEW targets. Lists behind the gates have a search's lengths,
+// whose longest targets keep the longer row waiting: up to VIT_WG_FEW_GATED (us at
+// M = 1500 for 1546 | 7975 of them: 845 | 2283 against 1240 | 1964; M = 2000, 1175 |
+// 5632: 1094 | 1899 against 1250 | 2019). Their number is not known on the host: both
+// kernels are launched, and the count on the device decides which leaves at once
+// (4 us). At ND = 8 the row gains little (350 against 386 ns). P7G_VIT_WG=0 selects
+// the one-wave kernel (for comparisons).
 #define VIT_WG_FEW 1024
+#define VIT_WG_FEW_GATED 4096
 static bool vit_wg_on()
 {
   static const bool on = [] { const char *v = getenv("P7G_VIT_WG"); return ! (v && v[0] == '0'); }();
@@ -601,23 +606,25 @@ hipError_t launch_vit(const DevProfile &p, const DevSeqs &s, const int32_t *list
 {
   if (maxn <= 0) return hipSuccess;
   // large models run the filter with several waves per target
-  const bool few = (gating ? maxn / 32 : maxn) <= VIT_WG_FEW;
   void *kw = nullptr;
-  int ww = 0;
+  int32_t upto = INT32_MAX;
   switch (p.vf_ND) {
-    case 12: if (few) { kw = (void *) k_vit_wg<12>; ww = VIT_W; } break;
-    case 16: if (few) { kw = (void *) k_vit_wg<16>; ww = VIT_W; } break;
-    case 20: kw = (void *) k_vit_wg<20>; ww = VIT_W; break;
-    case 24: kw = (void *) k_vit_wg<24>; ww = VIT_W; break;
-    case 32: kw = (void *) k_vit_wg<32>; ww = VIT_W; break;
-    case 40: kw = (void *) k_vit_wg<40>; ww = VIT_W; break;
+    case 12: kw = (void *) k_vit_wg<12>; upto = gating ? VIT_WG_FEW_GATED : VIT_WG_FEW; break;
+    case 16: kw = (void *) k_vit_wg<16>; upto = gating ? VIT_WG_FEW_GATED : VIT_WG_FEW; break;
+    case 20: kw = (void *) k_vit_wg<20>; break;
+    case 24: kw = (void *) k_vit_wg<24>; break;
+    case 32: kw = (void *) k_vit_wg<32>; break;
+    case 40: kw = (void *) k_vit_wg<40>; break;
     default: break;
   }
-  if (kw && p.vf_free && ! (lc.on && lc.xmove > 0) && vit_wg_on()) {
-    const unsigned grid = grid_for_waves_blk(kw, maxn * ww, 0, ww);
+  int32_t above = 0;
+  if (kw && p.vf_free && ! (lc.on && lc.xmove > 0) && vit_wg_on() && (gating || maxn <= upto)) {   // a caller's list holds maxn
+    const unsigned grid = grid_for_waves_blk(kw, std::min<int64_t>(maxn, upto) * VIT_W, 0, VIT_W);
     void *args[] = { (void *) &p, (void *) &s.res, (void *) &s.off, (void *) &s.len, (void *) &list, (void *) &count,
-                     &r, &l, &g, &gating, &lc };
-    return launch(kw, grid, 64 * ww, args, 0, st);
+                     &r, &l, &g, &gating, &lc, &upto };
+    const hipError_t e = launch(kw, grid, 64 * VIT_W, args, 0, st);
+    if (e != hipSuccess || maxn <= upto) return e;
+    above = upto;
   }
   void *k = nullptr;
   size_t lds = 0;
@@ -630,7 +637,7 @@ hipError_t launch_vit(const DevProfile &p, const DevSeqs &s, const int32_t *list
   }
   const unsigned grid = list_grid(k, maxn, lds, nthr / 64);
   void *args[] = { (void *) &p, (void *) &s.res, (void *) &s.off, (void *) &s.len, (void *) &list, (void *) &count,
-                   &r, &l, &g, &gating, &lc };
+                   &r, &l, &g, &gating, &lc, &above };
   return launch(k, grid, nthr, args, lds, st);
 }
 

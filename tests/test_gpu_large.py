@@ -5,9 +5,9 @@ the cooperative parsers take each of their other shapes (M = 1300, 1600,
 
 For these models the ungapped MSV pass runs in two chunks of model positions,
 joined by a boundary column in HBM (above M = 2560); the full MSV recurrence
-and Viterbi (above M = 2047) and Forward and Backward (B >= 32) run with four
-or eight waves per target, each wave owning a slice of every lane's
-positions; M = 2000 keeps the one-wave Viterbi with its whole table in LDS.
+(above M = 2047), Viterbi (above M = 2047, and from M = 1280 on in short lists as
+here) and Forward and Backward (B >= 16) run with four or eight waves per
+target, each wave owning a slice of every lane's positions.
 MSV and Viterbi must stay bit-exact against the oracle, Forward and Backward
 within 1e-4 nats of the oracle's fp32 restatement, and the whole pipeline
 must give the oracle's pass sets. The error of the fp32 Forward against the
@@ -25,8 +25,8 @@ from conftest import random_seqs
 pytestmark = pytest.mark.gpu
 
 LARGE = [2100, 2600, 5000]
-# every shape of the cooperative Viterbi kernel (ND = 20, 24, 32 at M = 3500, 40) and the one-wave
-# kernel with its whole table in LDS at its largest (ND = 16, M = 2000)
+# shapes of the cooperative Viterbi kernel (ND = 16 at M = 2000, 20, 24, 32 at M = 3500, 40); the
+# one-wave kernel at these sizes: test_gpu_rows.py, lists around the cooperative kernel's limit
 VIT_LARGE = [2000, 2100, 2600, 3500, 5000]
 # every instantiated shape of the cooperative Forward and Backward parsers (positions per lane
 # B = 24, 28, 32, 40, 48, 64, 80)

@@ -92,8 +92,9 @@ def test_row_scales_across_blocks(gpu, tmp_path, M, own):
 @pytest.mark.parametrize("M", [1, 2, 127, 128, 129, 257, 640, 1023, 1281, 1535, 1536, 2046, 2047, 2559, 3071, 4095])
 @pytest.mark.parametrize("tables", ["converted", "lazy", "loops"])
 def test_viterbi_rows_bit_exact(gpu, tmp_path, M, tables):
-    """Every instance at its largest model and just past it (ND dwords per lane hold
-    128 ND - 1 positions), as converted (each row's D->D paths closed), and with a ddbound
+    """Instances at their largest model and just past it (ND dwords per lane hold
+    128 ND - 1 positions; from M = 1280 on short lists like these run on several waves
+    per target where every row closes its D->D paths), as converted (each row's D->D paths closed), and with a ddbound
     that is no bound or loops that are not 0, which need the lazy test on every row."""
     rng = np.random.default_rng([8, M])
     h = synth.random_profile(M, rng, f"vit_M{M}")
@@ -117,6 +118,47 @@ def test_viterbi_rows_bit_exact(gpu, tmp_path, M, tables):
         xw[1, 0] = xw[2, 0] = xw[3, 0] = lm.xwmove[len(s)]
         st0, sc0, _ = oracle.vit_filter(s, t, xw)
         assert st0 == st[i] and (sc0 == sc[i] or (np.isinf(sc0) and np.isinf(sc[i]) and sc0 * sc[i] > 0)), (i, len(s), sc0, sc[i])
+
+
+@pytest.mark.parametrize("M", [1280, 1281, 1535, 1536, 2046])
+@pytest.mark.parametrize("n", [1024, 1025, 1500])
+def test_viterbi_lists_around_the_cooperative_kernels_limit(gpu, tmp_path, M, n):
+    """ND = 12 and 16 run a caller's lists of up to 1024 targets on several waves per target and
+    longer ones on one wave each, whose rows are closed too: both equal the oracle, homologs
+    that overflow among the targets. Behind the gates the limit is 4096, and the count on the
+    device decides between the two kernels."""
+    rng = np.random.default_rng([16, M])
+    h = synth.random_profile(M, rng, f"vitn_M{M}")
+    h.stats = (-9.0, 0.6931, -9.5, 0.6931, -5.0, 0.6931)
+    path = str(tmp_path / "vitn.hmm")
+    synth.write_hmm(path, [h])
+    om = gpu.OProfile.from_file(path)
+    cores = synth.emit_homologs(synth.read_hmm_probs(path), 3, rng)
+    kinds = random_seqs(rng, [1, 30, 63, 64, 65, 129, 200]) + [c[a:a + L] for c in cores for a, L in ((0, 60), (100, 130), (300, 500))]
+    t = om.tables()
+    lm = oracle.LengthModel(t, max(len(s) for s in kinds) + 1)
+    ref = []
+    for s in kinds:
+        xw = t["xw"].copy()
+        xw[1, 0] = xw[2, 0] = xw[3, 0] = lm.xwmove[len(s)]
+        ref.append(oracle.vit_filter(s, t, xw)[:2])
+    assert any(st for st, _ in ref) and any(np.isfinite(sc) for _, sc in ref)
+    same = lambda a, b: a == b or (np.isinf(a) and np.isinf(b) and a * b > 0)
+    sc, st = gpu.viterbi_batch(om, gpu.SeqDB.from_list([kinds[i % len(kinds)] for i in range(n)]))
+    for i in range(n):
+        st0, sc0 = ref[i % len(kinds)]
+        assert st0 == st[i] and same(sc0, sc[i]), (i, sc0, sc[i])
+    # F2 = 1e-30: what passes the first gate runs Viterbi, unless the bias filter's score alone is beyond F2
+    F = (0.99, 1e-30, 1e-30)
+    once = gpu.Pipeline(*F).run(om, gpu.SeqDB.from_list(kinds))
+    run = [i for i in range(len(kinds)) if not np.isnan(once["vfsc"][i])]
+    assert len(run) >= 3
+    n += 4096 - 1024
+    pick = [run[i % len(run)] for i in range(n)] + [i for i in range(len(kinds)) if i not in run] * 5
+    out = gpu.Pipeline(*F).run(om, gpu.SeqDB.from_list([kinds[i] for i in pick]))
+    assert int((~np.isnan(out["vfsc"])).sum()) == n
+    for j, i in enumerate(pick[:n]):
+        assert same(ref[i][1], out["vfsc"][j]), (j, i, ref[i], out["vfsc"][j])
 
 
 @pytest.mark.parametrize("M", [1, 127, 128, 129, 640, 1023, 1281, 2047, 2559, 3071, 4095])
