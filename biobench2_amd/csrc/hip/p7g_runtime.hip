@@ -3147,22 +3147,24 @@ static void dev_free(void *p) { (void) hipFree(p); }
 template <typename T> static hipError_t dev_alloc(T **p, int64_t n) { return hipMalloc((void **) p, sizeof(T) * (size_t) n); }
 
 // The pinned buffer single targets pass through: 64 bytes of result words, then
-// an array of rows (or the bias filter's odds), then the residues. Kept between
-// calls up to SINGLE_PIN_KEEP bytes; a longer target's buffer is given back when
-// its call ends. All single-target calls hold g_lock.
-#define SINGLE_PIN_KEEP (8 << 20)
+// an array of rows (or the bias filter's odds), then the residues. It is kept
+// between calls and at least doubles when it grows, up to SINGLE_PIN_KEEP bytes
+// (allocating pinned memory takes longer than these copies do); a target whose
+// arrays need more has them copied from and to the caller's memory, only its
+// result words pass through. All single-target calls hold g_lock.
+#define SINGLE_PIN_KEEP ((int64_t) 8 << 20)
 static int
 single_pin(int64_t bytes)
 {
   Single &o = g_one;
-  HIPCHK(keep_at_least(o.pin, o.pcap, bytes, std::max<int64_t>(bytes, 1 << 18), [](void *q) { (void) hipHostFree(q); },
+  HIPCHK(keep_at_least(o.pin, o.pcap, bytes, std::max({ bytes, (int64_t) 1 << 18, std::min(2 * o.pcap, SINGLE_PIN_KEEP) }), [](void *q) { (void) hipHostFree(q); },
                        [](uint8_t **q, int64_t n) { return hipHostMalloc((void **) q, (size_t) n, hipHostMallocDefault); }));
   return p7G_OK;
 }
 
 // Stages a target (and `rows`, nrows floats, to d_rows) and clears the counts,
-// with counts[which] = 1 and slot 0 in `list` when there is one. The pinned
-// buffer also has room for the rows the call returns.
+// with counts[which] = 1 and slot 0 in `list` when there is one. nrows is also
+// the size of the rows the call returns.
 static int
 single_stage(const uint8_t *dsq, int L, DevSeqs *s, int32_t *list, int which, const float *rows, float *d_rows, int64_t nrows)
 {
@@ -3172,14 +3174,24 @@ single_stage(const uint8_t *dsq, int L, DevSeqs *s, int32_t *list, int which, co
   HIPCHK(keep_at_least(o.res, o.cap, need, need, dev_free, dev_alloc<uint8_t>));
   if (! o.off) { HIPCHK(hipMalloc((void **) &o.off, 64)); HIPCHK(hipMalloc((void **) &o.len, 64)); }
   const int64_t rbytes = (nrows * 4 + 15) & ~(int64_t) 15;
-  if ((status = single_pin(64 + rbytes + need)) != p7G_OK) return status;
-  uint8_t *pr = o.pin + 64, *ps = pr + rbytes;
-  if (rows) memcpy(pr, rows, (size_t) nrows * 4);
-  memcpy(ps, dsq + 1, (size_t) L);
-  memset(ps + L, P7G_PADCODE, (size_t) (need - L));
+  const bool pinned = (64 + rbytes + need <= SINGLE_PIN_KEEP);
+  if ((status = single_pin(pinned ? 64 + rbytes + need : 64)) != p7G_OK) return status;
   SingleIn a;
-  a.src1 = ps; a.dst1 = o.res; a.n1 = need / 16;
-  a.src2 = pr; a.dst2 = d_rows; a.n2 = rows ? rbytes / 16 : 0;
+  a.src1 = a.src2 = nullptr; a.n1 = a.n2 = 0; a.dst1 = o.res; a.dst2 = d_rows;
+  if (pinned) {
+    uint8_t *pr = o.pin + 64, *ps = pr + rbytes;
+    if (rows) memcpy(pr, rows, (size_t) nrows * 4);
+    memcpy(ps, dsq + 1, (size_t) L);
+    memset(ps + L, P7G_PADCODE, (size_t) (need - L));
+    a.src1 = ps; a.n1 = need / 16;
+    if (rows) { a.src2 = pr; a.n2 = rbytes / 16; }
+  } else {
+    std::vector<uint8_t> h((size_t) need, P7G_PADCODE);
+    memcpy(h.data(), dsq + 1, (size_t) L);
+    HIPCHK(hipMemcpyAsync(o.res, h.data(), (size_t) need, hipMemcpyHostToDevice, g_stream));
+    if (rows) HIPCHK(hipMemcpyAsync(d_rows, rows, (size_t) nrows * 4, hipMemcpyHostToDevice, g_stream));
+    HIPCHK(hipStreamSynchronize(g_stream));                // h lives until its copy is done
+  }
   a.off = o.off; a.len = o.len; a.L = L; a.which = which;
   a.list = list; a.counts = g_work.l.counts; a.cursor = g_work.l.cursor;
   HIPCHK(launch_single_in(a, g_stream));
@@ -3194,14 +3206,15 @@ static int
 single_result(const void *w0, bool half, const int32_t *w1, int32_t out[2], const float *d_rows, float *rows, int64_t n)
 {
   Single &o = g_one;
+  const bool pinned = (64 + n * 4 <= o.pcap);
   SingleOut a;
-  a.src = d_rows; a.dst = (float *) (o.pin + 64); a.n = n;
+  a.src = d_rows; a.dst = (float *) (o.pin + 64); a.n = pinned ? n : 0;
   a.w0 = w0; a.w1 = w1; a.words = (int32_t *) o.pin; a.half = half ? 1 : 0;
   HIPCHK(launch_single_out(a, g_stream));
+  if (! pinned) HIPCHK(hipMemcpyAsync(rows, d_rows, (size_t) n * 4, hipMemcpyDeviceToHost, g_stream));
   HIPCHK(hipStreamSynchronize(g_stream));
   memcpy(out, o.pin, 8);
-  if (n) memcpy(rows, o.pin + 64, (size_t) n * 4);
-  if (o.pcap > SINGLE_PIN_KEEP) { (void) hipHostFree(o.pin); o.pin = nullptr; o.pcap = 0; }
+  if (pinned && n) memcpy(rows, o.pin + 64, (size_t) n * 4);
   return p7G_OK;
 }
 

@@ -289,3 +289,10 @@ def test_single_targets_pass_through_the_pinned_buffer(gpu, tmp_path, L):
                                     (gpu.forward_batch(om, db), f, fst, 1e-5), (gpu.backward_batch(om, db), b, bst, 1e-5)):
         assert st[0] == st1 and abs(sc[0] - one) <= tol * max(1.0, abs(one)), (sc[0], one)
     assert got[1].shape == (L + 1, 6) and np.isfinite(got[1]).all() and np.isfinite(got[2]).all()
+
+
+@pytest.mark.parametrize("L", [335539, 335540])
+def test_single_targets_around_the_kept_pinned_size(gpu, tmp_path, L):
+    """The longest target whose rows and residues fit the 8 MB that are kept, and one more
+    residue, whose arrays are copied from and to the caller's memory."""
+    test_single_targets_pass_through_the_pinned_buffer(gpu, tmp_path, L)
