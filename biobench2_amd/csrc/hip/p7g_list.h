@@ -133,7 +133,7 @@ __device__ __forceinline__ float fma2(float a, float b, float c, float d)
 __device__ __forceinline__ void fma_onto(float &x, float a, float t)
 {
   x = __builtin_fmaf(x, a, t);
-  asm("" :: "v"(t));
+  asm("" : "+v"(x) : "v"(t));
 }
 
 // v where the lane's bit of a constant mask is set, else w: one v_cndmask. The

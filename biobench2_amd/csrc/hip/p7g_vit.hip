@@ -151,7 +151,7 @@ void k_vit(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
   static_assert(TM == TM_LDS || TM == TM_TLDS, "Viterbi tables are in LDS, whole or transitions only");
   constexpr bool PIN = (TM == TM_LDS), PMDS = (ND < 10 && ND != 6);
   const int lw = list_waves(*count);
-  if (*count <= above || (int64_t) blockIdx.x * lw >= *count) return;
+  if (((ND == 12 || ND == 16) && *count <= above) || (int64_t) blockIdx.x * lw >= *count) return;
   extern __shared__ int lds[];
   const size_t rowd = (size_t) 64 * ND;
   const int *tbl = p.vf_tbl;                             // emission rows
