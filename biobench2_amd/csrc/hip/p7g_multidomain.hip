@@ -94,10 +94,11 @@ __device__ __forceinline__ void md_thresholds(const float *v, int n, double *th)
   for (int a = 0; a < n - 1; a++) th[a] = c[a] / tot;
 }
 
-// The workgroup is one wavefront, whose LDS operations complete in the order
-// it issues them: between lanes that only exchange data through LDS it is
-// enough that the compiler moves no memory operation across this point (a
-// workgroup barrier would also wait for the outstanding global stores).
+// Where one wavefront works alone, its LDS operations, and its loads and stores
+// of one address, complete in the order it issues them: between lanes that
+// exchange data so it is enough that the compiler moves no memory operation
+// across this point (a workgroup barrier would also wait for the outstanding
+// global stores, and waves that have left the workgroup could not reach it).
 __device__ __forceinline__ void md_sync()
 {
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -870,7 +871,8 @@ k_md_replay(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__
   for (int pos = tid + 1; pos <= Lr; pos += NT) acc[pos] = logf(__fdiv_rn(acc[pos], (float) nsamples));
   if (tid == 0) { O->rtrace = ntr; O->rdom = nseg; O->done = 1; }
   __syncthreads();
-  if (wv != 0) return;                                     // the rest is one wave's work
+  if (wv != 0) return;                                     // the rest is one wave's work, without barriers
+  auto l2_sync = []() { __threadfence(); md_sync(); };     // around counts made by atomics at L2
 
   // ---------------- 3. clustering ----------------
   // the two stacks of the linkage in LDS; each element's cluster and each
@@ -881,13 +883,13 @@ k_md_replay(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__
   MdSig *sig = (MdSig *) (lk + (J.segcap + 63) / 64);
   const int n = nseg;
   for (int v = z; v < n; v += 64) { av[v] = n - v - 1; ninc[v] = 0; }
-  __syncthreads();
+  l2_sync();
   int na = n, nb = 0, ncl = 0;
   while (na > 0) {
     na--;
     if (z == 0) bv[nb] = av[na];
     nb++;
-    __syncthreads();
+    md_sync();
     while (nb > 0) {
       nb--;
       const int v = bv[nb];
@@ -900,7 +902,7 @@ k_md_replay(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__
         const unsigned long long m = __ballot(l);
         if (z == 0) lk[w] = m;
       }
-      __syncthreads();
+      md_sync();
       // the linked slots, highest first: each leaves by taking the top's element
       for (int w = nw - 1; w >= 0; w--) {
         unsigned long long m = lk[w];
@@ -910,21 +912,21 @@ k_md_replay(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__
           const int a = w * 64 + bit;
           if (z == 0) { const int we = av[a]; av[a] = av[na - 1]; bv[nb] = we; }
           na--; nb++;
-          __syncthreads();
+          md_sync();
         }
       }
-      __syncthreads();
+      md_sync();
     }
     ncl++;
   }
-  __syncthreads();
+  md_sync();
   // posterior of each cluster: the traces with a member (members of one trace are adjacent)
   for (int h = z; h < n; h += 64) {
     bool first = true;
     for (int h2 = h - 1; h2 >= 0 && segs[h2].idx == segs[h].idx; h2--) if (asg[h2] == asg[h]) first = false;
     if (first) atomicAdd(&ninc[asg[h]], 1);
   }
-  __syncthreads();
+  l2_sync();
   int nsig = 0;
   for (int c = 0; c < ncl; c++) {
     const int ni = __hip_atomic_load(&ninc[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // counted at L2
@@ -941,12 +943,12 @@ k_md_replay(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__
     for (int e = 0; e < 4; e++) {                          // i, j, k, m: leftmost start, rightmost end with support
       const int w = hi4[e] - lo[e] + 1;
       for (int b = z; b < w; b += 64) hist[b] = 0;
-      __syncthreads();
+      l2_sync();
       for (int h = z; h < n; h += 64) if (asg[h] == c) {
         const int v = (e == 0) ? segs[h].i : (e == 1) ? segs[h].j : (e == 2) ? segs[h].k : segs[h].m;
         atomicAdd(&hist[v - lo[e]], 1);
       }
-      __syncthreads();
+      l2_sync();
       // the counts were made by atomics at L2: read them there too
       auto hcount = [&](int o) { return __hip_atomic_load(&hist[o], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
       int b = -1;
@@ -963,14 +965,14 @@ k_md_replay(const DevProfile p, const uint8_t *__restrict__ res, const MdJob *__
         b = -wave_max_i(bc == mc ? -bi : -0x7fffffff);
       }
       best[e] = lo[e] + b;
-      __syncthreads();
+      md_sync();
     }
     if (best[0] > best[1] || best[2] > best[3]) continue;
     if (nsig >= MD_MAXSIG) { status = 5; break; }
     if (z == 0) sig[nsig] = MdSig{ c, best[0], best[1], best[2], best[3], __fdiv_rn((float) ni, (float) nsamples) };
     nsig++;
   }
-  __syncthreads();
+  md_sync();
   if (status) { if (z == 0) { O->status = status; O->nc = 0; O->nseg = nseg; } return; }
   if (z == 0) {
     for (int a = 1; a < nsig; a++) {                       // start order; equal starts keep their order
