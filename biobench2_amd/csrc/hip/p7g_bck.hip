@@ -43,6 +43,8 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
   }
 #define BTR(A, T, j) (PIN ? A[j] : trr[(T) * rowf + (j) * 64])
   constexpr bool DOM = (MODE == 1), ENV = (MODE == 2), STREAM = (TM == TM_GLOB), PF = ! STREAM;
+  // which product of I's and M's update is rounded first (as FP in k_fwd: the order
+  // each size was first compiled with, the same in every mode)
   constexpr bool FI = (B == 1 || (B >= 6 && B <= 8)), FM = (B == 1 || (B >= 7 && B <= 8));
   const int64_t n = ENV ? min((int64_t) *count, dom.env_cap) : (int64_t) *count;
   const float eMove = ENV ? 1.0f : p.xfE_move, eLoop = ENV ? 0.0f : p.xfE_loop;

@@ -286,8 +286,12 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
   }
   // PF: a row's emission odds are loaded a row ahead (not where the positions
   // of a large model, or the alignment's state, already fill the registers).
-  // PIND: the D->D odds are pinned too.
-  constexpr bool FP = (B == 1 && MODE != 3);
+  // PIND: the D->D odds are pinned too. STREAM: nothing is (see stream_tables).
+  // FP: which product of xB * tBM + M * tMM is rounded before the other is fused
+  // onto it. The choice is the one each size was first compiled with, kept so that
+  // results stay; it depends on B alone, because the null2 pass must rescale the
+  // same rows as the envelope-score pass, whose scales Backward has taken.
+  constexpr bool FP = (B == 1);
   constexpr int EG = (MODE == 3) ? 8 : 16;
   constexpr bool STREAM = (TM == TM_GLOB && MODE != 3), PF = (MODE != 3 && B <= 28), PIND = (PIN && MODE != 3 && B <= 4);
   AffConst akc;

@@ -224,10 +224,10 @@ __device__ __forceinline__ void affine_fwd_scan(float (&D)[B], const float (&a)[
   // D(j) = D0(j) + a(j) * D(j-1), carried across lanes in increasing k
   float C = D[0];
 #pragma unroll
-  for (int j = 1; j < B; j++) C = D[j] + a[j] * C;
+  for (int j = 1; j < B; j++) C = __builtin_fmaf(a[j], C, D[j]);
   float cur = lane_carry_fwd(C, k);
 #pragma unroll
-  for (int j = 0; j < B; j++) { cur = D[j] + a[j] * cur; D[j] = cur; }
+  for (int j = 0; j < B; j++) { cur = __builtin_fmaf(a[j], cur, D[j]); D[j] = cur; }
 }
 
 // a(j) gives the D->D odds of the lane's position j (read twice per call, so
@@ -238,10 +238,10 @@ __device__ __forceinline__ void affine_bck_scan(float (&D)[B], A a, const AffCon
   // D(j) = c(j) + a(j) * D(j+1), carried across lanes in decreasing k
   float C = D[B-1];
 #pragma unroll
-  for (int j = B-2; j >= 0; j--) C = D[j] + a(j) * C;
+  for (int j = B-2; j >= 0; j--) C = __builtin_fmaf(a(j), C, D[j]);
   float cur = lane_carry_bck(C, k);
 #pragma unroll
-  for (int j = B-1; j >= 0; j--) { cur = D[j] + a(j) * cur; D[j] = cur; }
+  for (int j = B-1; j >= 0; j--) { cur = __builtin_fmaf(a(j), cur, D[j]); D[j] = cur; }
 }
 
 // The values of NT tables at a lane's B positions, read from memory where a row

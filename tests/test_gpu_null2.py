@@ -170,3 +170,66 @@ def test_null2_of_the_shortest_envelopes(gpu):
     regs = pli.regions()
     assert min(j - i + 1 for _, i, j, _, _ in regs) <= 3
     check_regions(pli, om, lambda q: seqs[q], min_checked=20)
+
+
+@pytest.mark.parametrize("M", [60, 100, 250, 500])
+def test_null2_rows_rescale_with_the_envelope_scores(gpu, tmp_path, M):
+    """Backward takes the row scales of the envelope-score pass, and the null2 pass runs those
+    Forward rows again: both must rescale the same ones, also where a row sum lies next to the
+    limit of 1e4. The odds of the residue in such a row are
+    moved in steps of one unit in the last place, so that the sum crosses the limit within
+    some hundred of them. The correction moves by parts in 1e5 then; were one pass to rescale
+    the row and the other not, every posterior behind it would be off by a factor of 1e4."""
+    rng = np.random.default_rng(18)
+    h = synth.random_profile(M, rng, f"limit_M{M}")
+    h.stats = (-9.0, 0.6931, -9.5, 0.6931, -5.0, 0.6931)
+    path = str(tmp_path / "limit.hmm")
+    synth.write_hmm(path, [h])
+    om = gpu.OProfile.from_file(path)
+    bg = lambda n: synth.iid_residues(n, rng)
+    seqs = [np.concatenate([bg(20), core[:75], bg(25)]) for core in synth.emit_homologs(synth.read_hmm_probs(path), 8, rng)]
+    t = om.tables()
+    db = gpu.SeqDB.from_list(seqs)
+    pli = gpu.Pipeline(1.0, 1.0, 1.0, domains=True)
+
+    def regions(tt):
+        om.load(tt)
+        pli.run(om, db)
+        return [r[:4] for r in pli.regions()], pli.region_null2()[0].astype(np.float64)
+
+    regs, _ = regions(t)
+    checked = 0
+    for n, (q, i, j, multi) in enumerate(regs):
+        env, xf = seqs[q][i - 1:j], oracle.unihit_xf(t, seqs[q].size)
+        rows = np.nonzero(oracle.fwd_parser(env, t, xf)[2][:, 5] > 1)[0]
+        if multi or not rows.size:
+            continue
+        r, x = int(rows[0]), int(env[rows[0] - 1])
+
+        def scaled(f):
+            tt = dict(t)
+            tt["rfv"] = t["rfv"].copy()
+            tt["rfv"][x] = (t["rfv"][x].astype(np.float64) * f).astype(np.float32)
+            return tt
+
+        def row_sum(f):
+            xm = oracle.fwd_parser(env, scaled(f), xf)[2]
+            return float(xm[r, 5]) if xm[r, 5] > 1 else float(xm[r, 0])
+
+        lo, hi = 0.05, 1.0                              # row_sum(lo) < 1e4 < row_sum(hi)
+        assert row_sum(lo) < 1e4 < row_sum(hi)
+        for _ in range(60):
+            mid = 0.5 * (lo + hi)
+            lo, hi = (lo, mid) if row_sum(mid) > 1e4 else (mid, hi)
+        if (q, i, j, multi) not in regions(scaled(lo))[0]:
+            continue                                    # not the same region with these odds
+        got = []
+        for d in range(-150, 151):
+            rg, dc = regions(scaled(lo * (1.0 + d * 2.0 ** -24)))
+            at = [k for k, (q2, i2, j2, m2) in enumerate(rg) if (q2, i2, j2, m2) == (q, i, j, multi)]
+            if at:
+                got.append(float(dc[at[0]]))
+        assert len(got) >= 200
+        assert max(got) - min(got) <= 1e-5 * (j - i + 1), (q, i, j, min(got), max(got), got)
+        checked += 1
+    assert checked >= 1
