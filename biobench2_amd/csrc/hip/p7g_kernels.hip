@@ -80,7 +80,6 @@ void k_msv_full(const DevProfile p, const int *__restrict__ tbl, int tbl_dwords,
 
   if ((int) (threadIdx.x >> 6) >= lw) return;
   for (int64_t t = queue_next(queue, 1); t < n; t = queue_next(queue, 1)) {
-    list_prio(t);
     const int slot = uni(list[t]);
     const int L = uni(len[slot]);
     const uint8_t *sq = res + off[slot];

@@ -92,17 +92,6 @@ __device__ __forceinline__ int list_waves(int64_t count)
   const int w = (int) (blockDim.x >> 6);
   return (w > LIST_SIMDS && count <= (int64_t) LIST_SIMDS * gridDim.x) ? LIST_SIMDS : w;
 }
-// The issue priority of a list's t-th target (longest first): the longest, one
-// per SIMD of the chip, before the others, whose rows fill the cycles between
-// theirs; among equals the last target to end would be the longest one. Forward
-// over 10,007 targets, M = 149: 1250 to 1127 us.
-__device__ __forceinline__ void list_prio(int64_t t)
-{
-  if (t < 1024) __builtin_amdgcn_s_setprio(3);
-  else if (t < 2048) __builtin_amdgcn_s_setprio(2);
-  else if (t < 4096) __builtin_amdgcn_s_setprio(1);
-  else __builtin_amdgcn_s_setprio(0);
-}
 // Their grid: enough workgroups for one wave per SIMD, none that cannot be resident.
 static inline unsigned list_grid(const void *kernel, int64_t maxn, size_t lds_bytes, int wpb)
 {

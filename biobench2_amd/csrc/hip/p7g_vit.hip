@@ -175,7 +175,6 @@ void k_vit(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
   int32_t *queue = (int32_t *) count + P7G_QOFF;
   if ((int) (threadIdx.x >> 6) >= lw) return;
   for (int64_t t = queue_next(queue, 1); t < n; t = queue_next(queue, 1)) {
-    list_prio(t);
     const int slot = uni(list[t]);
     const int L = uni(len[slot]);
     const uint8_t *sq = res + off[slot];

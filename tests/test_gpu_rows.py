@@ -225,7 +225,7 @@ def test_bias_rows_bit_exact(gpu, tmp_path, compo):
 
 @pytest.mark.parametrize("n", [1, 5, 4500, 12000])
 def test_lists_give_every_target_its_score(gpu, tmp_path, n):
-    """Short lists run on four waves of a workgroup, long ones on all, by falling priority:
+    """Short lists run on four waves of a workgroup, long ones on all:
     each target's scores are those of a list of its own few."""
     rng = np.random.default_rng(12)
     h = synth.random_profile(30, rng, "lists")
