@@ -498,8 +498,14 @@ void k_bck_wg(const DevProfile p, const uint8_t *__restrict__ res, const int64_t
   }
 }
 
+// the parser that keeps no rows; from B = 16 on k_bck_wg takes these calls
+template <int B, int TM> static void *bck_plain()
+{
+  if constexpr (B < 16) return (void *) k_bck<B, TM, 0>;
+  else return nullptr;
+}
 #define BCK_CASE(N, T) case N * 4 + T: k = dom.env_loop ? (void *) k_bck<N, T, 2> : (dom.pool || xmx_out) ? (void *) k_bck<N, T, 1> \
-                                          : (void *) k_bck<N, T, 0>; nthr = BCK_THREADS(N); break;
+                                          : bck_plain<N, T>(); nthr = BCK_THREADS(N); break;
 
 #define BCK_WG_CASE(N, W) case N: kw = xmx_out ? (void *) k_bck_wg<N, W, true> : (void *) k_bck_wg<N, W, false>; ww = W; break;
 hipError_t launch_bck(const DevProfile &p, const DevSeqs &s, const int32_t *list, const int32_t *count, int64_t maxn,
@@ -538,6 +544,7 @@ hipError_t launch_bck(const DevProfile &p, const DevSeqs &s, const int32_t *list
     FB_CASES(BCK_CASE)
     default: return hipErrorInvalidValue;
   }
+  if (! k) return hipErrorInvalidValue;
   const size_t lds = fb_lds(p, tm);
   const unsigned grid = list_grid(k, maxn, lds, nthr / 64);
   void *args[] = { (void *) &p, (void *) &s.res, (void *) &s.off, (void *) &s.len, (void *) &list, (void *) &count,

@@ -16,7 +16,6 @@ typedef short s2v __attribute__((ext_vector_type(2)));
 // Workgroup size of the one-target-per-wave list stages: 8 waves share one LDS
 // copy of the profile.
 #define LIST_BLOCK 512
-// 16-byte loads the bias filter's ordered sum keeps in flight.
 
 __device__ __forceinline__ int   s2i(s2v v) { return __builtin_bit_cast(int, v); }
 __device__ __forceinline__ s2v   i2s(int v) { return __builtin_bit_cast(s2v, v); }
@@ -30,7 +29,6 @@ __device__ __forceinline__ int   pair16(int v) { return (int)(((unsigned)v & 0xf
 __device__ __forceinline__ int wave_shr1(int v, int fill) { return __builtin_amdgcn_update_dpp(fill, v, 0x138, 0xf, 0xf, false); }
 __device__ __forceinline__ int wave_shl1(int v, int fill) { return __builtin_amdgcn_update_dpp(fill, v, 0x130, 0xf, 0xf, false); }
 __device__ __forceinline__ int row_shr1(int v, int fill)  { return __builtin_amdgcn_update_dpp(fill, v, 0x111, 0xf, 0xf, false); }
-__device__ __forceinline__ float wave_shl1f(float v) { return __builtin_bit_cast(float, wave_shl1(__builtin_bit_cast(int, v), 0)); }
 
 // Row shift of a packed block: the dword that becomes the new position pair 0.
 template <int G>

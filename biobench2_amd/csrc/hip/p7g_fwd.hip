@@ -811,8 +811,14 @@ void k_fwd_wg(const DevProfile p, const uint8_t *__restrict__ res, const int64_t
   }
 }
 
+// the parser that keeps no rows; from B = 16 on k_fwd_wg takes these calls
+template <int B, int TM> static void *fwd_plain()
+{
+  if constexpr (B < 16) return (void *) k_fwd<B, TM, 0>;
+  else return nullptr;
+}
 #define FWD_CASE(N, T) case N * 4 + T: k = dom.env_loop ? (dom.n2mode == 2 ? (void *) k_fwd<N, T, 3> : (void *) k_fwd<N, T, 2>) \
-                                          : (dom.pool || xmx_out) ? (void *) k_fwd<N, T, 1> : (void *) k_fwd<N, T, 0>; \
+                                          : (dom.pool || xmx_out) ? (void *) k_fwd<N, T, 1> : fwd_plain<N, T>(); \
                                           nthr = FWD_THREADS(N); break;
 
 #define FWD_WG_CASE(N, W) case N: kw = xmx_out ? (void *) k_fwd_wg<N, W, true> : (void *) k_fwd_wg<N, W, false>; ww = W; break;
@@ -854,6 +860,7 @@ hipError_t launch_fwd(const DevProfile &p, const DevSeqs &s, const int32_t *list
     FB_CASES(FWD_CASE)
     default: return hipErrorInvalidValue;
   }
+  if (! k) return hipErrorInvalidValue;
   // the null2 pass in workgroups of four waves (one per SIMD), so that one of
   // them fits on a compute unit beside a multidomain region's wave
   if (dom.env_loop && dom.n2mode == 2) nthr = std::min(nthr, NULL2_THREADS);

@@ -20,12 +20,9 @@
 //   2. k_msv_classify decides per target: overflow (some row reaches
 //      xE + bias >= 255), exact score (J never above base, xJ = max xE - tec), or
 //      "needs the J state" -> k_msv_full runs the row-serial recurrence.
-// Viterbi filter (vitfilter.c:84-249): int16 pairs with v_pk_add_i16 clamp =
-// _mm_adds_epi16 and v_pk_max_i16 = _mm_max_epi16; the lazy-F condition
-// (Dmax + ddbound > xB) is evaluated per row exactly as the reference does, and
-// when it holds the D->D closure is a max-plus prefix scan across the wave.
-// Forward/Backward parsers (fwdback.c:258-735): fp32, the D->D chain as an
-// affine prefix scan across the wave, sparse rescaling when xE > 1e4.
+// This file holds the MSV stage's decision and full recurrence, the bias filter,
+// domain decoding and the stages' compaction; Viterbi, Forward and Backward are in
+// files of their own.
 #include "p7g_list.h"
 
 /*****************************************************************
@@ -57,13 +54,12 @@ __global__ void k_msv_classify(const DevProfile p, const int32_t *__restrict__ l
 /*****************************************************************
  * 3. MSV stage, full recurrence (one target per wave, 64 lanes)
  *****************************************************************/
-// LDS: the score table is staged in LDS; otherwise (models whose table does
-// not fit, ND >= 24) the rows are read from global memory. Bound by the row's
-// chain of a long target alone: residues come 64 rows at a time and the scores a
-// row ahead. Lists of 60,013 targets, M = 86: 95 us; 5,003 targets with longer
+// The score table is staged in LDS (models of ND <= 16; larger ones run
+// k_msv_full_wg). Bound by the row's chain of a long target alone: residues come
+// 64 rows at a time and the scores a row ahead. Lists of 60,013 targets, M = 86: 95 us; 5,003 targets with longer
 // ones, M = 50: 88 us (217 and 205 us with both fetched in the row, the floor at
 // 0 as an instruction and a wave maximum every row).
-template <int ND, bool LDS>
+template <int ND>
 __global__ __launch_bounds__(512)
 void k_msv_full(const DevProfile p, const int *__restrict__ tbl, int tbl_dwords,
                 const uint8_t *__restrict__ res, const int64_t *__restrict__ off, const int32_t *__restrict__ len,
@@ -72,8 +68,8 @@ void k_msv_full(const DevProfile p, const int *__restrict__ tbl, int tbl_dwords,
   const int lw = list_waves(*count);
   if ((int64_t) blockIdx.x * lw >= *count) return;
   extern __shared__ int lds[];
-  const int *rows = tbl;
-  if (LDS) { stage_table(lds, tbl, (size_t) tbl_dwords); rows = lds; }
+  const int *rows = lds;
+  stage_table(lds, tbl, (size_t) tbl_dwords);
   const int z = threadIdx.x & 63;
   const int64_t n = *count;
   int32_t *queue = (int32_t *) count + P7G_QOFF;
@@ -948,7 +944,7 @@ hipError_t launch_msv_classify(const DevProfile &p, const DevSeqs &s, const int3
   return hipGetLastError();
 }
 
-#define MF_CASE(N, LDS) case N: k = (void *) k_msv_full<N, LDS>; break;
+#define MF_CASE(N) case N: k = (void *) k_msv_full<N>; break;
 hipError_t launch_msv_full(const DevProfile &p, const DevSeqs &s, const int32_t *list, const int32_t *count,
                            int64_t maxn, int16_t *xj, LenCfg lc, hipStream_t st)
 {
@@ -971,12 +967,10 @@ hipError_t launch_msv_full(const DevProfile &p, const DevSeqs &s, const int32_t 
   }
   void *k = nullptr;
   switch (p.mf_ND) {
-    MF_CASE(1, true) MF_CASE(2, true) MF_CASE(3, true) MF_CASE(4, true) MF_CASE(5, true) MF_CASE(6, true)
-    MF_CASE(8, true) MF_CASE(10, true) MF_CASE(12, true) MF_CASE(16, true) MF_CASE(20, true)
-    MF_CASE(24, false) MF_CASE(32, false) MF_CASE(40, false)
+    MF_CASE(1) MF_CASE(2) MF_CASE(3) MF_CASE(4) MF_CASE(5) MF_CASE(6) MF_CASE(8) MF_CASE(10) MF_CASE(12) MF_CASE(16)
     default: return hipErrorInvalidValue;
   }
-  const size_t lds = (p.mf_ND <= 20) ? p.mf_dwords * 4 : 0;
+  const size_t lds = p.mf_dwords * 4;
   const unsigned grid = list_grid(k, maxn, lds, LIST_BLOCK / 64);
   int tbl_dwords = (int) p.mf_dwords;
   void *args[] = { (void *) &p, (void *) &p.mf_tbl, &tbl_dwords, (void *) &s.res, (void *) &s.off, (void *) &s.len,

@@ -1,4 +1,4 @@
-"""Multidomain regions on the device (k_md_region; region_trace_ensemble,
+"""Multidomain regions on the device (k_md_fwd to k_md_replay; region_trace_ensemble,
 HMMER/src/p7_domaindef.c:600-690, and the rescoring of its clusters,
 :440-476): the region's multihit Forward matrix in the reference's operation
 order, 200 sampled traces from the seeded generator, null2 by trace, single-
