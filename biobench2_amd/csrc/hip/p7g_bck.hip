@@ -125,7 +125,7 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
     // One row, as in k_fwd: the emission odds come a row ahead (PF), Forward's
     // scale factors and the residues 64 rows at a time, and the row's specials
     // leave 64 rows at a time. A row of one target alone, M = 20 | 86 | 400 |
-    // 803: 190 | 218 | 320 | 497 ns (before 367 | 392 | 468 | 684 ns).
+    // 803: 188 | 195 | 301 | 499 ns (before 422 | 455 | 525 | 740 ns).
     float bE = 0.0f, bN = 0.0f, bJ = 0.0f, bB = 0.0f, bC = 0.0f, bS = 0.0f;
     float e[B];
     auto row = [&](int xoff, int xnext, int fsbits, int i, int u) {
@@ -271,7 +271,7 @@ void k_bck(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
 // constants, one for the waves' parts of the B sum and the slices' first M; the
 // next slice's D at its first position is the chain's carry into this one, and
 // every wave updates the special states by itself.
-// Bound by the row's chain of dependent steps; M = 2600 (B = 48, W = 4): 760 ns
+// Bound by the row's chain of dependent steps; M = 2600 (B = 48, W = 4): 761 ns
 // a row, where four barriers and odds loaded in the row made it 1250 ns.
 __device__ __forceinline__ void aff_setup_lane_bck(AffConst &k, float P)
 {
@@ -514,7 +514,7 @@ hipError_t launch_bck(const DevProfile &p, const DevSeqs &s, const int32_t *list
 {
   if (maxn <= 0) return hipSuccess;
   // large models run the parser with several waves per target, as Forward does
-  // (a single target's row of M = 1000 | 2600: 540 | 773 ns, one wave 949 | 3277 ns)
+  // (a single target's row of M = 1000 | 2600: 528 | 761 ns, one wave 922 | 3267 ns)
   void *kw = nullptr;
   int ww = 0;
   if (! dom.pool && ! dom.env_loop) {

@@ -136,8 +136,9 @@ __device__ __forceinline__ void list_append(bool pred, int32_t val, int32_t *__r
 }
 
 // Next item of a device work queue shared by the waves of one launch
-// (wave-uniform). Lists are in slot order, longest target first, so waves
-// taking items in queue order schedule the longest work first.
+// (wave-uniform). Lists compacted behind the gates are in slot order, longest
+// target first, so waves taking items in queue order schedule the longest work
+// first; a caller's list keeps the caller's order.
 __device__ __forceinline__ int queue_next(int32_t *q, int step)
 {
   int v = 0;

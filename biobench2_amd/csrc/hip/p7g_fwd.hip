@@ -386,9 +386,9 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
     // branch that it can do without: the next row's emission odds take this
     // row's registers once M is done (PF), a row's scale and specials go to
     // registers of lane u and leave 64 rows at a time, and the rescaling test
-    // is a scalar one. A row of one target alone, M = 20 | 86 | 400 | 803: 190 |
-    // 210 | 334 | 500 ns (with odds, residues and scales fetched in the row and
-    // the branches 289 | 310 | 434 | 646 ns).
+    // is a scalar one. A row of one target alone, M = 20 | 86 | 400 | 803: 198 |
+    // 209 | 352 | 513 ns (with odds, residues and scales fetched in the row and
+    // the branches 305 | 329 | 451 | 656 ns).
     float sbuf = 1.0f;                          // lane u: the scale of the block's row u
     float bE = 0.0f, bN = 0.0f, bJ = 0.0f, bB = 0.0f, bC = 0.0f;
     float e[PF ? B : 1];
@@ -594,7 +594,7 @@ void k_fwd(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
 // next slice's first position continues from (in row i+1 and, through M of the
 // position before it, which every wave forms again, in its own row's D). Every
 // wave updates the special states and rescales by itself, from the same sum.
-// Bound by the row's chain of dependent steps; M = 2600 (B = 48, W = 4): 820 ns
+// Bound by the row's chain of dependent steps; M = 2600 (B = 48, W = 4): 832 ns
 // a row, where four barriers and odds loaded in the row made it 1083 ns.
 __device__ __forceinline__ void aff_setup_lane(AffConst &k, float P)
 {
@@ -830,7 +830,7 @@ hipError_t launch_fwd(const DevProfile &p, const DevSeqs &s, const int32_t *list
   if (maxn <= 0) return hipSuccess;
   // large models run the parser with several waves per target (4 up to 48
   // positions per lane, 8 above), also for a single target, whose row of
-  // M = 1000 | 2600 takes 660 | 840 ns instead of one wave's 1034 | 2781 ns
+  // M = 1000 | 2600 takes 617 | 832 ns instead of one wave's 1028 | 2778 ns
   void *kw = nullptr;
   int ww = 0;
   if (! dom.pool && ! dom.env_loop) {

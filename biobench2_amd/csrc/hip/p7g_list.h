@@ -84,8 +84,10 @@ __device__ __forceinline__ void lds_barrier()
 // while the list has no more than four targets per workgroup, else all. A wave
 // alone on its SIMD issues an instruction in about 5 cycles, one of two in 8; the
 // workgroups of a short list would fill a few compute units with two waves per
-// SIMD and leave the others idle. Twelve queries at a time over 20,011 targets
-// (lists of 400): 54 to 44 ms.
+// SIMD and leave the others idle. Against all eight with a grid for eight, 200
+// targets of 350: Backward at M = 86 | 400 | 700 284 | 413 | 533 -> 243 | 329 |
+// 404 us; 1000 at M = 400: Viterbi 228 -> 192, Backward 437 -> 368 us. From about
+// 4200 targets on there is no difference.
 #define LIST_SIMDS 4
 __device__ __forceinline__ int list_waves(int64_t count)
 {

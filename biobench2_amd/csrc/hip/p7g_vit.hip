@@ -196,10 +196,11 @@ void k_vit(const DevProfile p, const uint8_t *__restrict__ res, const int64_t *_
       // the closure's scan: a row's chain is M from D, D from M, the scan. Bound
       // by that chain, and from ND = 4 on by the instructions of a lone wave
       // (one in 4-5 cycles, about 18 per dword). A row of one target, M = 86 |
-      // 250 | 400 | 803 (ND = 1 | 2 | 4 | 8): 128 | 164 | 230 | 386 ns; with the
-      // lazy test, the residues, odds and thresholds handled in the row 225 |
-      // 303 | 369 | 578 ns. 16,384 targets of 350: M = 400 1110 us (1189 before),
-      // 803 1704 (1891), 1500 2447 (2945).
+      // 400 | 803 (ND = 1 | 4 | 8): 121 | 232 | 379 ns; with the lazy test, the
+      // residues, odds and thresholds handled in the row 238 | 368 | 583 ns.
+      // 16,384 targets of 350: M = 400 1110 us (1189 before), 803 1704 (1891),
+      // 1500 2447 (2945). Where the closure hardly ever ran, a full chip pays for
+      // it: 60,000 targets at M = 20 1443 us (1314).
       int bm[ND], part[ND], e[ND];
       // xB and the specials change only on a row whose xE exceeds a threshold,
       // found by a ballot on the lanes' packed maxima; xB does not fall then
